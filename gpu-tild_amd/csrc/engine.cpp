@@ -96,9 +96,10 @@ int make_axis_plan(int N, AxisPlan& pl, std::vector<float2>& tw, std::string& er
 }
 
 // ---------------------------------------------------------------- tiles
-size_t tile_lds_bytes(int Nx, int nf, int By, int Bz) {
+size_t tile_lds_bytes(int Nx, int nf, int By, int Bz, bool plane_fwd) {
     size_t rows = (size_t)nf * By * Bz;
-    return rows * Nx * sizeof(unsigned long long) + lds_bytes(Nx, (int)((rows + 1) / 2));
+    return rows * Nx * sizeof(unsigned long long) +
+           (plane_fwd ? rows * sizeof(int) : lds_bytes(Nx, (int)((rows + 1) / 2)));
 }
 
 bool choose_tiles(int dim, const int* Nx, int P, int nf, int target_tiles, int want_by, int want_bz,
@@ -531,7 +532,7 @@ int Batch::tile_regions(int id, bool bin_only, std::string& err) {
     if (R.h.spread_mode != 2) return 0;
     if (int rc = unclaim(id, err)) return rc;
     PhaseMap* mp = R.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft}; };
     HIPCHK(launch_tile_count(ctx(PH_TCOUNT), 0));
     HIPCHK(launch_tile_scan(ctx(PH_SCAN)));
     if (!bin_only) HIPCHK(launch_tile_regions(stream_, d_reps_, id));
@@ -653,7 +654,7 @@ int Batch::upload_desc(int id, std::string& err) {
 
 // ---------------------------------------------------------------- work maps
 int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& err, bool reorder_only) {
-    for (int p = 0; p < PH_COUNT; ++p) { maps[p].host.clear(); maps[p].lds = 0; maps[p].n = 0; }
+    for (int p = 0; p < PH_COUNT; ++p) { maps[p].host.clear(); maps[p].lds = 0; maps[p].n = 0; maps[p].xfft = false; }
     for (int id : ids) {
         const Replica& R = *reps_[id];
         const RepDev& h = R.h;
@@ -675,7 +676,8 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         if (h.spread_mode == 2) {
             add(PH_TCOUNT, (h.ns + kCountBlock - 1) / kCountBlock, 0);
             add(PH_SCAN, 1, 0);
-            add(PH_TILE, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz));
+            add(PH_TILE, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd));
+            maps[PH_TILE].xfft = maps[PH_TILE].xfft || !h.plane_fwd;
             if (R.reorder_every > 0) add(PH_RTILE, h.ntiles, 0);
         } else {
             add(PH_SPREADA, R.nblk_part, 0);
@@ -1043,7 +1045,7 @@ int Batch::build_tables(Replica& R, const System& S, std::string& err) {
 // device step counter plus k, and one launch at the end advances the counter.
 int Batch::enqueue_steps(SetMaps& m, int nsteps, bool integrate, bool write_forces, std::string& err) {
     PhaseMap* mp = m.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft}; };
     for (int k = 0; k < nsteps; ++k) {
         HIPCHK(launch_spread(ctx(PH_SPREADA), k));
         HIPCHK(launch_x_r2c(ctx(PH_XA), true, 0, nullptr, nullptr));
@@ -1180,7 +1182,7 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
     for (int s = 0; s < n && !rc; ++s) {
         bool used[kKernelPhases][kSlots] = {};
         auto ctx = [&](Phase p, int ph, int slot) {
-            LaunchCtx c{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads};
+            LaunchCtx c{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft};
             if (c.n > 0) { c.t0 = ev[ph][slot][0]; c.t1 = ev[ph][slot][1]; used[ph][slot] = true; }
             return c;
         };
@@ -1254,7 +1256,7 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
 int Batch::forward_spectra(int id, std::string& err) {
     Replica& R = *reps_[id];
     PhaseMap* mp = R.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft}; };
     HIPCHK(launch_x_r2c(ctx(PH_XP), false, 0, nullptr, nullptr));
     HIPCHK(launch_mid(ctx(PH_PY), 1, 0, 0, 0, nullptr));
     if (R.dim == 3) HIPCHK(launch_mid(ctx(PH_MIDZ_H), 2, 0, 0, 0, nullptr));
@@ -1268,7 +1270,7 @@ int Batch::properties(int id, tild_props* out, std::string& err) {
     HIPCHK(hipSetDevice(device_));
     if (int rc = forward_spectra(id, err)) return rc;
     PhaseMap* mp = R.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft}; };
     HIPCHK(launch_kprops(ctx(PH_KPROPS), R.nq));
     HIPCHK(launch_reduce_rows(stream_, R.h.partials, R.nq, R.h.nchunk, R.d_results));
     HIPCHK(launch_bond_props(ctx(PH_PART)));

@@ -40,6 +40,7 @@ struct PhaseMap {
     size_t lds = 0;
     int n = 0;
     int threads = 0;   // block size where a pass has more than one (0: its default)
+    bool xfft = true;  // tiled deposit: some replica of the set transforms along x in it
     int cap = 0;       // work items the device buffer holds
 };
 
@@ -243,6 +244,8 @@ void set_last_error(const std::string& msg);
 // steers the choice; want_by/want_bz > 0 force a shape (autotuner sweeps).
 bool choose_tiles(int dim, const int* Nx, int P, int nf, int target_tiles, int want_by, int want_bz,
                   int& By, int& Bz);
-size_t tile_lds_bytes(int Nx, int nf, int By, int Bz);
+// LDS of a deposit block: its accumulator rows, plus the x transform's two buffers or,
+// where the plane pass transforms (plane_fwd), the table of its rows
+size_t tile_lds_bytes(int Nx, int nf, int By, int Bz, bool plane_fwd = false);
 
 }  // namespace tild

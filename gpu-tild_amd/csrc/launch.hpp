@@ -65,6 +65,7 @@ struct LaunchCtx {
     // step profile: events that take the kernel's own start and stop times
     hipEvent_t t0 = nullptr, t1 = nullptr;
     int threads = 0;    // block size where a pass has more than one (0: its default)
+    bool xfft = true;   // tiled deposit: some replica of the set transforms along x in it
 };
 
 // Launch on c.stream; with c.t0 set, through hipExtLaunchKernel, whose events take

@@ -365,7 +365,10 @@ __device__ __forceinline__ void load_srec4(const RepDev& r, int j0, int total, c
 // 1,000 beads plus their halo share (three blocks of 512 fit a CU; on the 640,000-bead
 // melt 17.5 us, against 19.6 with 256 threads and 22.8 with 1,024, where one block
 // fills a CU); NT = 256 for small tiles, where a larger block mostly idles.
-template <int kDepositThreads>
+// XFFT false: every replica of the set leaves the x transform to its forward plane pass,
+// so the block needs neither the transform's registers (79 VGPRs, six waves per SIMD)
+// nor its two LDS buffers (half of the block's LDS).
+template <int kDepositThreads, bool XFFT>
 __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* __restrict__ reps,
                                                               const WorkItem* __restrict__ wmap, int koff) {
     extern __shared__ unsigned long long tile_lds[];
@@ -407,7 +410,7 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
     if (t == 0 && threadIdx.x == 0) G(r.tovf)[(par ^ 1) * 32] = 0;
     for (int k = threadIdx.x; k < rows * Nx; k += kDepositThreads) patch[k] = 0ull;
     const int T = r.ntypes;
-    const int Ny = r.Ny, M = r.M, plane_fwd = r.plane_fwd;
+    const int Ny = r.Ny, M = r.M, plane_fwd = XFFT ? r.plane_fwd : 1;
     // where the plane pass transforms the densities the FFT scratch is free: it holds
     // the first density element of each tile row (f, lz, ly)
     int* const rowoff = (int*)fbuf;
@@ -528,6 +531,7 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
         }
         if (!plane_fwd) fbuf[n * ldb + j] = make_float2(v[0], v[1]);
     }
+    if constexpr (!XFFT) return;
     if (plane_fwd) return;   // the plane pass transforms the densities
     __syncthreads();
     const float2* res = lds_fft<kDepositThreads>(fbuf, fbuf + (size_t)Nx * ldb, ldb, npairs, r.ax[0]);
@@ -581,8 +585,13 @@ hipError_t launch_tile_regions_set(const LaunchCtx& c) {
 }
 hipError_t launch_tile_deposit(const LaunchCtx& c, int koff) {
     if (!c.n) return hipSuccess;
-    if (c.threads >= 512) TILD_LAUNCH(c, k_tile_deposit<512>, dim3(c.n), dim3(512), c.lds, c.reps, c.wmap, koff);
-    else TILD_LAUNCH(c, k_tile_deposit<256>, dim3(c.n), dim3(256), c.lds, c.reps, c.wmap, koff);
+    if (c.threads >= 512) {
+        if (c.xfft) TILD_LAUNCH(c, (k_tile_deposit<512, true>), dim3(c.n), dim3(512), c.lds, c.reps, c.wmap, koff);
+        else TILD_LAUNCH(c, (k_tile_deposit<512, false>), dim3(c.n), dim3(512), c.lds, c.reps, c.wmap, koff);
+    } else {
+        if (c.xfft) TILD_LAUNCH(c, (k_tile_deposit<256, true>), dim3(c.n), dim3(256), c.lds, c.reps, c.wmap, koff);
+        else TILD_LAUNCH(c, (k_tile_deposit<256, false>), dim3(c.n), dim3(256), c.lds, c.reps, c.wmap, koff);
+    }
     CHECK_LAUNCH(); return hipSuccess;
 }
 
