@@ -1,0 +1,6 @@
+// fft_last2.hip -- k_last_reg for longer axes (R1 >= 12), one or two types.
+#include "fft_last.hpp"
+
+namespace tild {
+TILD_LAST_REG_CLASS(2)
+}  // namespace tild

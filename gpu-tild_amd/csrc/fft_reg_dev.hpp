@@ -1,0 +1,18 @@
+// fft_reg_dev.hpp -- helpers of the register-resident FFT passes.
+#pragma once
+#include "device.hpp"
+
+namespace tild {
+
+// Products that the LDS-staged pass writes to LDS before its next stage adds them:
+// kept out of FMA contraction with those additions, as they are there.
+__device__ __forceinline__ float2 scaled(float s, float2 a) {
+#pragma clang fp contract(off)
+    return make_float2(s * a.x, s * a.y);
+}
+__device__ __forceinline__ float2 grad_line(float k, float2 a) {
+#pragma clang fp contract(off)
+    return make_float2(k * a.y, k * a.x);
+}
+
+}  // namespace tild

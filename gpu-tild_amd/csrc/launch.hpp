@@ -91,23 +91,27 @@ constexpr int kGradThreads = 256;                       // block of the y invers
 constexpr int kC2rThreads = 256;                        // block of the inverse x pass (records)
 constexpr size_t kPlaneLds = 163840;                    // LDS one block may use (MI355X)
 hipError_t launch_mid_grad(const LaunchCtx& c);
-// Two-stage Stockham plans R1 x R2 the register-resident passes are compiled for (the
-// benchmark workloads' axes: 160, 80, 64, 40, and the sweep's and server's 128, 50, 48,
-// 32, 30, 25 and 24 points).
-#define TILD_REG_PLANS(X) X(16, 10) X(10, 8) X(8, 8) X(8, 5) X(16, 8) X(10, 5) X(16, 3) X(8, 4) X(10, 3) X(5, 5) X(8, 3)
-// Fused last-axis pass with register-resident columns (fft_reg.hip): last axes with one
-// of those plans, at most four types (two on axes whose first radix is 16) plus charges.  Blocks of kLastRegThreads threads hold nl_last = kLastRegThreads / (2 R1)
+// Two-stage Stockham plans R1 x R2 the register-resident passes are compiled for: the
+// 5-smooth lengths from 24 to 256 that two radices up to 16 make (as the planner splits
+// them), and 21, 28, 35 and 63 points.
+#define TILD_REG_PLANS(X) \
+    X(6, 4) X(5, 5) X(9, 3) X(6, 5) X(8, 4) X(6, 6) X(8, 5) X(9, 5) X(8, 6) X(10, 5) X(9, 6) X(10, 6) X(8, 8) \
+    X(9, 8) X(15, 5) X(10, 8) X(10, 9) X(12, 8) X(10, 10) X(12, 9) X(12, 10) X(16, 8) X(12, 12) X(15, 10) \
+    X(16, 10) X(15, 12) X(16, 12) X(15, 15) X(16, 15) X(16, 16) X(7, 3) X(7, 4) X(7, 5) X(9, 7)
+// Fused last-axis pass with register-resident columns (fft_last.hpp): last axes with one
+// of those plans, at most four types (two on axes whose first radix is 12 or more) plus
+// charges.  Blocks of kLastRegThreads threads hold nl_last = kLastRegThreads / (2 R1)
 // columns; results agree with k_last_fused to rounding.
 constexpr int kLastRegThreads = 256;
-// the variants compiled in (plan R1 x R2, types, charge field): those that fit 256
-// registers per thread, so that every variant runs two waves per SIMD (160-point axes
-// up to two types)
+// the variants compiled in (plan R1 x R2, types, charge field): a thread of the middle
+// stage holds R2 values of every field, at most 40 of them
 __host__ __device__ constexpr bool last_reg_variant(int R1, int R2, int TT, int CH) {
-    return R1 == 16 ? TT <= 2 : TT <= 4;
+    return TT <= (R1 >= 12 ? 2 : 4) && (TT + CH) * R2 <= 40;
 }
-// the kernel instantiation of a type count: up to three types (class 0), four (class 1,
-// up to 256 registers, in a kernel of its own so that the others keep theirs)
-__host__ __device__ constexpr int last_reg_class(int TT) { return TT >= 4 ? 1 : 0; }
+// the kernel instantiation of a variant: plans with R1 <= 10 and up to two types (class 0)
+// or three and four (class 1: over 256 registers, in blocks whose LDS leaves one to a CU
+// anyway), and the longer plans (class 2)
+__host__ __device__ constexpr int last_reg_class(int R1, int TT) { return R1 >= 12 ? 2 : (TT >= 3 ? 1 : 0); }
 bool last_reg_plan(const AxisPlan& pl, int ntypes, int nf);
 inline int last_reg_lines(const AxisPlan& pl) { return kLastRegThreads / (2 * pl.rad[0]); }
 // the two exchange buffers, both stages' twiddles (2N - R1 - R2) and the ramp weights
@@ -116,6 +120,12 @@ inline size_t last_reg_lds_bytes(const AxisPlan& pl, int nf) {
     return (N * (3 * (size_t)nf * nl + 2) + 2 * N) * sizeof(float2) + kMaxRamp * sizeof(float);
 }
 hipError_t launch_last_reg(const LaunchCtx& c, int koff, int cls);
+hipError_t launch_last_reg_0(const LaunchCtx& c, int koff);   // one per class, in files of their own
+hipError_t launch_last_reg_1(const LaunchCtx& c, int koff);
+hipError_t launch_last_reg_2(const LaunchCtx& c, int koff);
+hipError_t configure_last_reg_0();
+hipError_t configure_last_reg_1();
+hipError_t configure_last_reg_2();
 // The y inverse of the gradient spectra with register-resident columns (3D, two-stage
 // y plans as above): blocks of kGradRegThreads threads, grad_reg_lines(plan) columns
 // each, grad_reg_chunks per (field, z) plane.
