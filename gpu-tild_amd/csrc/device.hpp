@@ -6,6 +6,7 @@
 // A single-replica step is the same launches with a one-entry map.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <cstddef>
 #include <cstdint>
 
 namespace tild {
@@ -23,83 +24,119 @@ constexpr int kMaxQuant = 128;     // property quantities per replica
 struct AxisPlan {
     int N;
     int nst;
-    int rad[kMaxStages];
-    int tw_off[kMaxStages];
     int ntw;            // twiddles in the table (at most N)
     const float2* tw;
+    int rad[kMaxStages];
+    int tw_off[kMaxStages];
 };
 // room for the twiddles of an N-point plan (ntw <= tw_elems(N))
 __host__ __device__ inline int tw_elems(int N) { return N > 1 ? N : 1; }
 
-// Per-replica descriptor (device memory).
-struct RepDev {
-    // geometry (initialize.cu:32-48)
+// Per-replica descriptor (device memory).  The fields the step kernels read come first,
+// grouped by kernel into 64-byte lines: a kernel requests the lines it needs at once
+// (warm_desc), where reading each field where it is used costs a scalar-cache miss per
+// line, one after the other (fifteen in the particle kernel).
+struct alignas(64) RepDev {
+    // line 0: sizes (initialize.cu:32-48), counters
     int dim, Nx, Ny, Nz, Nxh, M, Mh, ns, ntypes, nf, P;
-    float L[3], Lh[3], dx[3], gvol, kfac[3];   // kfac = 2 pi / L
-    float idx[3];                              // 1 / dx (FP32), for the spline weights
+    int step;                  // completed steps; X[step & 1] is current
+    uint32_t seed;
+    int spread_mode;           // 1 global atomics, 2 LDS-tiled sorted bins
+    int g3_off32;              // 1: nf*M*12 bytes of records fit 32-bit byte offsets
+    int grid_off32;            // 1: every grid buffer (rho, H, Gk, G3) fits 32-bit byte offsets
+    // line 1: box
+    float L[3], Lh[3], dx[3];
+    float idx[3];              // 1 / dx (FP32), for the spline weights
+    float kfac[3];             // 2 pi / L
+    float gvol;
+    // lines 2-3: particle state
+    float* X[2];               // ns*dim, double-buffered by step parity
+    float* XO;                 // ns*dim, GJF previous position
+    const int* tp;             // ns
+    const float* q;            // ns or null
+    const int* bond;           // ns*3 slots: (partner << bond_shift) | bond type; -1 = empty
+    int bond_shift;            // bits of the bond type (0 for one type)
+    int any_gjf;               // 1: some site integrates with GJF
+    float delt, noise_mag;
+    const float* bond_k;       // per bond type
+    const float* bond_r0;
+    const signed char* ikind;  // ns: 0 none, 1 EM, 2 GJF
+    float* fout;               // ns*dim (optional)
+    int* pid;                  // ns: original site id of each slot (noise key, host order)
+    float* G3;                 // nf*M*3 gather records (g_x, g_y, g_z)
+    const float* FPtab;        // T*dim*M net static field-phase forces per type (or null)
+    int plane_fwd;             // 1: the tiled deposit writes rho only; x R2C + y FFT run per plane
+    int srec;                  // 1: order-1 stencil records (stencil_record), 0: (x, y, z, type)
+    // lines 4-5: sorted-bin deposition: full-x slab tiles of By x Bz rows (By | Ny, Bz | Nz)
+    int By, Bz, nty, ntz, ntiles, nbuckets;
+    float iBy, iBz;            // 1 / By, 1 / Bz (FP32) for the bucket divisions
+    int tshift;                // log2 of the counter stride: one 128-byte line per bucket
+    int tslack;                // spare slots per region (0: count/4 + 16, < 0: none)
+    // per-step binning into fixed bucket regions (sized at creation and each reorder)
+    int* tclaim;               // 2 x (nbuckets << tshift) slot counters, by step parity
+    int* tbase;                // nbuckets + 1: first record of each bucket's region
+    int* tcap;                 // nbuckets: region sizes
+    float4* trec;              // records in bucket regions (16 bytes, either kind)
+    float* trecq;              // their charges (charged decks)
+    int* tovf;                 // overflow counts by step parity, at [0] and [32]
+    float4* tovf_rec;          // ns records that found their region full
+    int* tovf_b;               // their buckets
+    float* tovf_q;             // their charges
     // fixed-point densities: acc = round(w * 2^F), rho = acc * inv
-    float fix_scale, fixq_scale;
-    double fix_inv, fixq_inv;
     int fix_s2, fix_s3;        // order-1 integer weights: 44 - F and 52 - F (fixed_weight2/3)
     float fixq_s1;             // order-1 charge weights: fixq_scale 2^-22 per axis (fixed_charge)
-    // FFT plans (x, y, z) and chunk sizes of each pass
-    AxisPlan ax[3];
-    AxisPlan axr;  // inverse plan of the last axis: a two-stage plan reversed, else ax[dim - 1]
+    float fix_scale;
+    // line 6: grids
+    double fix_inv, fixq_inv;
+    float* rho;                // nf*M densities (x fastest)
+    float2* H;                 // nf*Mh half spectra
+    float2* Gk;                // nf*dim*Mh half spectra of the gathered fields
+    unsigned long long* acc;   // nf*M fixed-point accumulators
+    const float* Ctab;         // coupling tables C_IJ/M (I <= J) + charge table, blocked as
+                               // [column block][last-axis index][row][nl_last columns]
+    float fixq_scale;
+    int ctab_rows;             // rows of Ctab: T(T+1)/2 (+1 with charges)
+    // line 7: FFT passes
+    int ctab_charge;           // row of the charge kernel in Ctab (or -1)
+    int nramp, ramp_row0;      // ramped pair styles, see below
+    int reg_key[3];            // axis plans of two stages: R1 * 32 + R2 (else 0)
+    const float2* reg_tw[3];   // and their second stage's twiddles
+    const float2* reg_twr;     // the same of the last axis' inverse plan axr
+    int nl_last;   // batch columns per block, fused last-axis pass
+    int last_dirs; // directions per inverse batch of the fused last-axis pass (1..dim)
+    // line 8: block geometry (chunk sizes of each pass) and forms
     int nl_x;      // line pairs per block, forward x pass
     int nl_mid;    // batch columns per block, middle (y) pass
-    int nl_last;   // batch columns per block, fused last-axis pass
     int nr_c2r;    // rows per block, inverse x pass
     int mid_elems; // complex values per block of the middle-axis passes (0: kFftBudget)
-    int plane_fwd; // 1: the tiled deposit writes rho only; x R2C + y FFT run per plane
-    int last_dirs; // directions per inverse batch of the fused last-axis pass (1..dim)
     int last_reg;  // 1: the fused last-axis pass runs register-resident (k_last_reg)
     int grad_reg;  // 1: the y inverse of the gradient spectra runs register-resident (k_grad_reg)
     int plane_reg; // 1: the forward plane pass runs register-resident (k_plane_reg)
     int plane_inv; // 1: y inverse and x C2R run as one register-resident plane pass (k_plane_inv)
-    // particle state
-    float* X[2];            // ns*dim, double-buffered by step parity
-    float* XO;              // ns*dim, GJF previous position
-    const int* tp;          // ns
-    const float* q;         // ns or null
-    const int* bond;        // ns*3 slots: (partner << bond_shift) | bond type; -1 = empty
-    int bond_shift;         // bits of the bond type (0 for one type)
-    const float* bond_k;    // per bond type
-    const float* bond_r0;
-    const signed char* ikind;  // ns: 0 none, 1 EM, 2 GJF
-    float delt, noise_mag;
-    int any_gjf;            // 1: some site integrates with GJF
+    // FFT plans (x, y, z)
+    AxisPlan ax[3];
+    AxisPlan axr;  // inverse plan of the last axis: a two-stage plan reversed, else ax[dim - 1]
+    // per type
     float gjf_b[kMaxTypes], gjf_a[kMaxTypes], gjf_c1[kMaxTypes], gjf_c2[kMaxTypes],
           gjf_noise[kMaxTypes];
-    float* fout;            // ns*dim (optional)
-    int* pid;               // ns: original site id of each slot (noise key, host order)
+    // ramped pair styles (pair_style.cu:308-328): Ctab row ramp_row0 + j holds ramped
+    // style j's table per unit prefactor, added to pair row ramp_pair[j] with weight
+    // A_j(k) - ramp_A0[j] at 0-based step k, where A_j(0) = ramp_A0[j] and
+    // A_j(k) = ramp_c0[j] + ramp_c1[j] * (k + 1) after the first step
+    int ramp_pair[kMaxRamp];
+    double ramp_A0[kMaxRamp], ramp_c0[kMaxRamp], ramp_c1[kMaxRamp];
+    // spatial reorder: scratch, and the spare buffers swapped with the live arrays
     int *rsrc, *rorder, *rinv;   // ns each: scratch of the tiled spatial reorder
-    // spare buffers of the periodic spatial reorder, swapped with the live arrays
     float* XO_alt;
     int* tp_alt;
     float* q_alt;
     int* bond_alt;
     signed char* ikind_alt;
     int* pid_alt;
-    // grids
-    unsigned long long* acc;   // nf*M fixed-point accumulators
-    float* rho;                // nf*M densities (x fastest)
-    float2* H;                 // nf*Mh half spectra
-    float2* Gk;                // nf*dim*Mh half spectra of the gathered fields
-    float* G3;                 // nf*M*3 gather records (g_x, g_y, g_z), zero where rho <= 0
-    int g3_off32;              // 1: nf*M*12 bytes of records fit 32-bit byte offsets
-    int grid_off32;            // 1: every grid buffer (rho, H, Gk, G3) fits 32-bit byte offsets
-    const float* Ctab;         // coupling tables C_IJ/M (I <= J) + charge table, blocked as
-                               // [column block][last-axis index][row][nl_last columns]
-    int ctab_rows;             // rows of Ctab: T(T+1)/2 (+1 with charges)
-    const float* FPtab;        // T*dim*M net static field-phase forces per type (or null)
-    int ctab_charge;           // row of the charge kernel in Ctab (or -1)
-    // ramped pair styles (pair_style.cu:308-328): Ctab row ramp_row0 + j holds ramped
-    // style j's table per unit prefactor, added to pair row ramp_pair[j] with weight
-    // A_j(k) - ramp_A0[j] at 0-based step k, where A_j(0) = ramp_A0[j] and
-    // A_j(k) = ramp_c0[j] + ramp_c1[j] * (k + 1) after the first step
-    int nramp, ramp_row0;
-    int ramp_pair[kMaxRamp];
-    double ramp_A0[kMaxRamp], ramp_c0[kMaxRamp], ramp_c1[kMaxRamp];
+    // exact binning (spatial reorder, capacity sizing): counts, offsets, (bucket, slot)
+    int* tcnt;                 // nbuckets counters (zero between uses), bucket b at b << tshift
+    int* toff;                 // nbuckets + 1 exclusive offsets
+    int2* tkey;                // ns (bucket, slot)
     // property tables
     int nstyles, npairs, nq;
     int st_t1[64], st_t2[64];
@@ -110,32 +147,28 @@ struct RepDev {
     double* partials;          // nq * nchunk partial sums
     int nchunk;
     double* bpart;             // 7 * ceil(ns/256) bond-property partials
-    // sorted-bin deposition: full-x slab tiles of By x Bz rows (By | Ny, Bz | Nz)
-    int spread_mode;           // 1 global atomics, 2 LDS-tiled sorted bins
-    int By, Bz, nty, ntz, ntiles, nbuckets;
-    float iBy, iBz;            // 1 / By, 1 / Bz (FP32) for the bucket divisions
-    int tshift;                // log2 of the counter stride: one 128-byte line per bucket
-    // exact binning (spatial reorder, capacity sizing): counts, offsets, (bucket, slot)
-    int* tcnt;                 // nbuckets counters (zero between uses), bucket b at b << tshift
-    int* toff;                 // nbuckets + 1 exclusive offsets
-    int2* tkey;                // ns (bucket, slot)
-    // per-step binning into fixed bucket regions (sized at creation and each reorder)
-    int* tclaim;               // 2 x (nbuckets << tshift) slot counters, by step parity
-    int* tbase;                // nbuckets + 1: first record of each bucket's region
-    int* tcap;                 // nbuckets: region sizes
-    int tslack;                // spare slots per region (0: count/4 + 16, < 0: none)
-    int srec;                  // 1: order-1 stencil records (stencil_record), 0: (x, y, z, type)
-    float4* trec;              // records in bucket regions (16 bytes, either kind)
-    float* trecq;              // their charges (charged decks)
-    int* tovf;                 // overflow counts by step parity, at [0] and [32]
-    float4* tovf_rec;          // ns records that found their region full
-    int* tovf_b;               // their buckets
-    float* tovf_q;             // their charges
-    // counters
-    int step;                  // completed steps; X[step & 1] is current
-    uint32_t seed;
     int nP;
 };
+static_assert(offsetof(RepDev, L) == 64 && offsetof(RepDev, X) == 128 && offsetof(RepDev, bond_k) == 192 &&
+              offsetof(RepDev, By) == 256 && offsetof(RepDev, trec) == 320 && offsetof(RepDev, fix_inv) == 384 &&
+              offsetof(RepDev, ctab_charge) == 448 && offsetof(RepDev, nl_x) == 512, "RepDev: 64-byte lines");
+
+// Requests the given 64-byte lines of a descriptor together and waits once: the scalar
+// loads of their fields that follow hit the scalar cache.
+template <int... LINES>
+__device__ __forceinline__ void warm_desc(const RepDev& r) {
+    const int* p = (const int*)&r;
+    constexpr int n = sizeof...(LINES);
+    static_assert(n >= 4 && n <= 8, "warm_desc: four to eight lines");
+    const int v[n] = {p[LINES * 16]...};
+    if constexpr (n == 4) asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]));
+    else if constexpr (n == 5) asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]), "s"(v[4]));
+    else if constexpr (n == 6) asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]), "s"(v[4]), "s"(v[5]));
+    else if constexpr (n == 7)
+        asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]), "s"(v[4]), "s"(v[5]), "s"(v[6]));
+    else
+        asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]), "s"(v[4]), "s"(v[5]), "s"(v[6]), "s"(v[7]));
+}
 
 struct WorkItem { int rep, blk; };
 

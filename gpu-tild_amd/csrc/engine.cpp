@@ -281,6 +281,12 @@ int Batch::add_plain(const System& S, uint32_t seed, std::string& err) {
     for (int a = 0; a < D; ++a) h.ax[a].tw = d_tw + toff[a];
     h.axr.tw = d_tw + toff_r;
     if (D == 2) h.ax[2] = h.ax[1];
+    for (int a = 0; a < D; ++a)
+        if (h.ax[a].nst == 2) {
+            h.reg_key[a] = h.ax[a].rad[0] * 32 + h.ax[a].rad[1];
+            h.reg_tw[a] = h.ax[a].tw + h.ax[a].tw_off[1];
+        }
+    if (h.axr.nst == 2) h.reg_twr = h.axr.tw + h.axr.tw_off[1];
 
     // chunking of each pass
     const int rows = h.M / h.Nx;

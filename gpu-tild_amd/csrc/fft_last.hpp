@@ -60,8 +60,8 @@ __device__ __forceinline__ void last_reg_block(const RepDev& r, int blk, float2*
 
     // set-up, visible after the first barrier: twiddles and ramp weights into LDS
     {
-        const float2* tw1 = r.ax[la].tw + r.ax[la].tw_off[1];
-        const float2* tw2 = r.axr.tw + r.axr.tw_off[1];
+        const float2* tw1 = la == 2 ? r.reg_tw[2] : r.reg_tw[1];
+        const float2* tw2 = r.reg_twr;
         for (int t = threadIdx.x; t < NT1; t += NT) TW1[t] = gld(tw1 + t);
         for (int t = threadIdx.x; t < NT2; t += NT) TW2[t] = gld(tw2 + t);
         if ((int)threadIdx.x < r.nramp) rw[threadIdx.x] = ramp_weight(r, threadIdx.x, r.step + koff);
@@ -226,8 +226,8 @@ __global__ void __launch_bounds__(NT) k_last_reg(const RepDev* __restrict__ reps
     extern __shared__ float2 lds[];
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
-    const AxisPlan& pl = r.ax[r.dim - 1];
-    switch (pl.rad[0] * 32 + pl.rad[1]) {   // uniform per block
+    warm_desc<0, 1, 6, 7>(r);
+    switch (r.dim == 3 ? r.reg_key[2] : r.reg_key[1]) {   // uniform per block
 #define TILD_CASE(A, B) case A * 32 + B: last_reg_types<A, B, NT, CLS>(r, wi.blk, lds, koff); break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE

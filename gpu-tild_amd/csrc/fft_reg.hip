@@ -49,7 +49,7 @@ __device__ __forceinline__ void grad_reg_block(const RepDev& r, int blk, float2*
     float2* TW1 = X1 + N * ld;        // w_Ny^{i r}, i < R1, 1 <= r < R2
     const int b = (int)threadIdx.x % NB, i = (int)threadIdx.x / NB;
     {
-        const float2* tw1 = r.ax[1].tw + r.ax[1].tw_off[1];
+        const float2* tw1 = r.reg_tw[1];
         for (int t = threadIdx.x; t < NT1; t += NT) TW1[t] = gld(tw1 + t);
     }
     // element (n, column b) of slot s: 32-bit offsets from the uniform base
@@ -109,8 +109,8 @@ __global__ void __launch_bounds__(NT) k_grad_reg(const RepDev* __restrict__ reps
     extern __shared__ float2 lds[];
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
-    const AxisPlan& pl = r.ax[1];
-    switch (pl.rad[0] * 32 + pl.rad[1]) {   // uniform per block
+    warm_desc<0, 1, 6, 7>(r);
+    switch (r.reg_key[1]) {   // uniform per block
 #define TILD_CASE(A, B) case A * 32 + B: grad_reg_block<A, B, NT>(r, wi.blk, lds); break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
@@ -144,8 +144,8 @@ __device__ __forceinline__ void plane_reg_block(const RepDev& r, int blk, float2
     float2* TWx = Xb + N * ldp;        // w_N^{i r} of the x plan and of the y plan
     float2* TWy = TWx + NT1;
     {
-        const float2* tx = r.ax[0].tw + r.ax[0].tw_off[1];
-        const float2* ty = r.ax[1].tw + r.ax[1].tw_off[1];
+        const float2* tx = r.reg_tw[0];
+        const float2* ty = r.reg_tw[1];
         for (int t = threadIdx.x; t < NT1; t += NT) { TWx[t] = gld(tx + t); TWy[t] = gld(ty + t); }
     }
     const uint32_t pbase = (uint32_t)f * (uint32_t)r.M + (uint32_t)z * (uint32_t)(N * N);
@@ -216,8 +216,8 @@ __global__ void __launch_bounds__(NT) k_plane_reg(const RepDev* __restrict__ rep
     extern __shared__ float2 lds[];
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
-    const AxisPlan& pl = r.ax[0];
-    switch (pl.rad[0] * 32 + pl.rad[1]) {   // uniform per block
+    warm_desc<0, 1, 6, 7>(r);
+    switch (r.reg_key[0]) {   // uniform per block
 #define TILD_CASE(A, B) case A * 32 + B: plane_reg_block<A, B, NT>(r, wi.blk, lds); break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
@@ -259,7 +259,7 @@ __device__ __forceinline__ void plane_inv_block(const RepDev& r, int blk, float2
     float2* X = lds;                   // N x LA: y stages, then the x exchange (N x LC)
     float2* TW = X + N * LA;           // w_N^{i r}, i < R1, 1 <= r < R2 (same plan on x and y)
     {
-        const float2* tw = r.ax[1].tw + r.ax[1].tw_off[1];
+        const float2* tw = r.reg_tw[1];
         for (int t = threadIdx.x; t < NT1; t += NT) TW[t] = gld(tw + t);
     }
     const uint32_t Mhu = (uint32_t)r.Mh;
@@ -407,8 +407,8 @@ __global__ void __launch_bounds__(NT) k_plane_inv(const RepDev* __restrict__ rep
     extern __shared__ float2 lds[];
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
-    const AxisPlan& pl = r.ax[1];
-    switch (pl.rad[0] * 32 + pl.rad[1]) {   // uniform per block
+    warm_desc<0, 1, 3, 6, 7>(r);
+    switch (r.reg_key[1]) {   // uniform per block
 #define TILD_CASE(A, B) \
     case A * 32 + B: if constexpr ((A * B / 2 + 1) * (A > B ? A : B) <= NT) plane_inv_block<A, B, NT>(r, wi.blk, lds); break;
         TILD_REG_PLANS(TILD_CASE)

@@ -494,6 +494,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) k_
     extern __shared__ float2 lds[];
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
+    if (RECORDS) warm_desc<0, 1, 3, 6, 7, 8, 9, 10>(r);   // with the x plan
     if (RECORDS && r.grid_off32 && !r.FPtab) {   // the common layouts, per block (uniform)
         if (r.dim == 3 && r.nf == 2) { x_c2r_records<2, 3, NT>(r, wi, lds); return; }
         if (r.dim == 3 && r.nf == 5) { x_c2r_records<5, 3, NT>(r, wi, lds); return; }
@@ -929,6 +930,7 @@ __global__ void __launch_bounds__(256) k_particles(const RepDev* __restrict__ re
                                                    int write_forces, int koff) {
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
+    warm_desc<0, 1, 2, 3, 4, 5>(r);
     const int i = wi.blk * 256 + threadIdx.x;
     const bool valid = i < r.ns;
     if (!CLAIM && !valid) return;

@@ -374,6 +374,7 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
     extern __shared__ unsigned long long tile_lds[];
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
+    warm_desc<0, 3, 4, 5, 6>(r);
     const int D = r.dim, P = r.P, Nx = r.Nx, Nxh = r.Nxh;
     const int By = r.By, Bz = r.Bz, nf = r.nf;
     const int t = wi.blk, ty = t % r.nty, tz = t / r.nty;
