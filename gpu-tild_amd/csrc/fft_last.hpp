@@ -6,18 +6,22 @@
 // inverse transforms of w and -i k_la w -- for last axes with a two-stage plan
 // N = R1 R2 (TILD_REG_PLANS; R1 >= R2).  Each
 // thread keeps its Stockham columns in registers between the stages, so a block makes
-// two LDS exchanges and two barriers, where the LDS-staged form stages every value
+// three LDS exchanges and three barriers, where the LDS-staged form stages every value
 // through LDS and ends each of its nine phases with a barrier:
 //
-//   A  task (b, i < R2, field): rows i + R2 r (r < R1) of column b, read from HBM
-//      straight into registers; DFT_R1; exchange.
-//   B  thread (b, i < R1, h < 2): twiddles w_N^{i r}, DFT_R2 -> rho_f(k) at
-//      k = i + R1 q; the coupling in registers; inverse direction h (conj(w) or
-//      conj(-i k w)) is transformed by the Stockham plan R2 x R1, whose first stage
-//      (radix R2, no twiddles) reads exactly the values k = i + R1 q this thread holds;
-//      exchange.
-//   C  task (b, j < R2, line): twiddles w_N^{j r}, DFT_R1 -> rows j + R2 q; store.
+//   A   thread (b, i < R2, f): rows i + R2 r of column b of field f, read from HBM
+//       straight into registers; DFT_R1; exchange.
+//   B1  thread (b, i < R1, f): twiddles w_N^{i r}, DFT_R2 -> rho_f(k) at k = i + R1 q,
+//       back to the rows it read, where the threads of the other fields find it.
+//   B2  thread (b, i, f): w_f(k) = sum_J C_fJ rho_J at those k, and the first stage of its
+//       two inverse lines conj(w), conj(-i k w) by the Stockham plan R2 x R1, whose first
+//       stage (radix R2, no twiddles) reads exactly the values k = i + R1 q; exchange.
+//   C   task (b, j < R2, line): twiddles w_N^{j r}, DFT_R1 -> rows j + R2 q; store.
 //
+// One field per thread in the middle stages: a thread that took every field (and one of
+// the two inverse lines, so that two threads repeated the forward stage) issued 1.5 times
+// the instructions and held up to 256 registers; the stage was the longest of the block
+// (2.7 of 7.7 us on a 192-point film's 13 blocks, where it ran one wave per SIMD).
 // The transforms and sums are those of the LDS-staged pass (whose inverse also runs the
 // reversed plan RepDev::axr); the two agree to rounding, since the compiler contracts
 // multiplies into the following additions differently where one keeps in registers
@@ -32,161 +36,160 @@ namespace tild {
 
 namespace {
 
-// One block: NB = NT / (2 R1) adjacent columns q0 .. q0 + NB - 1 of the last-axis lines
-// (fewer in the last block), TT types and CH charge fields (NF = TT + CH fields).  Two
-// threads share each (column, i) of the middle stage: both run the forward stage and
-// the coupling, and each transforms one of the two inverse directions.
-// LDS: the forward exchange (N x ldx), the inverse exchange (N x ldy), both stages'
-// twiddles, then the ramp weights (last_reg_lds_bytes).
+// One block: NB = last_reg_cols(R1, NF) adjacent columns q0 .. q0 + NB - 1 of the
+// last-axis lines (fewer in the last block), TT types and CH charge fields (NF = TT + CH).
+// LDS: the forward exchange (N x ldx), the inverse exchange (N x ldy), the inverse
+// stage's twiddles, then the ramp weights (last_reg_lds_bytes).
 template <int R1, int R2, int NT, int TT, int CH>
 __device__ __forceinline__ void last_reg_block(const RepDev& r, int blk, float2* lds, int koff) {
-    constexpr int N = R1 * R2, NF = TT + CH, NR = TT * (TT + 1) / 2, NB = NT / (2 * R1);
+    constexpr int N = R1 * R2, NF = TT + CH, NB = last_reg_cols(R1, NF);
     constexpr int ldx = NF * NB + 1, ldy = 2 * NF * NB + 1;
-    constexpr int NT1 = R1 * (R2 - 1), NT2 = R2 * (R1 - 1);
+    constexpr int NT2 = R2 * (R1 - 1);
+    static_assert(R2 <= R1 && NB * R1 * NF <= NT && NT2 <= NT, "k_last_reg: one middle-stage task per thread");
     const int la = r.dim - 1, D = r.dim;
     const int Q = la == 2 ? r.Ny * r.Nxh : r.Nxh;   // plane size = line stride
     const int q0 = blk * NB;
     const int nb = min(NB, Q - q0);
     float2* X1 = lds;                               // N x ldx: forward exchange
     float2* Y1 = lds + N * ldx;                     // N x ldy: inverse exchange
-    float2* TW1 = Y1 + N * ldy;                     // w_N^{i r}, i < R1, 1 <= r < R2 (forward stage 2)
-    float2* TW2 = TW1 + NT1;                        // w_N^{j r}, j < R2, 1 <= r < R1 (inverse stage 2)
+    float2* TW2 = Y1 + N * ldy;                     // w_N^{j r}, j < R2, 1 <= r < R1 (inverse stage 2)
     float* rw = (float*)(TW2 + NT2);                // ramp weights of this step
-    // phase B: thread (b, i, h), h = the inverse direction it transforms
-    const int b = (int)threadIdx.x % NB, i = ((int)threadIdx.x / NB) % R1, h = (int)threadIdx.x / (NB * R1);
+    // lanes: column, then field, then i (the fields' LDS rows are NB values apart, which
+    // spreads a wave's accesses over the banks)
+    const int b = (int)threadIdx.x % NB, f = ((int)threadIdx.x / NB) % NF, i = (int)threadIdx.x / (NB * NF);
+    const bool live = b < nb && i < R1;
     // grid buffers below 4 GiB (required on the host): 32-bit element offsets
     const uint32_t Qu = (uint32_t)Q, Mhu = (uint32_t)r.Mh;
-    const bool liveB = h < 2 && b < nb;
 
-    // set-up, visible after the first barrier: twiddles and ramp weights into LDS
-    {
-        const float2* tw1 = la == 2 ? r.reg_tw[2] : r.reg_tw[1];
-        const float2* tw2 = r.reg_twr;
-        for (int t = threadIdx.x; t < NT1; t += NT) TW1[t] = gld(tw1 + t);
-        for (int t = threadIdx.x; t < NT2; t += NT) TW2[t] = gld(tw2 + t);
-        if ((int)threadIdx.x < r.nramp) rw[threadIdx.x] = ramp_weight(r, threadIdx.x, r.step + koff);
-    }
-    // coupling rows of this thread's phase-B nodes, requested before anything else
-    const int nrows = r.ctab_rows;
-    // element (n, row) of this thread's column: cb0 + (n nrows + row) NB, from the
-    // uniform table base (every offset 32-bit)
-    const uint32_t cb0 = (uint32_t)blk * (uint32_t)(N * nrows * NB) + (uint32_t)b;
-    auto ctab = [&](int n, int row) { return G(at32(r.Ctab, cb0 + (uint32_t)((n * nrows + row) * NB)))[0]; };
-    // up to three types every row of the thread's nodes is requested at block start
-    // and held through the forward stages; with four (ten rows per node) each node's
-    // rows are requested where the coupling uses them, which keeps the pass within 256
-    // registers
-    constexpr bool kEarly = NR <= 6;
-    constexpr int QE = kEarly ? R2 : 1;
-    float c[QE][NR], cq[QE];
-    auto load_rows = [&](int q, int slot) {
-#pragma unroll
-        for (int k = 0; k < NR; ++k) c[slot][k] = ctab(i + R1 * q, k);
-        cq[slot] = CH ? ctab(i + R1 * q, r.ctab_charge) : 0.f;
-    };
-    if (kEarly && liveB) {
-#pragma unroll
-        for (int q = 0; q < R2; ++q) load_rows(q, q < QE ? q : 0);
-    }
-
-    // ---- A: task (b, i < R2, f): rows i + R2 r of field f, DFT_R1 (Stockham stage 1:
-    // out[i R1 + q])
-    // lanes: column, then field, then i (the fields' LDS rows are NB values apart,
-    // which spreads a wave's writes over the banks)
-    for (int task = threadIdx.x; task < NB * R2 * NF; task += NT) {
-        const int ba = task % NB, f = (task / NB) % NF, ia = task / (NB * NF);
-        if (ba >= nb) continue;
-        float2 v[R1];
+    // everything the block reads is requested before the first wait: this thread's rows
+    // of the spectrum, its twiddles of both stages and its coupling rows
+    float2 t2 = make_float2(0.f, 0.f);
+    if ((int)threadIdx.x < NT2) t2 = gld(r.reg_twr + threadIdx.x);
+    float2 v[R1];
+    const bool liveA = b < nb && i < R2;
+    if (liveA) {
 #pragma unroll
         for (int rr = 0; rr < R1; ++rr)
-            v[rr] = gld(at32((const float2*)r.H, (uint32_t)f * Mhu + (uint32_t)(ia + R2 * rr) * Qu + (uint32_t)(q0 + ba)));
+            v[rr] = gld(at32((const float2*)r.H, (uint32_t)f * Mhu + (uint32_t)(i + R2 * rr) * Qu + (uint32_t)(q0 + b)));
+    }
+    // coupling rows of w_f: pidx(lo, hi) = lo TT - lo (lo - 1) / 2 + (hi - lo) for the
+    // types, the charge row for the charge field.  Element (n, row) of column b:
+    // cb0 + (n nrows + row) NB from the uniform table base.
+    const int nrows = r.ctab_rows;
+    const uint32_t cb0 = (uint32_t)blk * (uint32_t)(N * nrows * NB) + (uint32_t)b;
+    auto ctab = [&](int n, int row) { return G(at32(r.Ctab, cb0 + (uint32_t)((n * nrows + row) * NB)))[0]; };
+    const bool isq = CH && f == TT;
+    auto pidx = [&](int J) {
+        const int lo = min(f, J), hi = max(f, J);
+        return lo * TT - lo * (lo - 1) / 2 + (hi - lo);
+    };
+    float2 t1[R2];
+    float c[R2][TT];
+    if (live) {
+        const float2* tw1 = la == 2 ? r.reg_tw[2] : r.reg_tw[1];
+#pragma unroll
+        for (int rr = 1; rr < R2; ++rr) t1[rr] = gld(tw1 + (i * (R2 - 1) + rr - 1));
+#pragma unroll
+        for (int J = 0; J < TT; ++J) {
+            const int row = isq ? r.ctab_charge : pidx(J);
+#pragma unroll
+            for (int q = 0; q < R2; ++q) c[q][J] = ctab(i + R1 * q, row);
+        }
+    }
+    if ((int)threadIdx.x < r.nramp) rw[threadIdx.x] = ramp_weight(r, threadIdx.x, r.step + koff);
+
+    // ---- A: DFT_R1 of rows i + R2 r (Stockham stage 1: out[i R1 + q])
+    if (liveA) {
         Dft<R1>::run(v);
 #pragma unroll
-        for (int q = 0; q < R1; ++q) X1[(ia * R1 + q) * ldx + f * NB + ba] = v[q];
+        for (int q = 0; q < R1; ++q) X1[(i * R1 + q) * ldx + f * NB + b] = v[q];
     }
+    if ((int)threadIdx.x < NT2) TW2[threadIdx.x] = t2;
     __syncthreads();
 
-    // ---- B: stage 2 (radix R2, twiddles w_N^{i r}) -> rho_f(k), k = i + R1 q
-    if (liveB) {
-        float2 w[NF][R2];
+    // ---- B1: stage 2 (radix R2, twiddles w_N^{i r}) -> rho_f(k), k = i + R1 q
+    float2 w[R2];
+    if (live) {
 #pragma unroll
-        for (int f = 0; f < NF; ++f)
+        for (int rr = 0; rr < R2; ++rr) w[rr] = X1[(i + R1 * rr) * ldx + f * NB + b];
+        // With four types or charges the twiddles count as read here: which of a sum's two products
+        // the compiler fuses follows the order their operands are read in, and this order
+        // keeps the rounding that such decks have had.
+        if constexpr (TT == 4 || CH) {
 #pragma unroll
-            for (int rr = 0; rr < R2; ++rr) w[f][rr] = X1[(i + R1 * rr) * ldx + f * NB + b];
-        float2 t[R2];
-#pragma unroll
-        for (int rr = 1; rr < R2; ++rr) t[rr] = TW1[i * (R2 - 1) + rr - 1];
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-#pragma unroll
-            for (int rr = 1; rr < R2; ++rr) w[f][rr] = cmul(w[f][rr], t[rr]);
-            Dft<R2>::run(w[f]);
+            for (int rr = 1; rr < R2; ++rr) asm volatile("" : "+v"(t1[rr].x), "+v"(t1[rr].y));
         }
-        // coupling: w_I = sum_J C_IJ rho_J over the symmetric rows pidx(lo, hi) =
-        // lo TT - lo (lo - 1) / 2 + (hi - lo); ramped styles add their weighted rows;
-        // charges w_c = G_c rho_c
+#pragma unroll
+        for (int rr = 1; rr < R2; ++rr) w[rr] = cmul(w[rr], t1[rr]);
+        Dft<R2>::run(w);
+        if constexpr (NF > 1) {
+#pragma unroll
+            for (int q = 0; q < R2; ++q) X1[(i + R1 * q) * ldx + f * NB + b] = w[q];
+        }
+    }
+    if constexpr (NF > 1) __syncthreads();
+
+    // ---- B2: coupling and the first stage of the two inverse lines
+    if (live) {
+        for (int j = 0; j < r.nramp; ++j) {   // ramped styles add their weighted rows (uniform trip count)
+            const float wj = rw[j];
+            const int rp = r.ramp_pair[j];
+#pragma unroll
+            for (int J = 0; J < TT; ++J) {
+                const bool on = !isq && rp == pidx(J);
+#pragma unroll
+                for (int q = 0; q < R2; ++q) {
+                    const float cr = wj * ctab(i + R1 * q, r.ramp_row0 + j);
+                    c[q][J] += on ? cr : 0.f;
+                }
+            }
+        }
+        // w_f = sum_J C_fJ rho_J; charges w_c = G_c rho_c
+#pragma unroll
+        for (int q = 0; q < R2; ++q) {
+            float2 acc = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int J = 0; J < TT; ++J) {
+                const float2 rh = NF > 1 ? X1[(i + R1 * q) * ldx + J * NB + b] : w[q];
+                acc.x += c[q][J] * rh.x; acc.y += c[q][J] * rh.y;
+            }
+            w[q] = isq ? scaled(c[q][0], w[q]) : acc;
+        }
+        // the inverse is conj(FFT(conj)): conj(w) = (w.x, -w.y), then conj(-i k_la w) =
+        // (k w.y, k w.x), k_la = 0 on the Nyquist plane; first stage of the R2 x R1 plan:
+        // radix R2, out[i R2 + q]
+        float2 z[R2];
+#pragma unroll
+        for (int q = 0; q < R2; ++q) z[q] = make_float2(w[q].x, -w[q].y);
+        Dft<R2>::run(z);
+#pragma unroll
+        for (int q = 0; q < R2; ++q) Y1[(i * R2 + q) * ldy + f * NB + b] = z[q];
 #pragma unroll
         for (int q = 0; q < R2; ++q) {
             const int n = i + R1 * q;
-            const int cs = kEarly ? q : 0;     // slot of this node's rows
-            if (!kEarly) load_rows(q, 0);
-            for (int j = 0; j < r.nramp; ++j) {   // uniform trip count
-                const float v = rw[j] * ctab(n, r.ramp_row0 + j);
-#pragma unroll
-                for (int k = 0; k < NR; ++k) c[cs][k] += r.ramp_pair[j] == k ? v : 0.f;
-            }
-            float2 rh[NF];
-#pragma unroll
-            for (int f = 0; f < NF; ++f) rh[f] = w[f][q];
-#pragma unroll
-            for (int I = 0; I < TT; ++I) {
-                float2 acc = make_float2(0.f, 0.f);
-#pragma unroll
-                for (int J = 0; J < TT; ++J) {
-                    const int lo = I < J ? I : J, hi = I < J ? J : I;
-                    const float cc = c[cs][lo * TT - lo * (lo - 1) / 2 + (hi - lo)];
-                    acc.x += cc * rh[J].x; acc.y += cc * rh[J].y;
-                }
-                w[I][q] = acc;
-            }
-            if (CH) w[TT][q] = scaled(cq[cs], rh[TT]);
+            const float kl = 2 * n == N ? 0.f : r.kfac[la] * (float)(2 * n < N ? n : n - N);
+            z[q] = grad_line(kl, w[q]);
         }
-        // this thread's inverse lines (the inverse is conj(FFT(conj))): h = 0
-        // conj(w) = (w.x, -w.y), h = 1 conj(-i k_la w) = (k w.y, k w.x), k_la = 0 on the
-        // Nyquist plane; first stage of the R2 x R1 plan: radix R2, out[i R2 + q]
+        Dft<R2>::run(z);
 #pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            float2 z[R2];
-#pragma unroll
-            for (int q = 0; q < R2; ++q) {
-                const int n = i + R1 * q;
-                const float2 a = w[f][q];
-                const float kl = 2 * n == N ? 0.f : r.kfac[la] * (float)(2 * n < N ? n : n - N);
-                z[q] = h == 0 ? make_float2(a.x, -a.y) : grad_line(kl, a);
-            }
-            Dft<R2>::run(z);
-#pragma unroll
-            for (int q = 0; q < R2; ++q) Y1[(i * R2 + q) * ldy + (h * NF + f) * NB + b] = z[q];
-        }
+        for (int q = 0; q < R2; ++q) Y1[(i * R2 + q) * ldy + (NF + f) * NB + b] = z[q];
     }
     __syncthreads();
 
     // ---- C: stage 2 of the R2 x R1 plan (radix R1, twiddles w_N^{j r}, including the
     // unit ones of j = 0 as the staged pass multiplies them) -> rows j + R2 q.  One task
-    // per (column, j, line), spread over all threads.
-    // lanes: column, then line, then j (lines NB values apart in LDS: a wave's reads of
-    // one row fall in distinct banks)
+    // per (column, line, j), spread over all threads.
     for (int task = threadIdx.x; task < NB * R2 * 2 * NF; task += NT) {
         const int bc = task % NB, rest = task / NB, line = rest % (2 * NF), j = rest / (2 * NF);   // line = o NF + f
         if (bc >= nb) continue;
-        const int o = line >= NF ? 1 : 0, f = line - o * NF;
+        const int o = line >= NF ? 1 : 0, fl = line - o * NF;
         float2 z[R1];
 #pragma unroll
         for (int rr = 0; rr < R1; ++rr) z[rr] = Y1[(j + R2 * rr) * ldy + line * NB + bc];
 #pragma unroll
         for (int rr = 1; rr < R1; ++rr) z[rr] = cmul(z[rr], TW2[j * (R1 - 1) + rr - 1]);
         Dft<R1>::run(z);
-        const uint32_t o0 = (uint32_t)(f * D + (o == 0 ? 0 : la)) * Mhu + (uint32_t)j * Qu + (uint32_t)(q0 + bc);
+        const uint32_t o0 = (uint32_t)(fl * D + (o == 0 ? 0 : la)) * Mhu + (uint32_t)j * Qu + (uint32_t)(q0 + bc);
         const uint32_t step = (uint32_t)R2 * Qu;
 #pragma unroll
         for (int q = 0; q < R1; ++q) gst(at32(r.Gk, o0 + (uint32_t)q * step), conjf2(z[q]));
@@ -195,7 +198,7 @@ __device__ __forceinline__ void last_reg_block(const RepDev& r, int blk, float2*
 
 template <int R1, int R2, int NT, int TT, int CH, int CLS>
 __device__ __forceinline__ void last_reg_variant_block(const RepDev& r, int blk, float2* lds, int koff) {
-    if constexpr (last_reg_variant(R1, R2, TT, CH) && last_reg_class(R1, TT) == CLS)
+    if constexpr (last_reg_variant(R1, R2, TT, CH) && last_reg_class(R1, R2, TT) == CLS)
         last_reg_block<R1, R2, NT, TT, CH>(r, blk, lds, koff);
 }
 

@@ -95,29 +95,33 @@ hipError_t launch_mid_grad(const LaunchCtx& c);
 // 5-smooth lengths from 24 to 256 that two radices up to 16 make (as the planner splits
 // them), and 21, 28, 35 and 63 points.
 #define TILD_REG_PLANS(X) \
-    X(6, 4) X(5, 5) X(9, 3) X(6, 5) X(8, 4) X(6, 6) X(8, 5) X(9, 5) X(8, 6) X(10, 5) X(9, 6) X(10, 6) X(8, 8) \
+    X(8, 3) X(5, 5) X(9, 3) X(10, 3) X(8, 4) X(6, 6) X(8, 5) X(9, 5) X(16, 3) X(10, 5) X(9, 6) X(10, 6) X(8, 8) \
     X(9, 8) X(15, 5) X(10, 8) X(10, 9) X(12, 8) X(10, 10) X(12, 9) X(12, 10) X(16, 8) X(12, 12) X(15, 10) \
     X(16, 10) X(15, 12) X(16, 12) X(15, 15) X(16, 15) X(16, 16) X(7, 3) X(7, 4) X(7, 5) X(9, 7)
 // Fused last-axis pass with register-resident columns (fft_last.hpp): last axes with one
 // of those plans, at most four types (two on axes whose first radix is 12 or more) plus
-// charges.  Blocks of kLastRegThreads threads hold nl_last = kLastRegThreads / (2 R1)
+// charges.  Blocks of kLastRegThreads threads hold nl_last = last_reg_cols
 // columns; results agree with k_last_fused to rounding.
 constexpr int kLastRegThreads = 256;
 // the variants compiled in (plan R1 x R2, types, charge field): a thread of the middle
-// stage holds R2 values of every field, at most 40 of them
+// stage holds a coupling coefficient per type for each of its R2 values, at most 40
 __host__ __device__ constexpr bool last_reg_variant(int R1, int R2, int TT, int CH) {
-    return TT <= (R1 >= 12 ? 2 : 4) && (TT + CH) * R2 <= 40;
+    return TT <= (R1 >= 12 ? 2 : 4) && TT * R2 <= 40;
 }
-// the kernel instantiation of a variant: plans with R1 <= 10 and up to two types (class 0)
-// or three and four (class 1: over 256 registers, in blocks whose LDS leaves one to a CU
-// anyway), and the longer plans (class 2)
-__host__ __device__ constexpr int last_reg_class(int R1, int TT) { return R1 >= 12 ? 2 : (TT >= 3 ? 1 : 0); }
+// the kernel instantiation of a variant: plans of short axes with up to two types (class 0)
+// or three and four (class 1), and those with R1 >= 12 of the longer axes (class 2); 16 x 3
+// is with the short ones, so that a sweep of sides up to 50 launches one class
+__host__ __device__ constexpr int last_reg_class(int R1, int R2, int TT) {
+    return R1 * R2 > 64 && R1 >= 12 ? 2 : (TT >= 3 ? 1 : 0);
+}
 bool last_reg_plan(const AxisPlan& pl, int ntypes, int nf);
-inline int last_reg_lines(const AxisPlan& pl) { return kLastRegThreads / (2 * pl.rad[0]); }
-// the two exchange buffers, both stages' twiddles (2N - R1 - R2) and the ramp weights
+// columns of a block: one middle-stage thread per (column, i < R1, field)
+__host__ __device__ constexpr int last_reg_cols(int R1, int nf) { return kLastRegThreads / (R1 * nf); }
+inline int last_reg_lines(const AxisPlan& pl, int nf) { return last_reg_cols(pl.rad[0], nf); }
+// the two exchange buffers, the inverse stage's twiddles and the ramp weights
 inline size_t last_reg_lds_bytes(const AxisPlan& pl, int nf) {
-    const size_t N = (size_t)pl.N, nl = (size_t)last_reg_lines(pl);
-    return (N * (3 * (size_t)nf * nl + 2) + 2 * N) * sizeof(float2) + kMaxRamp * sizeof(float);
+    const size_t N = (size_t)pl.N, nl = (size_t)last_reg_lines(pl, nf);
+    return (N * (3 * (size_t)nf * nl + 2) + N) * sizeof(float2) + kMaxRamp * sizeof(float);
 }
 hipError_t launch_last_reg(const LaunchCtx& c, int koff, int cls);
 hipError_t launch_last_reg_0(const LaunchCtx& c, int koff);   // one per class, in files of their own
