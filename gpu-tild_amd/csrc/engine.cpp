@@ -549,7 +549,7 @@ int Batch::tile_regions(int id, bool bin_only, std::string& err) {
     if (R.h.spread_mode != 2) return 0;
     if (int rc = unclaim(id, err)) return rc;
     PhaseMap* mp = R.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].anyrec}; };
     HIPCHK(launch_tile_count(ctx(PH_TCOUNT), 0));
     HIPCHK(launch_tile_scan(ctx(PH_SCAN)));
     if (!bin_only) HIPCHK(launch_tile_regions(stream_, d_reps_, id));
@@ -671,7 +671,7 @@ int Batch::upload_desc(int id, std::string& err) {
 
 // ---------------------------------------------------------------- work maps
 int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& err, bool reorder_only) {
-    for (int p = 0; p < PH_COUNT; ++p) { maps[p].host.clear(); maps[p].lds = 0; maps[p].n = 0; maps[p].xfft = false; }
+    for (int p = 0; p < PH_COUNT; ++p) { maps[p].host.clear(); maps[p].lds = 0; maps[p].n = 0; maps[p].xfft = false; maps[p].anyrec = false; }
     for (int id : ids) {
         const Replica& R = *reps_[id];
         const RepDev& h = R.h;
@@ -681,6 +681,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
             maps[ph].lds = std::max(maps[ph].lds, lds);
         };
         add(PH_PART, R.nblk_part, 0);
+        maps[PH_PART].anyrec = maps[PH_PART].anyrec || h.P > 1;
         if (reorder_only) {   // the passes of reorder_set (tiled replicas)
             add(PH_TCOUNT, (h.ns + kCountBlock - 1) / kCountBlock, 0);
             add(PH_SCAN, 1, 0);
@@ -695,6 +696,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
             add(PH_SCAN, 1, 0);
             add(PH_TILE, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd));
             maps[PH_TILE].xfft = maps[PH_TILE].xfft || !h.plane_fwd;
+            maps[PH_TILE].anyrec = maps[PH_TILE].anyrec || !h.srec;
             if (R.reorder_every > 0) add(PH_RTILE, h.ntiles, 0);
         } else {
             add(PH_SPREADA, R.nblk_part, 0);
@@ -728,13 +730,16 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
     }
     // Deposit block size: 512 threads when the set's tiles hold ~600 beads or more on
     // average (one or two records per thread), else 256 (small tiles leave most of a
-    // larger block idle, and the deposit of a sweep of small replicas took twice as long)
+    // larger block idle, and the deposit of a sweep of small replicas took twice as long).
+    // A bead of a higher order counts by its nodes against order 1's.
     {
         long long beads = 0, tiles = 0;
         int want = -1;   // the block size the set's tiled replicas ask for, if they agree
         for (int id : ids)
             if (reps_[id]->h.spread_mode == 2) {
-                beads += reps_[id]->ns; tiles += reps_[id]->h.ntiles;
+                const long long np = std::max(reps_[id]->h.P, 1) + 1, d = reps_[id]->dim;
+                beads += (long long)reps_[id]->ns * (d == 3 ? np * np * np / 8 : np * np / 4);
+                tiles += reps_[id]->h.ntiles;
                 const int w = reps_[id]->dep_threads;
                 want = want == -1 ? w : (want == w ? want : 0);
             }
@@ -1065,7 +1070,7 @@ int Batch::build_tables(Replica& R, const System& S, std::string& err) {
 // device step counter plus k, and one launch at the end advances the counter.
 int Batch::enqueue_steps(SetMaps& m, int nsteps, bool integrate, bool write_forces, std::string& err) {
     PhaseMap* mp = m.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].anyrec}; };
     for (int k = 0; k < nsteps; ++k) {
         HIPCHK(launch_spread(ctx(PH_SPREADA), k));
         HIPCHK(launch_x_r2c(ctx(PH_XA), true, 0, nullptr, nullptr));
@@ -1203,7 +1208,7 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
     for (int s = 0; s < n && !rc; ++s) {
         bool used[kKernelPhases][kSlots] = {};
         auto ctx = [&](Phase p, int ph, int slot) {
-            LaunchCtx c{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft};
+            LaunchCtx c{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].anyrec};
             if (c.n > 0) { c.t0 = ev[ph][slot][0]; c.t1 = ev[ph][slot][1]; used[ph][slot] = true; }
             return c;
         };
@@ -1278,7 +1283,7 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
 int Batch::forward_spectra(int id, std::string& err) {
     Replica& R = *reps_[id];
     PhaseMap* mp = R.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].anyrec}; };
     HIPCHK(launch_x_r2c(ctx(PH_XP), false, 0, nullptr, nullptr));
     HIPCHK(launch_mid(ctx(PH_PY), 1, 0, 0, 0, nullptr));
     if (R.dim == 3) HIPCHK(launch_mid(ctx(PH_MIDZ_H), 2, 0, 0, 0, nullptr));
@@ -1292,7 +1297,7 @@ int Batch::properties(int id, tild_props* out, std::string& err) {
     HIPCHK(hipSetDevice(device_));
     if (int rc = forward_spectra(id, err)) return rc;
     PhaseMap* mp = R.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].anyrec}; };
     HIPCHK(launch_kprops(ctx(PH_KPROPS), R.nq));
     HIPCHK(launch_reduce_rows(stream_, R.h.partials, R.nq, R.h.nchunk, R.d_results));
     HIPCHK(launch_bond_props(ctx(PH_PART)));

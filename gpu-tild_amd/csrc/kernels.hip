@@ -750,6 +750,47 @@ __device__ __forceinline__ void gather_acc(const float (&W)[3][5], const float3 
             }
 }
 
+// The same in z slabs of NP x NP records, the records of a slab requested before the first
+// is used (orders 2-4, whose whole stencil would not fit the registers), in gather_sum's
+// order.
+template <int D, int NP, bool OFF32>
+__device__ __forceinline__ void gather_slabs(const RepDev& r, const float (&W)[3][5], const int (&n0)[3], size_t fb,
+                                             float (&acc)[3]) {
+    int yy[NP], xx[NP];
+    yy[0] = n0[1]; xx[0] = n0[0];
+#pragma unroll
+    for (int k = 1; k < NP; ++k) {
+        yy[k] = wrap_next(yy[k - 1], r.Ny);
+        xx[k] = wrap_next(xx[k - 1], r.Nx);
+    }
+    int zz = n0[2];
+    float wz[NP];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) wz[k] = W[2][k];
+    // rolled, the z weights shifted down a register per slab: one slab's records in flight
+#pragma unroll 1
+    for (int iz = 0; iz < (D == 3 ? NP : 1); ++iz) {
+        float3 g[NP * NP];
+#pragma unroll
+        for (int iy = 0; iy < NP; ++iy) {
+            const int rowb = (zz * r.Ny + yy[iy]) * r.Nx;
+#pragma unroll
+            for (int ix = 0; ix < NP; ++ix) g[iy * NP + ix] = gather_rec<NP, OFF32>(r.G3, fb, rowb + xx[ix]);
+        }
+        if constexpr (D == 3) zz = wrap_next(zz, r.Nz);
+#pragma unroll
+        for (int iy = 0; iy < NP; ++iy)
+#pragma unroll
+            for (int ix = 0; ix < NP; ++ix) {
+                const float w = D == 3 ? W[0][ix] * W[1][iy] * wz[0] : W[0][ix] * W[1][iy];
+                const float3 v = g[iy * NP + ix];
+                acc[0] += w * v.x; acc[1] += w * v.y; acc[2] += w * v.z;
+            }
+#pragma unroll
+        for (int k = 0; k + 1 < NP; ++k) wz[k] = wz[k + 1];
+    }
+}
+
 // Gathered force of one bead: its type's records, plus q times the charge records
 // (a second sweep, so that no more than one stencil of records is in flight).
 template <int D, int NP, bool OFF32>
@@ -856,7 +897,19 @@ __device__ __forceinline__ void particle_bead(const RepDev& r, int i, int write_
     float f[3] = {0.f, 0.f, 0.f};
     float z[4] = {0.f, 0.f, 0.f, 0.f}, zo[4] = {0.f, 0.f, 0.f, 0.f};
     const uint32_t stepc = (uint32_t)(step + 1);
-    if constexpr (NP > 0) {
+    if constexpr (NP > 2) {
+        if constexpr (INTEGRATE) {
+            normals4(r.seed, site, stepc, z);
+            if (r.any_gjf && stepc > 1u) normals4(r.seed, site, stepc - 1u, zo);
+        }
+        gather_slabs<D, NP, OFF32>(r, W, n0, (size_t)t * r.M, f);
+        if (charged) {
+            float fc[3] = {0.f, 0.f, 0.f};
+            gather_slabs<D, NP, OFF32>(r, W, n0, (size_t)r.ntypes * r.M, fc);
+#pragma unroll
+            for (int d = 0; d < D; ++d) f[d] += qi * fc[d];
+        }
+    } else if constexpr (NP > 0) {
         float3 g[(D == 3 ? NP : 1) * NP * NP];
         gather_load<D, NP, OFF32>(r, n0, (size_t)t * r.M, g);
         if constexpr (INTEGRATE) {
@@ -924,7 +977,9 @@ __device__ __forceinline__ void particle_bead(const RepDev& r, int i, int write_
 // CLAIM (integrating steps of LDS-tiled replicas): the block then claims the next
 // step's bucket slots from the positions it has just written, which takes the bucket
 // claim pass out of every step but the first of a run.
-template <bool INTEGRATE, bool CLAIM>
+// HIGH: some replica of the set has an order above 1, whose bodies (z slabs of 9, 16 or 25
+// records in flight) are in an instantiation of their own for their registers' sake.
+template <bool INTEGRATE, bool CLAIM, bool HIGH>
 __global__ void __launch_bounds__(256) k_particles(const RepDev* __restrict__ reps,
                                                    const WorkItem* __restrict__ wmap,
                                                    int write_forces, int koff) {
@@ -936,10 +991,21 @@ __global__ void __launch_bounds__(256) k_particles(const RepDev* __restrict__ re
     if (!CLAIM && !valid) return;
     const int step = r.step + koff;
     BeadNext nx{make_float4(0.f, 0.f, 0.f, 0.f), 0.f};
-    // unrolled bodies: the default order P = 1 on grids whose records fit 32-bit
-    // offsets, and P = 0; any other case takes the looped body
+    // unrolled bodies: the default order P = 1 and the orders above it on grids whose
+    // records fit 32-bit offsets, and P = 0; any other case takes the looped body
     if (valid) {
-        if (r.P == 1 && r.g3_off32) {
+        if (HIGH && r.P > 1 && r.g3_off32) {
+            if constexpr (HIGH) {
+                switch (r.P * 4 + r.dim) {
+                    case 11: particle_bead<INTEGRATE, 3, 3, true>(r, i, write_forces, step, nx); break;
+                    case 10: particle_bead<INTEGRATE, 2, 3, true>(r, i, write_forces, step, nx); break;
+                    case 15: particle_bead<INTEGRATE, 3, 4, true>(r, i, write_forces, step, nx); break;
+                    case 14: particle_bead<INTEGRATE, 2, 4, true>(r, i, write_forces, step, nx); break;
+                    case 19: particle_bead<INTEGRATE, 3, 5, true>(r, i, write_forces, step, nx); break;
+                    default: particle_bead<INTEGRATE, 2, 5, true>(r, i, write_forces, step, nx); break;
+                }
+            }
+        } else if (r.P == 1 && r.g3_off32) {
             if (r.dim == 3) particle_bead<INTEGRATE, 3, 2, true>(r, i, write_forces, step, nx);
             else particle_bead<INTEGRATE, 2, 2, true>(r, i, write_forces, step, nx);
         } else if (r.P == 0) {
@@ -1170,14 +1236,22 @@ hipError_t launch_mid_grad(const LaunchCtx& c) {
     TILD_LAUNCH(c, k_mid_grad<kGradThreads>, dim3(c.n), dim3(kGradThreads), c.lds, c.reps, c.wmap);
     CHECK_LAUNCH(); return hipSuccess;
 }
+template <bool INTEGRATE, bool CLAIM, bool HIGH>
+static void particles_launch(const LaunchCtx& c, int write_forces, int koff) {
+    TILD_LAUNCH(c, (k_particles<INTEGRATE, CLAIM, HIGH>), dim3(c.n), dim3(256), 0, c.reps, c.wmap, write_forces, koff);
+}
 hipError_t launch_particles(const LaunchCtx& c, bool integrate, int write_forces, int koff, bool claim) {
     if (!c.n) return hipSuccess;
-    if (integrate && claim)
-        TILD_LAUNCH(c, (k_particles<true, true>), dim3(c.n), dim3(256), 0, c.reps, c.wmap, write_forces, koff);
-    else if (integrate)
-        TILD_LAUNCH(c, (k_particles<true, false>), dim3(c.n), dim3(256), 0, c.reps, c.wmap, write_forces, koff);
-    else
-        TILD_LAUNCH(c, (k_particles<false, false>), dim3(c.n), dim3(256), 0, c.reps, c.wmap, write_forces, koff);
+    if (integrate && claim) {
+        if (c.anyrec) particles_launch<true, true, true>(c, write_forces, koff);
+        else particles_launch<true, true, false>(c, write_forces, koff);
+    } else if (integrate) {
+        if (c.anyrec) particles_launch<true, false, true>(c, write_forces, koff);
+        else particles_launch<true, false, false>(c, write_forces, koff);
+    } else {
+        if (c.anyrec) particles_launch<false, false, true>(c, write_forces, koff);
+        else particles_launch<false, false, false>(c, write_forces, koff);
+    }
     CHECK_LAUNCH(); return hipSuccess;
 }
 // avg_sk (Compute.cu:83-117): acc(k) += rho_t(k) rho_t(k) / M over the half spectrum,

@@ -66,6 +66,7 @@ struct LaunchCtx {
     hipEvent_t t0 = nullptr, t1 = nullptr;
     int threads = 0;    // block size where a pass has more than one (0: its default)
     bool xfft = true;   // tiled deposit: some replica of the set transforms along x in it
+    bool anyrec = true; // ... deposits position records; particles: some replica's order is above 1
 };
 
 // Launch on c.stream; with c.t0 set, through hipExtLaunchKernel, whose events take

@@ -303,32 +303,75 @@ __device__ __forceinline__ void deposit_srec(const SrecTile& c, const float4 rec
     }
 }
 
-__device__ __forceinline__ void deposit_record_any(const RepDev& r, const float4 rec, float qi,
-                                                   unsigned long long* patch, int y0, int z0, int By, int Bz) {
-    const int D = r.dim, P = r.P, Nx = r.Nx, T = r.ntypes;
-    const int tp = __float_as_int(rec.w);
+// Round to nearest of w 2^F (|w 2^F| < 2^51) as a 64-bit integer: adding 1.5 2^52 in FP64
+// leaves the integer in the low mantissa bits, ties to even, the same integer as
+// __float2ll_rn of the FP32 product (scaling by a power of two is exact) in a third of its
+// instructions.
+__device__ __forceinline__ unsigned long long round_scaled(float w, double scale) {
+    const double magic = 6755399441055744.0;   // 1.5 2^52
+    return (unsigned long long)(__double_as_longlong(__builtin_fma((double)w, scale, magic)) - __double_as_longlong(magic));
+}
+
+// Deposit one position record (x, y, z, type) of order P = NP - 1 (0 and 2-4) into the
+// tile's rows [f][lz][ly][x]; stencil rows outside the tile belong to a neighbouring tile
+// and are skipped.  Unrolled: with run-time loops a record took 1,300 instructions and more,
+// a third of them in the rounding to 64-bit integers (order 3 on a 48^3 grid, 41,480 beads:
+// 34.7 us).
+template <int NP, int D>
+__device__ __forceinline__ void deposit_posrec(const RepDev& r, const float4 rec, float qi,
+                                               unsigned long long* patch, int y0, int z0, int By, int Bz) {
+    const int Nx = r.Nx, tp = __float_as_int(rec.w);
     float W[3][5];
-    int n0[3];
-    n0[0] = stencil_1d(rec.x, r.dx[0], r.idx[0], Nx, P, W[0]);
-    n0[1] = stencil_1d(rec.y, r.dx[1], r.idx[1], r.Ny, P, W[1]);
-    if (D == 3) n0[2] = stencil_1d(rec.z, r.dx[2], r.idx[2], r.Nz, P, W[2]);
-    else { n0[2] = 0; W[2][0] = 1.f; }
-    const int nz = D == 3 ? P + 1 : 1;
-    for (int iz = 0, zz = n0[2]; iz < nz; ++iz, zz = wrap_next(zz, r.Nz)) {
+    int n0[3] = {0, 0, 0};
+    W[2][0] = 1.f;
+    n0[0] = stencil_1d(rec.x, r.dx[0], r.idx[0], Nx, NP - 1, W[0]);
+    n0[1] = stencil_1d(rec.y, r.dx[1], r.idx[1], r.Ny, NP - 1, W[1]);
+    if constexpr (D == 3) n0[2] = stencil_1d(rec.z, r.dx[2], r.idx[2], r.Nz, NP - 1, W[2]);
+    // a position that is not a number has weights that are none and deposits nothing, as
+    // where such a weight is converted to an integer
+    const float wsum = W[0][NP - 1] + W[1][NP - 1] + W[2][0] + (rec.x + rec.y + rec.z);
+    if (wsum != wsum) return;
+    int xx[NP];
+    xx[0] = n0[0];
+#pragma unroll
+    for (int k = 1; k < NP; ++k) xx[k] = wrap_next(xx[k - 1], Nx);
+    const double scale = (double)r.fix_scale;
+    const bool charged = r.trecq != nullptr;
+    const uint32_t trow = (uint32_t)(tp * Bz), qrow = (uint32_t)(r.ntypes * Bz);
+    int zz = n0[2];
+#pragma unroll
+    for (int iz = 0; iz < (D == 3 ? NP : 1); ++iz) {
         const int lz = zz - z0;
-        if (lz < 0 || lz >= Bz) continue;
-        for (int iy = 0, yy = n0[1]; iy <= P; ++iy, yy = wrap_next(yy, r.Ny)) {
+        zz = wrap_next(zz, r.Nz);
+        if ((unsigned)lz >= (unsigned)Bz) continue;
+        int yy = n0[1];
+#pragma unroll
+        for (int iy = 0; iy < NP; ++iy) {
             const int ly = yy - y0;
-            if (ly < 0 || ly >= By) continue;
-            unsigned long long* rowp = patch + ((size_t)(tp * Bz + lz) * By + ly) * Nx;
-            unsigned long long* rowq = patch + ((size_t)(T * Bz + lz) * By + ly) * Nx;
-            for (int ix = 0, xx = n0[0]; ix <= P; ++ix, xx = wrap_next(xx, Nx)) {
+            yy = wrap_next(yy, r.Ny);
+            if ((unsigned)ly >= (unsigned)By) continue;
+            unsigned long long* rowp = patch + ((trow + (uint32_t)lz) * (uint32_t)By + (uint32_t)ly) * (uint32_t)Nx;
+            unsigned long long* rowq = patch + ((qrow + (uint32_t)lz) * (uint32_t)By + (uint32_t)ly) * (uint32_t)Nx;
+#pragma unroll
+            for (int ix = 0; ix < NP; ++ix) {
+                // Wx Wy Wz in the reference's product order (device_grid_utils.cu:329)
                 const float w = D == 3 ? W[0][ix] * W[1][iy] * W[2][iz] : W[0][ix] * W[1][iy];
-                atomicAdd(rowp + xx, (unsigned long long)__float2ll_rn(w * r.fix_scale));
-                if (r.trecq)
-                    atomicAdd(rowq + xx, (unsigned long long)__float2ll_rn((w * qi) * r.fixq_scale));
+                atomicAdd(rowp + xx[ix], round_scaled(w, scale));
+                if (charged) atomicAdd(rowq + xx[ix], (unsigned long long)__float2ll_rn((w * qi) * r.fixq_scale));
             }
         }
+    }
+}
+
+template <int D>
+__device__ __forceinline__ void deposit_record_any(const RepDev& r, const float4 rec, float qi,
+                                                   unsigned long long* patch, int y0, int z0, int By, int Bz) {
+    switch (r.P) {
+        case 0: deposit_posrec<1, D>(r, rec, qi, patch, y0, z0, By, Bz); break;
+        case 1: deposit_record<2>(r, rec, qi, patch, y0, z0, By, Bz); break;
+        case 2: deposit_posrec<3, D>(r, rec, qi, patch, y0, z0, By, Bz); break;
+        case 3: deposit_posrec<4, D>(r, rec, qi, patch, y0, z0, By, Bz); break;
+        default: deposit_posrec<5, D>(r, rec, qi, patch, y0, z0, By, Bz); break;
     }
 }
 
@@ -368,14 +411,16 @@ __device__ __forceinline__ void load_srec4(const RepDev& r, int j0, int total, c
 // XFFT false: every replica of the set leaves the x transform to its forward plane pass,
 // so the block needs neither the transform's registers (79 VGPRs, six waves per SIMD)
 // nor its two LDS buffers (half of the block's LDS).
-template <int kDepositThreads, bool XFFT>
+// ANYREC: some replica of the set deposits position records (orders 0 and 2-4); without
+// them the kernel holds the stencil-record path only, and its registers.
+template <int kDepositThreads, bool XFFT, bool ANYREC>
 __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* __restrict__ reps,
                                                               const WorkItem* __restrict__ wmap, int koff) {
     extern __shared__ unsigned long long tile_lds[];
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
     warm_desc<0, 3, 4, 5, 6>(r);
-    const int D = r.dim, P = r.P, Nx = r.Nx, Nxh = r.Nxh;
+    const int D = r.dim, Nx = r.Nx, Nxh = r.Nxh;
     const int By = r.By, Bz = r.Bz, nf = r.nf;
     const int t = wi.blk, ty = t % r.nty, tz = t / r.nty;
     const int y0 = ty * By, z0 = tz * Bz;
@@ -434,7 +479,7 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
         prev = shift;
         total += n;
     }
-    if (r.srec) {
+    if (!ANYREC || r.srec) {
         // stencil records: the region decides the row offsets (own 0-3, y neighbour
         // 4-5, z neighbour 6-7, yz neighbour 8); four records per thread are in flight
         // at a time, the first four across the barrier that ends the clearing
@@ -455,14 +500,14 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
                 else deposit_srec<2>(c, rec[k], qi[k], patch, dy, 0);
             }
         }
-    } else {
+    } else if constexpr (ANYREC) {
         __syncthreads();
         for (int j = threadIdx.x; j < total; j += kDepositThreads) {
             const int p = region_pos(j, start, dsh);
             const float4 rec = gld(r.trec + p);
             const float qi = r.trecq ? G((const float*)r.trecq)[p] : 0.f;
-            if (P == 1) deposit_record<2>(r, rec, qi, patch, y0, z0, By, Bz);
-            else deposit_record_any(r, rec, qi, patch, y0, z0, By, Bz);
+            if (D == 3) deposit_record_any<3>(r, rec, qi, patch, y0, z0, By, Bz);
+            else deposit_record_any<2>(r, rec, qi, patch, y0, z0, By, Bz);
         }
     }
     // beads whose region was full: the same bucket test over the overflow list
@@ -474,14 +519,13 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
         if (src < 0) continue;
         const float4 rec = gld(r.tovf_rec + j);
         const float qi = r.trecq ? G((const float*)r.tovf_q)[j] : 0.f;
-        if (r.srec) {
+        if (!ANYREC || r.srec) {
             const int dy = (src >= 4 && src < 6) || src == 8 ? -By : 0, dz = src >= 6 ? -Bz : 0;
             if (D == 3) deposit_srec<3>(SrecTile(r, 3), rec, qi, patch, dy, dz);
             else deposit_srec<2>(SrecTile(r, 2), rec, qi, patch, dy, 0);
-        } else if (P == 1) {
-            deposit_record<2>(r, rec, qi, patch, y0, z0, By, Bz);
-        } else {
-            deposit_record_any(r, rec, qi, patch, y0, z0, By, Bz);
+        } else if constexpr (ANYREC) {
+            if (D == 3) deposit_record_any<3>(r, rec, qi, patch, y0, z0, By, Bz);
+            else deposit_record_any<2>(r, rec, qi, patch, y0, z0, By, Bz);
         }
     }
     __syncthreads();
@@ -584,15 +628,17 @@ hipError_t launch_tile_regions_set(const LaunchCtx& c) {
     hipLaunchKernelGGL(k_tile_regions_set, dim3(c.n), dim3(1024), 0, c.stream, c.reps, c.wmap);
     CHECK_LAUNCH(); return hipSuccess;
 }
+template <int NT, bool XFFT, bool ANYREC>
+static void deposit_launch(const LaunchCtx& c, int koff) {
+    TILD_LAUNCH(c, (k_tile_deposit<NT, XFFT, ANYREC>), dim3(c.n), dim3(NT), c.lds, c.reps, c.wmap, koff);
+}
 hipError_t launch_tile_deposit(const LaunchCtx& c, int koff) {
     if (!c.n) return hipSuccess;
-    if (c.threads >= 512) {
-        if (c.xfft) TILD_LAUNCH(c, (k_tile_deposit<512, true>), dim3(c.n), dim3(512), c.lds, c.reps, c.wmap, koff);
-        else TILD_LAUNCH(c, (k_tile_deposit<512, false>), dim3(c.n), dim3(512), c.lds, c.reps, c.wmap, koff);
-    } else {
-        if (c.xfft) TILD_LAUNCH(c, (k_tile_deposit<256, true>), dim3(c.n), dim3(256), c.lds, c.reps, c.wmap, koff);
-        else TILD_LAUNCH(c, (k_tile_deposit<256, false>), dim3(c.n), dim3(256), c.lds, c.reps, c.wmap, koff);
-    }
+    static void (*const kernels[8])(const LaunchCtx&, int) = {
+        deposit_launch<256, false, false>, deposit_launch<256, false, true>, deposit_launch<256, true, false>,
+        deposit_launch<256, true, true>,   deposit_launch<512, false, false>, deposit_launch<512, false, true>,
+        deposit_launch<512, true, false>,  deposit_launch<512, true, true>};
+    kernels[(c.threads >= 512 ? 4 : 0) + (c.xfft ? 2 : 0) + (c.anyrec ? 1 : 0)](c, koff);
     CHECK_LAUNCH(); return hipSuccess;
 }
 
