@@ -1397,37 +1397,34 @@ static void unpermute(const T* in, T* out, size_t n, const std::vector<int>& pid
     for (size_t p = 0; p < pid.size(); ++p)
         for (int d = 0; d < D; ++d) out[(size_t)pid[p] * D + d] = in[p * D + d];
 }
+int Batch::to_host(const Replica& R, const float* dev, float* host, std::string& err) {
+    const size_t bytes = (size_t)R.ns * R.dim * sizeof(float);
+    if (R.permuted) {   // a permuted replica has reorder buffers
+        HIPCHK(launch_site_order(stream_, dev, R.h.pid, R.h.XO_alt, R.ns, R.dim, true));
+        dev = R.h.XO_alt;
+    }
+    HIPCHK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream_));
+    HIPCHK(hipStreamSynchronize(stream_));
+    return 0;
+}
+
+int Batch::to_device(const Replica& R, const float* host, float* dev, std::string& err) {
+    const size_t bytes = (size_t)R.ns * R.dim * sizeof(float);
+    HIPCHK(hipMemcpyAsync(R.permuted ? R.h.XO_alt : dev, host, bytes, hipMemcpyHostToDevice, stream_));
+    if (R.permuted) HIPCHK(launch_site_order(stream_, R.h.XO_alt, R.h.pid, dev, R.ns, R.dim, false));
+    return 0;
+}
+
 int Batch::get_positions(int id, float* x, size_t n, std::string& err) {
     Replica* R = rep(id);
     if (!R || !x || n != (size_t)R->ns * R->dim) { err = "get_positions: size mismatch"; return -TILD_ERR_ARG; }
-    if (!R->permuted) {
-        HIPCHK(hipMemcpyAsync(x, R->h.X[R->step & 1], n * 4, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
-        return 0;
-    }
-    std::vector<float> tmp(n);
-    std::vector<int> pid;
-    HIPCHK(hipMemcpyAsync(tmp.data(), R->h.X[R->step & 1], n * 4, hipMemcpyDeviceToHost, stream_));
-    if (int rc = fetch_pid(*R, pid, err)) return rc;
-    unpermute(tmp.data(), x, n, pid, R->dim);
-    return 0;
+    return to_host(*R, R->h.X[R->step & 1], x, err);
 }
 
 int Batch::set_positions(int id, const float* x, size_t n, std::string& err) {
     Replica* R = rep(id);
     if (!R || !x || n != (size_t)R->ns * R->dim) { err = "set_positions: size mismatch"; return -TILD_ERR_ARG; }
-    std::vector<float> tmp;
-    const float* src = x;
-    if (R->permuted) {   // slot p holds site pid[p]
-        std::vector<int> pid;
-        if (int rc = fetch_pid(*R, pid, err)) return rc;
-        tmp.resize(n);
-        const int D = R->dim;
-        for (int p = 0; p < R->ns; ++p)
-            for (int d = 0; d < D; ++d) tmp[(size_t)p * D + d] = x[(size_t)pid[p] * D + d];
-        src = tmp.data();
-    }
-    HIPCHK(hipMemcpyAsync(R->h.X[R->step & 1], src, n * 4, hipMemcpyHostToDevice, stream_));
+    if (int rc = to_device(*R, x, R->h.X[R->step & 1], err)) return rc;
     HIPCHK(hipMemsetAsync(R->h.XO, 0, n * 4, stream_));   // xo = x
     if (int rc = tile_regions(id, false, err)) return rc;   // new positions, new bucket sizes
     HIPCHK(hipStreamSynchronize(stream_));
@@ -1437,12 +1434,7 @@ int Batch::set_positions(int id, const float* x, size_t n, std::string& err) {
 int Batch::get_state(int id, int* step, float* xo, size_t n, std::string& err) {
     Replica* R = rep(id);
     if (!R || !step || !xo || n != (size_t)R->ns * R->dim) { err = "get_state: size mismatch"; return -TILD_ERR_ARG; }
-    std::vector<float> tmp(n);
-    HIPCHK(hipMemcpyAsync(tmp.data(), R->h.XO, n * 4, hipMemcpyDeviceToHost, stream_));
-    HIPCHK(hipStreamSynchronize(stream_));
-    std::vector<int> pid;
-    if (R->permuted) { if (int rc = fetch_pid(*R, pid, err)) return rc; }
-    unpermute(tmp.data(), xo, n, pid, R->dim);
+    if (int rc = to_host(*R, R->h.XO, xo, err)) return rc;
     *step = R->step;
     return 0;
 }
@@ -1458,18 +1450,7 @@ int Batch::set_state(int id, int step, const float* xo, size_t n, std::string& e
     PhaseMap* mp = R->maps;
     const LaunchCtx rctx{d_reps_, mp[PH_SCAN].dev, mp[PH_SCAN].n, 0, stream_};
     if (tiled) HIPCHK(launch_tile_reset(rctx, 0));
-    std::vector<float> tmp;
-    const float* src = xo;
-    if (R->permuted) {   // slot p holds site pid[p]
-        std::vector<int> pid;
-        if (int rc = fetch_pid(*R, pid, err)) return rc;
-        tmp.resize(n);
-        const int D = R->dim;
-        for (int p = 0; p < R->ns; ++p)
-            for (int d = 0; d < D; ++d) tmp[(size_t)p * D + d] = xo[(size_t)pid[p] * D + d];
-        src = tmp.data();
-    }
-    HIPCHK(hipMemcpyAsync(R->h.XO, src, n * 4, hipMemcpyHostToDevice, stream_));
+    if (int rc = to_device(*R, xo, R->h.XO, err)) return rc;
     // the positions live in the buffer of the step's parity
     if ((step & 1) != (R->step & 1))
         HIPCHK(hipMemcpyAsync(R->h.X[step & 1], R->h.X[R->step & 1], n * 4, hipMemcpyDeviceToDevice, stream_));
@@ -1483,17 +1464,7 @@ int Batch::set_state(int id, int step, const float* xo, size_t n, std::string& e
 int Batch::get_forces(int id, float* f, size_t n, std::string& err) {
     Replica* R = rep(id);
     if (!R || !f || n != (size_t)R->ns * R->dim) { err = "get_forces: size mismatch"; return -TILD_ERR_ARG; }
-    if (!R->permuted) {
-        HIPCHK(hipMemcpyAsync(f, R->d_fout, n * 4, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
-        return 0;
-    }
-    std::vector<float> tmp(n);
-    std::vector<int> pid;
-    HIPCHK(hipMemcpyAsync(tmp.data(), R->d_fout, n * 4, hipMemcpyDeviceToHost, stream_));
-    if (int rc = fetch_pid(*R, pid, err)) return rc;
-    unpermute(tmp.data(), f, n, pid, R->dim);
-    return 0;
+    return to_host(*R, R->d_fout, f, err);
 }
 
 int Batch::get_density(int id, int type, float* rho, size_t n, std::string& err) {

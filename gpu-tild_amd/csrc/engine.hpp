@@ -227,6 +227,11 @@ private:
     int unclaim(int id, std::string& err);
     static void drop_graphs(SetMaps& m);
     int fetch_pid(const Replica& R, std::vector<int>& pid, std::string& err);
+    // per-bead device array (dim floats) <-> host array in site order.  A permuted replica's
+    // beads change order on the device, through the spare buffer of its spatial reorder
+    // (which only the next reorder writes, and the stream orders it after the copy).
+    int to_host(const Replica& R, const float* dev, float* host, std::string& err);
+    int to_device(const Replica& R, const float* host, float* dev, std::string& err);
     void free_maps(PhaseMap* maps);
 };
 

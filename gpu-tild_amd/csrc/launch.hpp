@@ -197,6 +197,10 @@ struct ReorderBufs {
 };
 size_t reorder_tmp_bytes(int ns, int bits);
 
+// Site-order copy of a permuted per-bead array of D floats: dst[pid[p]] = src[p] (to_site)
+// or dst[p] = src[pid[p]].
+hipError_t launch_site_order(hipStream_t s, const float* src, const int* pid, float* dst, int ns, int D, bool to_site);
+
 // Neighbour-list build (device buffers, all indexed by site id except cell_slots).
 struct NlistArgs {
     const unsigned char* member;   // ns group-membership flags

@@ -101,6 +101,24 @@ __device__ __forceinline__ void reorder_swap(RepDev& r) {
 
 __global__ void k_reorder_swap(RepDev* reps, int rep) { reorder_swap(reps[rep]); }
 
+// Site-order copies of a permuted per-bead array for the getters (to_site: dst[pid[p]] =
+// src[p]) and the setters (dst[p] = src[pid[p]]); D floats per bead.
+__global__ void __launch_bounds__(256) k_site_order(const float* __restrict__ src, const int* __restrict__ pid,
+                                                    float* __restrict__ dst, int ns, int D, int to_site) {
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= ns) return;
+    const size_t s = (size_t)pid[p] * D, q = (size_t)p * D;
+    for (int d = 0; d < D; ++d) {
+        if (to_site) dst[s + d] = src[q + d];
+        else dst[q + d] = src[s + d];
+    }
+}
+
+hipError_t launch_site_order(hipStream_t s, const float* src, const int* pid, float* dst, int ns, int D, bool to_site) {
+    hipLaunchKernelGGL(k_site_order, dim3((ns + 255) / 256), dim3(256), 0, s, src, pid, dst, ns, D, to_site ? 1 : 0);
+    return hipGetLastError();
+}
+
 // ---- tiled replicas: reuse the last step's bucket order -----------------------------
 // The step's binning left every bead's bucket (tile, halo class) and slot in tkey and
 // the bucket offsets in toff, so the beads of tile t occupy [toff[4t], toff[4t+4]) of
