@@ -513,12 +513,15 @@ int Batch::add_plain(const System& S, uint32_t seed, std::string& err) {
     // forward plane pass: tiled 3D replicas with even Ny and even tile height (the
     // row pairing (y, y+1) of the tiled x transform), planes within one block's LDS
     h.plane_fwd = 0;
-    if (D == 3 && h.spread_mode == 2 && tune_.plane >= 0 && h.Ny % 2 == 0 && h.By % 2 == 0 &&
-        plane_r2c_lds(h) <= kPlaneLds)
+    // its register-resident form: square planes with a two-stage plan, odd sides too (whose
+    // last row pairs with zeros)
+    const bool preg = !tune_.staged && h.grid_off32 && plane_reg_plan(h.ax[0], h.ax[1]) &&
+                      plane_reg_lds_bytes(h.ax[0]) <= kPlaneLds;
+    const bool even = h.Ny % 2 == 0;
+    if (D == 3 && h.spread_mode == 2 && tune_.plane >= 0 &&
+        (even ? h.By % 2 == 0 && plane_r2c_lds(h) <= kPlaneLds : preg))
         h.plane_fwd = 1;
-    // its register-resident form: square planes with a two-stage plan
-    h.plane_reg = h.plane_fwd && !tune_.staged && h.grid_off32 && plane_reg_plan(h.ax[0], h.ax[1]) &&
-                  plane_reg_lds_bytes(h.ax[0]) <= kPlaneLds ? 1 : 0;
+    h.plane_reg = h.plane_fwd && preg ? 1 : 0;
     // the y inverse and the x C2R as one pass per (field, z) plane: square planes with an
     // even two-stage plan, no field phases (whose records need the densities)
     h.plane_inv = D == 3 && !tune_.staged && h.grid_off32 && !h.FPtab && plane_inv_plan(h.ax[0], h.ax[1]) &&
@@ -711,7 +714,9 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         }
         if (D == 3) {
             MidGeom g = mid_grad_geom(h);
-            if (h.plane_inv) add(PH_PLANEI, h.nf * h.Nz, plane_inv_lds_bytes(h.ax[1]));
+            if (h.plane_inv)
+                add(plane_inv_threads(h.ax[1].rad[0], h.ax[1].rad[1]) == kPlaneInvWide ? PH_PLANEIW : PH_PLANEI, h.nf * h.Nz,
+                    plane_inv_lds_bytes(h.ax[1]));
             else if (h.grad_reg) add(PH_MIDY_GR, h.nf * h.Nz * grad_reg_chunks(h.ax[1], h.Nxh), grad_reg_lds_bytes(h.ax[1]));
             else add(PH_MIDY_G, g.nouter * g.nchunk, lds_bytes(g.N, 3 * g.nl));
             MidGeom gz = mid_geom(h, 2, h.nf);
@@ -751,7 +756,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
     // records; for the FFT passes adjacent column batches, whose rows share cache lines
     // that a single L2 then fetches once.
     for (Phase ph : {PH_PART, PH_TCOUNT, PH_SPREADA, PH_TILE, PH_XA, PH_XP, PH_MIDY_H, PH_MIDY_G, PH_MIDY_GR,
-                     PH_MIDZ_H, PH_PY, PH_LAST, PH_LASTR, PH_LASTR4, PH_LASTRW, PH_C2R, PH_PLANEF, PH_PLANER, PH_PLANEI}) {
+                     PH_MIDZ_H, PH_PY, PH_LAST, PH_LASTR, PH_LASTR4, PH_LASTRW, PH_C2R, PH_PLANEF, PH_PLANER, PH_PLANEI, PH_PLANEIW}) {
         std::vector<WorkItem>& v = maps[ph].host;
         const size_t n = v.size(), q = n / kXcds, rm = n % kXcds;
         if (n < 2 * (size_t)kXcds) continue;
@@ -764,7 +769,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
     }
     for (int p = 0; p < PH_COUNT; ++p) {
         maps[p].n = (int)maps[p].host.size();
-        if (maps[p].lds > ((p == PH_PLANEF || p == PH_PLANER || p == PH_PLANEI || p == PH_LAST || p == PH_LASTR || p == PH_LASTR4 || p == PH_LASTRW) ? kPlaneLds : (size_t)kMaxLds)) { err = "pass needs more LDS than a block may use"; return -TILD_ERR_UNSUPPORTED; }
+        if (maps[p].lds > ((p == PH_PLANEF || p == PH_PLANER || p == PH_PLANEI || p == PH_PLANEIW || p == PH_LAST || p == PH_LASTR || p == PH_LASTR4 || p == PH_LASTRW) ? kPlaneLds : (size_t)kMaxLds)) { err = "pass needs more LDS than a block may use"; return -TILD_ERR_UNSUPPORTED; }
         if (maps[p].dev && (!reorder_only || maps[p].cap < maps[p].n)) {
             // reused buffers are last read by the previous reorder's launches
             HIPCHK(hipStreamSynchronize(stream_));
@@ -1085,7 +1090,8 @@ int Batch::enqueue_steps(SetMaps& m, int nsteps, bool integrate, bool write_forc
         HIPCHK(launch_mid_grad(ctx(PH_MIDY_G)));
         HIPCHK(launch_grad_reg(ctx(PH_MIDY_GR)));
         HIPCHK(launch_x_c2r(ctx(PH_C2R), true, 0, nullptr, nullptr));
-        HIPCHK(launch_plane_inv(ctx(PH_PLANEI)));
+        HIPCHK(launch_plane_inv(ctx(PH_PLANEI), false));
+        HIPCHK(launch_plane_inv(ctx(PH_PLANEIW), true));
         // integrating steps claim the next step's records; a force evaluation leaves
         // positions and records as they are
         HIPCHK(launch_particles(ctx(PH_PART), integrate, write_forces ? 1 : 0, k, integrate));
@@ -1229,7 +1235,8 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
         ok(launch_mid_grad(ctx(PH_MIDY_G, 4, 0)));
         ok(launch_grad_reg(ctx(PH_MIDY_GR, 4, 1)));
         ok(launch_x_c2r(ctx(PH_C2R, 5, 0), true, 0, nullptr, nullptr));
-        ok(launch_plane_inv(ctx(PH_PLANEI, 5, 1)));
+        ok(launch_plane_inv(ctx(PH_PLANEI, 5, 1), false));
+        ok(launch_plane_inv(ctx(PH_PLANEIW, 5, 2), true));
         ok(launch_particles(ctx(PH_PART, 6, 0), true, 0, 0, true));
         ok(launch_advance(stream_, d_reps_, m->d_ids, m->nids, 1, ev[7][0][0], ev[7][0][1]));
         used[7][0] = m->nids > 0;

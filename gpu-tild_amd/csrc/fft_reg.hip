@@ -121,7 +121,8 @@ __global__ void __launch_bounds__(NT) k_grad_reg(const RepDev* __restrict__ reps
 // ------------------------------------------------------------------ plane forward (3D)
 // x R2C and y FFT of one (field, z) density plane (the operation of k_plane_r2c,
 // kernels.hip) for square planes Nx = Ny with a two-stage plan R1 x R2:
-//   A  task (pair j, i < R2): rows 2j and 2j+1 at x = i + R2 r as one complex line, DFT_R1;
+//   A  task (pair j, i < R2): rows 2j and 2j+1 at x = i + R2 r as one complex line (an odd
+//      side's last row with zeros), DFT_R1;
 //   B  task (j, i < R1): twiddles, DFT_R2 -> Z_j(k), k = i + R1 q; exchange;
 //   C  task (column k < Nxh, i < R2): the half spectra of rows y = i + R2 r unpacked on
 //      the fly from Z_{y/2}(k) and Z_{y/2}(N - k), DFT_R1;
@@ -136,7 +137,7 @@ __device__ __forceinline__ float half_of(float a) {
 
 template <int R1, int R2, int NT>
 __device__ __forceinline__ void plane_reg_block(const RepDev& r, int blk, float2* lds) {
-    constexpr int N = R1 * R2, NP = N / 2, NXH = N / 2 + 1, ldp = NP | 1, ldc = NXH | 1;
+    constexpr int N = R1 * R2, NP = (N + 1) / 2, NXH = N / 2 + 1, ldp = NP | 1, ldc = NXH | 1;
     constexpr int NT1 = R1 * (R2 - 1), LDA = (N * ldp > N * ldc) ? N * ldp : N * ldc;
     const int z = blk % r.Nz, f = blk / r.Nz;
     float2* Xa = lds;                  // x stage-1 output, later the y stage-1 output (N x ldc)
@@ -156,7 +157,9 @@ __device__ __forceinline__ void plane_reg_block(const RepDev& r, int blk, float2
 #pragma unroll
         for (int rr = 0; rr < R1; ++rr) {
             const uint32_t o = pbase + (uint32_t)(2 * j * N + i + R2 * rr);
-            v[rr] = make_float2(G(at32((const float*)r.rho, o))[0], G(at32((const float*)r.rho, o + N))[0]);
+            const float a = G(at32((const float*)r.rho, o))[0];
+            const float c = N % 2 == 0 || 2 * j + 1 < N ? G(at32((const float*)r.rho, o + N))[0] : 0.f;
+            v[rr] = make_float2(a, c);
         }
         Dft<R1>::run(v);
 #pragma unroll
@@ -410,7 +413,7 @@ __global__ void __launch_bounds__(NT) k_plane_inv(const RepDev* __restrict__ rep
     warm_desc<0, 1, 3, 6, 7>(r);
     switch (r.reg_key[1]) {   // uniform per block
 #define TILD_CASE(A, B) \
-    case A * 32 + B: if constexpr ((A * B / 2 + 1) * (A > B ? A : B) <= NT) plane_inv_block<A, B, NT>(r, wi.blk, lds); break;
+    case A * 32 + B: if constexpr (plane_inv_threads(A, B) == NT) plane_inv_block<A, B, NT>(r, wi.blk, lds); break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
         default: break;   // excluded by plane_inv_plan on the host
@@ -419,19 +422,22 @@ __global__ void __launch_bounds__(NT) k_plane_inv(const RepDev* __restrict__ rep
 
 bool plane_inv_plan(const AxisPlan& px, const AxisPlan& py) {
     if (!(px.N == py.N && grad_reg_plan(py))) return false;
-    const int rmax = py.rad[0] > py.rad[1] ? py.rad[0] : py.rad[1];
-    return (py.N / 2 + 1) * rmax <= kPlaneInvThreads && plane_inv_lds_bytes(py) <= kPlaneLds / 2;
+    return plane_inv_threads(py.rad[0], py.rad[1]) > 0;
 }
 
-hipError_t launch_plane_inv(const LaunchCtx& c) {
+hipError_t launch_plane_inv(const LaunchCtx& c, bool wide) {
     if (!c.n) return hipSuccess;
-    TILD_LAUNCH(c, k_plane_inv<kPlaneInvThreads>, dim3(c.n), dim3(kPlaneInvThreads), c.lds, c.reps, c.wmap);
+    if (wide) TILD_LAUNCH(c, k_plane_inv<kPlaneInvWide>, dim3(c.n), dim3(kPlaneInvWide), c.lds, c.reps, c.wmap);
+    else TILD_LAUNCH(c, k_plane_inv<kPlaneInvThreads>, dim3(c.n), dim3(kPlaneInvThreads), c.lds, c.reps, c.wmap);
     return hipGetLastError();
 }
 
 hipError_t configure_plane_inv() {
-    return hipFuncSetAttribute((const void*)k_plane_inv<kPlaneInvThreads>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)(kPlaneLds / 2));
+    hipError_t e = hipFuncSetAttribute((const void*)k_plane_inv<kPlaneInvThreads>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kPlaneLds / 2));
+    if (e != hipSuccess) return e;
+    return hipFuncSetAttribute((const void*)k_plane_inv<kPlaneInvWide>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)kPlaneLds);
 }
 
 bool plane_reg_plan(const AxisPlan& px, const AxisPlan& py) {

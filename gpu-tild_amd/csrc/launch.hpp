@@ -147,21 +147,30 @@ hipError_t launch_grad_reg(const LaunchCtx& c);
 constexpr int kPlaneRegThreads = 512;
 bool plane_reg_plan(const AxisPlan& px, const AxisPlan& py);
 inline size_t plane_reg_lds_bytes(const AxisPlan& pl) {
-    const size_t N = (size_t)pl.N, ldp = (size_t)((pl.N / 2) | 1), ldc = (size_t)((pl.N / 2 + 1) | 1);
+    const size_t N = (size_t)pl.N, ldp = (size_t)(((pl.N + 1) / 2) | 1), ldc = (size_t)((pl.N / 2 + 1) | 1);
     return (N * (ldp > ldc ? ldp : ldc) + N * ldp + 2 * N) * sizeof(float2);
 }
 hipError_t launch_plane_reg(const LaunchCtx& c);
 hipError_t configure_plane_reg();
 // Register-resident inverse plane pass (y inverse + x C2R into the gather records) of
 // square planes with a two-stage plan: one block of kPlaneInvThreads threads per (field,
-// z) plane, two blocks to a CU.
-constexpr int kPlaneInvThreads = 512;
-inline size_t plane_inv_lds_bytes(const AxisPlan& pl) {
-    const size_t N = (size_t)pl.N, la = (size_t)((3 * (pl.N / 2 + 1)) | 1);
-    return (N * la + (size_t)pl.rad[0] * (pl.rad[1] - 1)) * sizeof(float2);
+// z) plane, two blocks to a CU; planes whose y stages outgrow those threads or whose LDS
+// leaves one block to a CU (75 to 108 points a side) take kPlaneInvWide threads, which
+// fill the CU.
+constexpr int kPlaneInvThreads = 512, kPlaneInvWide = 1024;
+__host__ __device__ constexpr size_t plane_inv_lds(int R1, int R2) {
+    const size_t N = (size_t)R1 * R2, la = (3 * (N / 2 + 1)) | 1;
+    return (N * la + (size_t)R1 * (R2 - 1)) * sizeof(float2);
 }
+// the block size of a plan (0: no such pass)
+__host__ __device__ constexpr int plane_inv_threads(int R1, int R2) {
+    const int tasks = (R1 * R2 / 2 + 1) * (R1 > R2 ? R1 : R2);
+    return tasks <= kPlaneInvThreads && plane_inv_lds(R1, R2) <= kPlaneLds / 2 ? kPlaneInvThreads
+           : (tasks <= kPlaneInvWide && plane_inv_lds(R1, R2) <= kPlaneLds ? kPlaneInvWide : 0);
+}
+inline size_t plane_inv_lds_bytes(const AxisPlan& pl) { return plane_inv_lds(pl.rad[0], pl.rad[1]); }
 bool plane_inv_plan(const AxisPlan& px, const AxisPlan& py);
-hipError_t launch_plane_inv(const LaunchCtx& c);
+hipError_t launch_plane_inv(const LaunchCtx& c, bool wide);
 hipError_t configure_plane_inv();
 hipError_t configure_last_reg();
 hipError_t launch_plane_r2c(const LaunchCtx& c);

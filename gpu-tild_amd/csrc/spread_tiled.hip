@@ -554,6 +554,16 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
         }
         return;
     }
+    if (plane_fwd && off32) {   // odd rows: one node per task
+        Digits2 gq(threadIdx.x, kDepositThreads, dNx);
+        for (int task = threadIdx.x; task < rows * Nx; task += kDepositThreads, gq.step()) {
+            const int n = gq.lo, rr = gq.hi;
+            const double inv = rr < trows ? inv_t : inv_q;
+            G(at32(rho, (uint32_t)rowoff[rr] + (uint32_t)n))[0] =
+                (float)((double)(long long)patch[(size_t)rr * Nx + n] * inv);
+        }
+        return;
+    }
     // task = j * Nx + n; rows 2j and 2j + 1 are (f, lz, ly) with ly fastest
     Digits2 gt(threadIdx.x, kDepositThreads, dNx);
     for (int task = threadIdx.x; task < npairs * Nx; task += kDepositThreads, gt.step()) {
