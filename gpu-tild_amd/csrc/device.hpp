@@ -99,7 +99,7 @@ struct alignas(64) RepDev {
     // line 7: FFT passes
     int ctab_charge;           // row of the charge kernel in Ctab (or -1)
     int nramp, ramp_row0;      // ramped pair styles, see below
-    int reg_key[3];            // axis plans of two stages: R1 * 32 + R2 (else 0)
+    int reg_key[3];            // axes of a register-resident plan: R1 * 32 + R2 (else 0)
     const float2* reg_tw[3];   // and their second stage's twiddles
     const float2* reg_twr;     // the same of the last axis' inverse plan axr
     int nl_last;   // batch columns per block, fused last-axis pass
@@ -113,6 +113,7 @@ struct alignas(64) RepDev {
     int grad_reg;  // 1: the y inverse of the gradient spectra runs register-resident (k_grad_reg)
     int plane_reg; // 1: the forward plane pass runs register-resident (k_plane_reg)
     int plane_inv; // 1: y inverse and x C2R run as one register-resident plane pass (k_plane_inv)
+    int c2r_reg;   // 1: the x C2R runs register-resident (k_c2r_reg)
     // FFT plans (x, y, z)
     AxisPlan ax[3];
     AxisPlan axr;  // inverse plan of the last axis: a two-stage plan reversed, else ax[dim - 1]

@@ -107,8 +107,11 @@ int make_axis_plan(int N, AxisPlan& pl, std::vector<float2>& tw, std::string& er
 }
 
 // ---------------------------------------------------------------- tiles
-size_t tile_lds_bytes(int Nx, int nf, int By, int Bz, bool plane_fwd) {
+size_t tile_lds_bytes(int Nx, int nf, int By, int Bz, bool plane_fwd, bool xreg) {
     size_t rows = (size_t)nf * By * Bz;
+    if (!plane_fwd && xreg)
+        return rows * Nx * sizeof(unsigned long long) + fft_buf_bytes(Nx, (int)((rows + 1) / 2)) + Nx * sizeof(float2) +
+               rows * sizeof(int);
     return rows * Nx * sizeof(unsigned long long) +
            (plane_fwd ? rows * sizeof(int) : lds_bytes(Nx, (int)((rows + 1) / 2)));
 }
@@ -293,7 +296,7 @@ int Batch::add_plain(const System& S, uint32_t seed, std::string& err) {
     h.axr.tw = d_tw + toff_r;
     if (D == 2) h.ax[2] = h.ax[1];
     for (int a = 0; a < D; ++a)
-        if (h.ax[a].nst == 2) {
+        if (!tune_.staged && grad_reg_plan(h.ax[a])) {   // the plans compiled in
             h.reg_key[a] = h.ax[a].rad[0] * 32 + h.ax[a].rad[1];
             h.reg_tw[a] = h.ax[a].tw + h.ax[a].tw_off[1];
         }
@@ -527,6 +530,18 @@ int Batch::add_plain(const System& S, uint32_t seed, std::string& err) {
     h.plane_inv = D == 3 && !tune_.staged && h.grid_off32 && !h.FPtab && plane_inv_plan(h.ax[0], h.ax[1]) &&
                   h.ax[0].rad[0] == h.ax[1].rad[0] && h.ax[0].rad[1] == h.ax[1].rad[1] ? 1 : 0;
 
+    // the register form of the x C2R into the records, where the plane pass does not run: one
+    // stage-B task per thread, and no more rows per block than leave a block for every CU
+    // (a small launch is bound by one block's chain of phases)
+    h.c2r_reg = h.reg_key[0] && h.grid_off32 && !h.FPtab && !h.plane_inv ? 1 : 0;
+    if (h.c2r_reg) {
+        int nr = std::max(1, kC2rRegThreads / (nc * h.ax[0].rad[0]));
+        nr = std::max(1, std::min(nr, rows / 256));
+        if (tune_.c2r_rows > 0) nr = std::min(tune_.c2r_rows, rows);
+        while (nr > 1 && c2r_reg_lds_bytes(h.Nx, nr * nc) > kMaxLds) --nr;
+        h.nr_c2r = nr;
+    }
+
     int id = -1;
     for (int k = 0; k < (int)reps_.size(); ++k) if (!reps_[k]) { id = k; break; }
     if (id < 0) { id = (int)reps_.size(); reps_.emplace_back(); }
@@ -697,7 +712,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         if (h.spread_mode == 2) {
             add(PH_TCOUNT, (h.ns + kCountBlock - 1) / kCountBlock, 0);
             add(PH_SCAN, 1, 0);
-            add(PH_TILE, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd));
+            add(PH_TILE, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd, h.reg_key[0] && h.grid_off32));
             maps[PH_TILE].xfft = maps[PH_TILE].xfft || !h.plane_fwd;
             maps[PH_TILE].anyrec = maps[PH_TILE].anyrec || !h.srec;
             if (R.reorder_every > 0) add(PH_RTILE, h.ntiles, 0);
@@ -730,7 +745,8 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         }
         else add(PH_LAST, (Q + h.nl_last - 1) / h.nl_last, last_lds_bytes(Nla, h.nf, h.last_dirs, h.nl_last));
         const int nc = (h.nf * D + 1) / 2;
-        if (!h.plane_inv) add(PH_C2R, (rows + h.nr_c2r - 1) / h.nr_c2r, lds_bytes(h.Nx, h.nr_c2r * nc));
+        if (h.c2r_reg) add(PH_C2RR, (rows + h.nr_c2r - 1) / h.nr_c2r, c2r_reg_lds_bytes(h.Nx, h.nr_c2r * nc));
+        else if (!h.plane_inv) add(PH_C2R, (rows + h.nr_c2r - 1) / h.nr_c2r, lds_bytes(h.Nx, h.nr_c2r * nc));
         add(PH_KPROPS, h.nchunk > 0 ? h.nchunk : 1, 0);
     }
     // Deposit block size: 512 threads when the set's tiles hold ~600 beads or more on
@@ -756,7 +772,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
     // records; for the FFT passes adjacent column batches, whose rows share cache lines
     // that a single L2 then fetches once.
     for (Phase ph : {PH_PART, PH_TCOUNT, PH_SPREADA, PH_TILE, PH_XA, PH_XP, PH_MIDY_H, PH_MIDY_G, PH_MIDY_GR,
-                     PH_MIDZ_H, PH_PY, PH_LAST, PH_LASTR, PH_LASTR4, PH_LASTRW, PH_C2R, PH_PLANEF, PH_PLANER, PH_PLANEI, PH_PLANEIW}) {
+                     PH_MIDZ_H, PH_PY, PH_LAST, PH_LASTR, PH_LASTR4, PH_LASTRW, PH_C2R, PH_C2RR, PH_PLANEF, PH_PLANER, PH_PLANEI, PH_PLANEIW}) {
         std::vector<WorkItem>& v = maps[ph].host;
         const size_t n = v.size(), q = n / kXcds, rm = n % kXcds;
         if (n < 2 * (size_t)kXcds) continue;
@@ -1090,6 +1106,7 @@ int Batch::enqueue_steps(SetMaps& m, int nsteps, bool integrate, bool write_forc
         HIPCHK(launch_mid_grad(ctx(PH_MIDY_G)));
         HIPCHK(launch_grad_reg(ctx(PH_MIDY_GR)));
         HIPCHK(launch_x_c2r(ctx(PH_C2R), true, 0, nullptr, nullptr));
+        HIPCHK(launch_c2r_reg(ctx(PH_C2RR)));
         HIPCHK(launch_plane_inv(ctx(PH_PLANEI), false));
         HIPCHK(launch_plane_inv(ctx(PH_PLANEIW), true));
         // integrating steps claim the next step's records; a force evaluation leaves
@@ -1235,6 +1252,7 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
         ok(launch_mid_grad(ctx(PH_MIDY_G, 4, 0)));
         ok(launch_grad_reg(ctx(PH_MIDY_GR, 4, 1)));
         ok(launch_x_c2r(ctx(PH_C2R, 5, 0), true, 0, nullptr, nullptr));
+        ok(launch_c2r_reg(ctx(PH_C2RR, 5, 3)));
         ok(launch_plane_inv(ctx(PH_PLANEI, 5, 1), false));
         ok(launch_plane_inv(ctx(PH_PLANEIW, 5, 2), true));
         ok(launch_particles(ctx(PH_PART, 6, 0), true, 0, 0, true));

@@ -32,7 +32,7 @@ constexpr int kProfPhases = 9;   // claim, deposit, forward plane, last_fused, y
 // skip MIDY_G and C2R); PLANEF: x R2C + y FFT of tiled 3D replicas with even Ny
 // (their deposit writes densities only and they skip MIDY_H).
 enum Phase { PH_PART = 0, PH_SPREADA, PH_XA, PH_XP, PH_SCAN, PH_TILE, PH_MIDY_H, PH_MIDY_G,
-             PH_MIDZ_H, PH_PY, PH_LAST, PH_C2R, PH_PLANEF, PH_TCOUNT, PH_KPROPS, PH_RTILE, PH_LASTR, PH_MIDY_GR, PH_PLANER, PH_LASTR4, PH_LASTRW, PH_PLANEI, PH_PLANEIW, PH_COUNT };
+             PH_MIDZ_H, PH_PY, PH_LAST, PH_C2R, PH_PLANEF, PH_TCOUNT, PH_KPROPS, PH_RTILE, PH_LASTR, PH_MIDY_GR, PH_PLANER, PH_LASTR4, PH_LASTRW, PH_PLANEI, PH_PLANEIW, PH_C2RR, PH_COUNT };
 
 struct PhaseMap {
     std::vector<WorkItem> host;
@@ -252,6 +252,7 @@ bool choose_tiles(int dim, const int* Nx, int P, int nf, int target_tiles, int w
                   int& By, int& Bz);
 // LDS of a deposit block: its accumulator rows, plus the x transform's two buffers or,
 // where the plane pass transforms (plane_fwd), the table of its rows
-size_t tile_lds_bytes(int Nx, int nf, int By, int Bz, bool plane_fwd = false);
+// (xreg: the register form of the x transform, one buffer, twiddles and a row table)
+size_t tile_lds_bytes(int Nx, int nf, int By, int Bz, bool plane_fwd = false, bool xreg = false);
 
 }  // namespace tild

@@ -420,6 +420,134 @@ __global__ void __launch_bounds__(NT) k_plane_inv(const RepDev* __restrict__ rep
     }
 }
 
+// ------------------------------------------------------------------ x C2R
+// Inverse x transform of the half spectra into the gather records (the operation of
+// k_x_c2r, kernels.hip) for two-stage x plans, where the plane pass does not run (2D, and
+// planes of unequal sides); nr_c2r rows per block, nc complex lines per row:
+//   A  task (line b, i < R2): Z = A + i B at k = i + R2 r of the full spectrum straight
+//      from the half spectra (the upper half by Hermitian symmetry), DFT_R1; exchange;
+//   B  task (b, i < R1): twiddles, DFT_R2 -> the real lines, over the values the task read;
+//   C  the records (g_x, g_y, g_z), stored in order.
+// Two barriers; the staged form has four and waits for its second stage's twiddles.  It
+// reads each half-spectrum value twice (the second time from cache), which is why grids of
+// many planes take the plane pass instead.
+namespace {
+__device__ __forceinline__ float2 x_gradient(float kx, float2 a) {   // -i k_x a
+#pragma clang fp contract(off)
+    return make_float2(kx * a.y, -kx * a.x);
+}
+
+template <int R1, int R2, int NT>
+__device__ __forceinline__ void c2r_reg_block(const RepDev& r, int blk, float2* lds) {
+    constexpr int N = R1 * R2, NXH = N / 2 + 1, NT1 = R1 * (R2 - 1);
+    static_assert(NT1 <= NT, "c2r_reg_block: one twiddle per thread");
+    const int D = r.dim, NL = r.nf * D, nc = (NL + 1) / 2;
+    const int nrows = r.M / N;                 // rows of one field
+    const int row0 = blk * r.nr_c2r;
+    const int rows = min(r.nr_c2r, nrows - row0);
+    const int nb = rows * nc, ldb = nb | 1;
+    float2* X = lds;                           // N x ldb
+    float2* TW = X + N * ((r.nr_c2r * nc) | 1);
+    float2 tw = make_float2(0.f, 0.f);
+    if ((int)threadIdx.x < NT1) tw = gld(r.reg_tw[0] + threadIdx.x);
+    const float kf = r.kfac[0];
+    const uint32_t line = (uint32_t)nrows * (uint32_t)NXH;   // one line's half spectra
+    const FastDiv dnc(nc);
+    const bool fuse = D == 2 && r.nf == 2;
+    for (int task = threadIdx.x; task < nb * R2; task += NT) {
+        const int i = task % R2, b = task / R2;
+        int j;
+        const int rr0 = dnc.div(b, j);
+        const int la = 2 * j, lb = la + 1;
+        const bool two = lb < NL;
+        const bool xa = D == 3 ? la % 3 == 0 : true, xb = D == 3 && lb % 3 == 0;   // x derivatives (2D: every even line)
+        const uint32_t o = (uint32_t)la * line + (uint32_t)(row0 + rr0) * (uint32_t)NXH;
+        float2 A[R1], B[R1];
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) {
+            const int kn = i + R2 * rr;
+            const uint32_t kk = (uint32_t)(kn >= NXH ? N - kn : kn);
+            A[rr] = gld(at32((const float2*)r.Gk, o + kk));
+            B[rr] = two ? gld(at32((const float2*)r.Gk, o + line + kk)) : make_float2(0.f, 0.f);
+        }
+        float2 v[R1];
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) {
+            const int kn = i + R2 * rr;
+            const bool upper = kn >= NXH;
+            const int kk = upper ? N - kn : kn;
+            const bool self = kk == 0 || 2 * kk == N;             // self-conjugate column
+            const float kx = self && kk != 0 ? 0.f : kf * (float)kk;
+            float2 a = A[rr], c = B[rr];
+            if (xa) a = x_gradient(kx, a);
+            if (xb) c = x_gradient(kx, c);
+            if (self) { a.y = 0.f; c.y = 0.f; }
+            // conj(Z) is transformed (the inverse as conj(FFT(conj))); products round before
+            // they are added, as in the staged form, except where that form fuses them: the
+            // lower half's real part with two fields in 2D
+            const float re = fuse ? __builtin_fmaf(kx, A[rr].y, -c.y) : a.x - c.y;
+            v[rr] = upper ? make_float2(a.x + c.y, a.y - c.x) : make_float2(re, -(a.y + c.x));
+        }
+        Dft<R1>::run(v);
+#pragma unroll
+        for (int q = 0; q < R1; ++q) X[(i * R1 + q) * ldb + b] = v[q];
+    }
+    if ((int)threadIdx.x < NT1) TW[threadIdx.x] = tw;
+    __syncthreads();
+    const FastDiv dnb(nb);
+    for (int task = threadIdx.x; task < nb * R1; task += NT) {
+        int b;
+        const int i = dnb.div(task, b);
+        float2 w[R2];
+#pragma unroll
+        for (int rr = 0; rr < R2; ++rr) w[rr] = X[(i + R1 * rr) * ldb + b];
+#pragma unroll
+        for (int rr = 1; rr < R2; ++rr) w[rr] = cmul(w[rr], lds_twiddle(TW + i * (R2 - 1) + rr - 1));
+        Dft<R2>::run(w);
+#pragma unroll
+        for (int q = 0; q < R2; ++q) X[(i + R1 * q) * ldb + b] = w[q];
+    }
+    __syncthreads();
+    const FastDiv dnf(r.nf);
+    for (int task = threadIdx.x; task < rows * r.nf * N; task += NT) {
+        const int x = task % N;
+        int f;
+        const int rr0 = dnf.div(task / N, f);
+        float g[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (d < D) {
+                const int l = f * D + d;
+                const float2 z = X[x * ldb + rr0 * nc + l / 2];
+                g[d] = (l & 1) ? -z.y : z.x;   // conj of the forward result
+            }
+        }
+        const uint32_t fn = (uint32_t)f * (uint32_t)r.M + (uint32_t)(row0 + rr0) * (uint32_t)N + (uint32_t)x;
+        gst3((float*)((char*)r.G3 + ((fn << 3) + (fn << 2))), g[0], g[1], g[2]);   // 12 fn bytes, no mask (see k_x_c2r)
+    }
+}
+}  // namespace
+
+template <int NT>
+__global__ void __launch_bounds__(NT) k_c2r_reg(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
+    extern __shared__ float2 lds[];
+    const WorkItem wi = wmap[blockIdx.x];
+    const RepDev& r = reps[wi.rep];
+    warm_desc<0, 1, 3, 6, 7, 8>(r);
+    switch (r.reg_key[0]) {   // uniform per block
+#define TILD_CASE(A, B) case A * 32 + B: c2r_reg_block<A, B, NT>(r, wi.blk, lds); break;
+        TILD_REG_PLANS(TILD_CASE)
+#undef TILD_CASE
+        default: break;   // reg_key holds compiled plans only
+    }
+}
+
+hipError_t launch_c2r_reg(const LaunchCtx& c) {
+    if (!c.n) return hipSuccess;
+    TILD_LAUNCH(c, k_c2r_reg<kC2rRegThreads>, dim3(c.n), dim3(kC2rRegThreads), c.lds, c.reps, c.wmap);
+    return hipGetLastError();
+}
+
 bool plane_inv_plan(const AxisPlan& px, const AxisPlan& py) {
     if (!(px.N == py.N && grad_reg_plan(py))) return false;
     return plane_inv_threads(py.rad[0], py.rad[1]) > 0;

@@ -23,6 +23,7 @@
 // a new replica.  Bucket and halo classes are defined in tile_dev.hpp.
 #include "device.hpp"
 #include "fft_dev.hpp"
+#include "fft_reg_dev.hpp"
 #include "launch.hpp"
 #include "tile_dev.hpp"
 
@@ -404,6 +405,70 @@ __device__ __forceinline__ void load_srec4(const RepDev& r, int j0, int total, c
     }
 }
 
+// Densities of a tile's rows and their x R2C for axes with a two-stage plan R1 x R2, row
+// pairs as complex lines with columns in registers between the stages (the transform of
+// the LDS-staged form, in three phases instead of five):
+//   A  task (pair j, i < R2): rows 2j and 2j + 1 at x = i + R2 r from the fixed-point
+//      rows, written to rho on the way; DFT_R1; exchange;
+//   B  task (j, i < R1): twiddles, DFT_R2 -> Z_j(k), over the values the task read;
+//   C  the two rows' half spectra from Z_k and Z_{N-k}, stored.
+// X: N x ldb exchange; TW: w_N^{i r}; rowid: global row (f, z, y) of each tile row.
+template <int R1, int R2, int NT>
+__device__ __forceinline__ void deposit_xfft(const RepDev& r, const unsigned long long* patch, float2* X, const float2* TW,
+                                             const int* rowid, int rows, int trows) {
+    constexpr int N = R1 * R2, NXH = N / 2 + 1;
+    const int npairs = (rows + 1) / 2, ldb = npairs | 1;
+    const double inv_t = r.fix_inv, inv_q = r.fixq_inv;
+    float* const rho = r.rho;
+    for (int task = threadIdx.x; task < npairs * R2; task += NT) {
+        const int i = task % R2, j = task / R2;
+        const int ra = 2 * j;
+        const bool two = ra + 1 < rows;
+        const double ia = ra < trows ? inv_t : inv_q, ib = ra + 1 < trows ? inv_t : inv_q;
+        const uint32_t oa = (uint32_t)rowid[ra] * (uint32_t)N, ob = two ? (uint32_t)rowid[ra + 1] * (uint32_t)N : 0u;
+        float2 v[R1];
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) {
+            const int n = i + R2 * rr;
+            v[rr].x = (float)((double)(long long)patch[ra * N + n] * ia);
+            G(at32(rho, oa + (uint32_t)n))[0] = v[rr].x;
+            v[rr].y = 0.f;
+            if (two) {
+                v[rr].y = (float)((double)(long long)patch[(ra + 1) * N + n] * ib);
+                G(at32(rho, ob + (uint32_t)n))[0] = v[rr].y;
+            }
+        }
+        Dft<R1>::run(v);
+#pragma unroll
+        for (int q = 0; q < R1; ++q) X[(i * R1 + q) * ldb + j] = v[q];
+    }
+    __syncthreads();
+    const FastDiv dnp(npairs);
+    for (int task = threadIdx.x; task < npairs * R1; task += NT) {
+        int j;
+        const int i = dnp.div(task, j);
+        float2 w[R2];
+#pragma unroll
+        for (int rr = 0; rr < R2; ++rr) w[rr] = X[(i + R1 * rr) * ldb + j];
+#pragma unroll
+        for (int rr = 1; rr < R2; ++rr) w[rr] = cmul(w[rr], lds_twiddle(TW + i * (R2 - 1) + rr - 1));
+        Dft<R2>::run(w);
+#pragma unroll
+        for (int q = 0; q < R2; ++q) X[(i + R1 * q) * ldb + j] = w[q];
+    }
+    __syncthreads();
+    for (int task = threadIdx.x; task < npairs * NXH; task += NT) {
+        const int k = task % NXH, j = task / NXH;
+        const float2 Zk = X[k * ldb + j];
+        const float2 Zm = X[(k == 0 ? 0 : N - k) * ldb + j];
+        gst(at32(r.H, (uint32_t)rowid[2 * j] * (uint32_t)NXH + (uint32_t)k),
+            make_float2(0.5f * (Zk.x + Zm.x), 0.5f * (Zk.y - Zm.y)));
+        if (2 * j + 1 < rows)
+            gst(at32(r.H, (uint32_t)rowid[2 * j + 1] * (uint32_t)NXH + (uint32_t)k),
+                make_float2(0.5f * (Zk.y + Zm.y), 0.5f * (Zm.x - Zk.x)));
+    }
+}
+
 // Deposit one tile's rows and transform them along x.  NT = 512 for tiles of about
 // 1,000 beads plus their halo share (three blocks of 512 fit a CU; on the 640,000-bead
 // melt 17.5 us, against 19.6 with 256 threads and 22.8 with 1,024, where one block
@@ -419,7 +484,8 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
     extern __shared__ unsigned long long tile_lds[];
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
-    warm_desc<0, 3, 4, 5, 6>(r);
+    if (XFFT) warm_desc<0, 3, 4, 5, 6, 7>(r);
+    else warm_desc<0, 3, 4, 5, 6>(r);
     const int D = r.dim, Nx = r.Nx, Nxh = r.Nxh;
     const int By = r.By, Bz = r.Bz, nf = r.nf;
     const int t = wi.blk, ty = t % r.nty, tz = t / r.nty;
@@ -460,6 +526,18 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
     // where the plane pass transforms the densities the FFT scratch is free: it holds
     // the first density element of each tile row (f, lz, ly)
     int* const rowoff = (int*)fbuf;
+    // register form of the x transform: its twiddles and row table sit behind the exchange
+    const bool xreg = XFFT && !plane_fwd && r.reg_key[0] && r.grid_off32;
+    float2* const xtw = fbuf + (size_t)Nx * (((rows + 1) / 2) | 1);
+    int* const rowid = (int*)(xtw + Nx);
+    if (XFFT && xreg) {
+        const int ntw = Nx - (r.reg_key[0] >> 5);   // R1 (R2 - 1)
+        for (int k = threadIdx.x; k < ntw; k += kDepositThreads) xtw[k] = gld(r.reg_tw[0] + k);
+        for (int rr = threadIdx.x; rr < rows; rr += kDepositThreads) {
+            const int ly = rr % By, lz = (rr / By) % Bz, f = rr / (By * Bz);
+            rowid[rr] = (f * r.Nz + z0 + lz) * Ny + (y0 + ly);
+        }
+    }
     if (plane_fwd)
         for (int rr = threadIdx.x; rr < rows; rr += kDepositThreads) {
             const int ly = rr % By, lz = (rr / By) % Bz, f = rr / (By * Bz);
@@ -530,6 +608,15 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
     }
     __syncthreads();
     // densities of the tile rows -> rho and the x-axis R2C (pairs of rows)
+    if (XFFT && xreg) {
+        switch (r.reg_key[0]) {   // uniform
+#define TILD_CASE(A, B) case A * 32 + B: deposit_xfft<A, B, kDepositThreads>(r, patch, fbuf, xtw, rowid, rows, T * By * Bz); break;
+            TILD_REG_PLANS(TILD_CASE)
+#undef TILD_CASE
+            default: break;   // reg_key holds compiled plans only
+        }
+        return;
+    }
     const int npairs = (rows + 1) / 2;
     const int ldb = npairs | 1;
     const FastDiv dNx(Nx), dNxh(Nxh), dBy(By), dBz(Bz);
