@@ -99,8 +99,8 @@ struct alignas(64) RepDev {
     // line 7: FFT passes
     int ctab_charge;           // row of the charge kernel in Ctab (or -1)
     int nramp, ramp_row0;      // ramped pair styles, see below
-    int reg_key[3];            // axes of a register-resident plan: R1 * 32 + R2 (else 0)
-    const float2* reg_tw[3];   // and their second stage's twiddles
+    int reg_key[3];            // axes of a compiled register plan: reg_plan_key (else 0)
+    const float2* reg_tw[3];   // and the twiddles of their second group of stages
     const float2* reg_twr;     // the same of the last axis' inverse plan axr
     int nl_last;   // batch columns per block, fused last-axis pass
     int last_dirs; // directions per inverse batch of the fused last-axis pass (1..dim)
@@ -114,6 +114,9 @@ struct alignas(64) RepDev {
     int plane_reg; // 1: the forward plane pass runs register-resident (k_plane_reg)
     int plane_inv; // 1: y inverse and x C2R run as one register-resident plane pass (k_plane_inv)
     int c2r_reg;   // 1: the x C2R runs register-resident (k_c2r_reg)
+    int plane_rect;   // 1: the forward plane pass of other planes runs register-resident (k_plane_rect)
+    int yfwd_reg;  // 1: the forward y pass runs register-resident (k_yfwd_reg)
+    int plane_all; // 1: y inverse and x C2R of all fields run as one plane pass (k_plane_all)
     // FFT plans (x, y, z)
     AxisPlan ax[3];
     AxisPlan axr;  // inverse plan of the last axis: a two-stage plan reversed, else ax[dim - 1]

@@ -29,7 +29,7 @@ namespace {
 struct RadixSearch {
     static constexpr int kDepth = 16;
     int best[kDepth], nbest = -1, cur[kDepth], ncur = 0;
-    void run(int n, const int* radices, int nrad) {
+    void run(int n) {
         if (n == 1) {
             if (nbest < 0 || ncur < nbest || (ncur == nbest && cur[0] < best[0])) {
                 for (int i = 0; i < ncur; ++i) best[i] = cur[i];
@@ -38,24 +38,13 @@ struct RadixSearch {
             return;
         }
         if ((nbest >= 0 && ncur + 1 > nbest) || ncur == kDepth) return;
-        for (int k = 0; k < nrad; ++k) {
-            const int R = radices[k];
+        static const int kRadices[] = {16, 10, 8, 7, 5, 4, 3, 2};
+        for (int R : kRadices)
             if (n % R == 0 && (ncur == 0 || R <= cur[ncur - 1])) {
                 cur[ncur++] = R;
-                run(n / R, radices, nrad);
+                run(n / R);
                 --ncur;
             }
-        }
-    }
-    // Radices 16, 10, 8, 7, 5, 4, 3 and 2 first: they make two stages of 24, 30 and 48
-    // points too, where 6 x 4, 6 x 5 and 8 x 6 measured the same, and the transform of a
-    // length keeps its rounding.  The lengths they leave at three stages (27, 36, 45, 60,
-    // 96, 192, 225, ...) take 6, 9, 12 and 15 as well.
-    void plan(int n) {
-        static const int kFirst[] = {16, 10, 8, 7, 5, 4, 3, 2};
-        static const int kAll[] = {16, 15, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
-        run(n, kFirst, 8);
-        if (nbest < 0 || nbest > 2) run(n, kAll, 12);
     }
 };
 }  // namespace
@@ -65,7 +54,7 @@ const char* plan_axis(int N, AxisPlan& pl, float2* tw, int* ntw) {
     pl.N = N;
     if (N < 1 || N > kFftBudget) return "FFT length outside [1, 2048]";
     RadixSearch rs;
-    if (N > 1) rs.plan(N);
+    if (N > 1) rs.run(N);
     else rs.nbest = 0;
     if (rs.nbest < 0) return "FFT length has a prime factor above 7";
     if (rs.nbest > kMaxStages) return "too many FFT stages";
@@ -296,11 +285,12 @@ int Batch::add_plain(const System& S, uint32_t seed, std::string& err) {
     h.axr.tw = d_tw + toff_r;
     if (D == 2) h.ax[2] = h.ax[1];
     for (int a = 0; a < D; ++a)
-        if (!tune_.staged && grad_reg_plan(h.ax[a])) {   // the plans compiled in
-            h.reg_key[a] = h.ax[a].rad[0] * 32 + h.ax[a].rad[1];
-            h.reg_tw[a] = h.ax[a].tw + h.ax[a].tw_off[1];
+        if (const RegDims rd = reg_dims(h.ax[a]); !tune_.staged && rd.key) {   // the plans compiled in
+            h.reg_key[a] = rd.key;
+            h.reg_tw[a] = h.ax[a].tw + h.ax[a].tw_off[rd.group2];
         }
     if (h.axr.nst == 2) h.reg_twr = h.axr.tw + h.axr.tw_off[1];
+    else h.reg_twr = h.reg_tw[lax];
 
     // chunking of each pass
     const int rows = h.M / h.Nx;
@@ -516,26 +506,29 @@ int Batch::add_plain(const System& S, uint32_t seed, std::string& err) {
     // forward plane pass: tiled 3D replicas with even Ny and even tile height (the
     // row pairing (y, y+1) of the tiled x transform), planes within one block's LDS
     h.plane_fwd = 0;
-    // its register-resident form: square planes with a two-stage plan, odd sides too (whose
-    // last row pairs with zeros)
-    const bool preg = !tune_.staged && h.grid_off32 && plane_reg_plan(h.ax[0], h.ax[1]) &&
-                      plane_reg_lds_bytes(h.ax[0]) <= kPlaneLds;
-    const bool even = h.Ny % 2 == 0;
-    if (D == 3 && h.spread_mode == 2 && tune_.plane >= 0 &&
-        (even ? h.By % 2 == 0 && plane_r2c_lds(h) <= kPlaneLds : preg))
+    if (D == 3 && h.spread_mode == 2 && tune_.plane >= 0 && h.Ny % 2 == 0 && h.By % 2 == 0 &&
+        plane_r2c_lds(h) <= kPlaneLds)
         h.plane_fwd = 1;
-    h.plane_reg = h.plane_fwd && preg ? 1 : 0;
+    // its register-resident forms: square planes of the kept plans, and any others of
+    // compiled plans; without a plane pass the y transform alone
+    h.plane_reg = h.plane_fwd && !tune_.staged && h.grid_off32 && plane_reg_plan(h.ax[0], h.ax[1]) &&
+                  plane_reg_lds_bytes(h.ax[0]) <= kPlaneLds ? 1 : 0;
+    h.plane_rect = h.plane_fwd && !h.plane_reg && h.grid_off32 && h.reg_key[0] && h.reg_key[1] &&
+                   plane_rect_lds_bytes(h.Nx, h.Ny) <= kPlaneLds ? 1 : 0;
+    h.yfwd_reg = D == 3 && !h.plane_fwd && h.grid_off32 && h.reg_key[1] && grad_reg_plan(h.ax[1]) ? 1 : 0;
     // the y inverse and the x C2R as one pass per (field, z) plane: square planes with an
     // even two-stage plan, no field phases (whose records need the densities)
     h.plane_inv = D == 3 && !tune_.staged && h.grid_off32 && !h.FPtab && plane_inv_plan(h.ax[0], h.ax[1]) &&
                   h.ax[0].rad[0] == h.ax[1].rad[0] && h.ax[0].rad[1] == h.ax[1].rad[1] ? 1 : 0;
+    h.plane_all = D == 3 && !tune_.staged && h.grid_off32 && !h.FPtab && h.grad_reg && plane_all_plan(h.ax[0], h.ax[1], h.nf) ? 1 : 0;
 
     // the register form of the x C2R into the records, where the plane pass does not run: one
     // stage-B task per thread, and no more rows per block than leave a block for every CU
     // (a small launch is bound by one block's chain of phases)
-    h.c2r_reg = h.reg_key[0] && h.grid_off32 && !h.FPtab && !h.plane_inv ? 1 : 0;
+    h.c2r_reg = h.reg_key[0] && h.grid_off32 && !h.FPtab && !h.plane_inv && !h.plane_all ? 1 : 0;
     if (h.c2r_reg) {
-        int nr = std::max(1, kC2rRegThreads / (nc * h.ax[0].rad[0]));
+        const RegDims rd = reg_dims(h.ax[0]);
+        int nr = std::max(1, kC2rRegThreads / (nc * std::max(rd.R1, rd.R2)));
         nr = std::max(1, std::min(nr, rows / 256));
         if (tune_.c2r_rows > 0) nr = std::min(tune_.c2r_rows, rows);
         while (nr > 1 && c2r_reg_lds_bytes(h.Nx, nr * nc) > kMaxLds) --nr;
@@ -724,14 +717,15 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
             MidGeom g = mid_geom(h, 1, h.nf);
             add(PH_PY, g.nouter * g.nchunk, lds_bytes(g.N, g.nl));
             if (D == 3 && h.plane_reg) add(PH_PLANER, h.nf * h.Nz, plane_reg_lds_bytes(h.ax[0]));
+            else if (D == 3 && h.plane_rect) add(PH_PLANERECT, h.nf * h.Nz, plane_rect_lds_bytes(h.Nx, h.Ny));
+            else if (D == 3 && h.yfwd_reg) add(PH_YFWD, h.nf * h.Nz * grad_reg_chunks(h.ax[1], h.Nxh), yfwd_reg_lds_bytes(h.ax[1]));
             else if (D == 3 && h.plane_fwd) add(PH_PLANEF, h.nf * h.Nz, plane_r2c_lds(h));
             else if (D == 3) add(PH_MIDY_H, g.nouter * g.nchunk, lds_bytes(g.N, g.nl));
         }
         if (D == 3) {
             MidGeom g = mid_grad_geom(h);
-            if (h.plane_inv)
-                add(plane_inv_threads(h.ax[1].rad[0], h.ax[1].rad[1]) == kPlaneInvWide ? PH_PLANEIW : PH_PLANEI, h.nf * h.Nz,
-                    plane_inv_lds_bytes(h.ax[1]));
+            if (h.plane_inv) add(PH_PLANEI, h.nf * h.Nz, plane_inv_lds_bytes(h.ax[1]));
+            else if (h.plane_all) add(plane_all_threads(h.Ny, h.nf) == kPlaneInvWide ? PH_PLANEAW : PH_PLANEA, h.Nz, plane_all_lds(h.Ny, h.nf));
             else if (h.grad_reg) add(PH_MIDY_GR, h.nf * h.Nz * grad_reg_chunks(h.ax[1], h.Nxh), grad_reg_lds_bytes(h.ax[1]));
             else add(PH_MIDY_G, g.nouter * g.nchunk, lds_bytes(g.N, 3 * g.nl));
             MidGeom gz = mid_geom(h, 2, h.nf);
@@ -740,13 +734,13 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         const int la = D - 1, Nla = la == 2 ? h.Nz : h.Ny, Q = la == 2 ? h.Ny * h.Nxh : h.Nxh;
         if (h.last_reg) {
             const Phase cls[3] = {PH_LASTR, PH_LASTR4, PH_LASTRW};
-            add(cls[last_reg_class(h.ax[la].rad[0], h.ax[la].rad[1], h.ntypes)], (Q + h.nl_last - 1) / h.nl_last,
+            add(cls[last_reg_class(h.ax[la].N, h.ntypes)], (Q + h.nl_last - 1) / h.nl_last,
                 last_reg_lds_bytes(h.ax[la], h.nf));
         }
         else add(PH_LAST, (Q + h.nl_last - 1) / h.nl_last, last_lds_bytes(Nla, h.nf, h.last_dirs, h.nl_last));
         const int nc = (h.nf * D + 1) / 2;
         if (h.c2r_reg) add(PH_C2RR, (rows + h.nr_c2r - 1) / h.nr_c2r, c2r_reg_lds_bytes(h.Nx, h.nr_c2r * nc));
-        else if (!h.plane_inv) add(PH_C2R, (rows + h.nr_c2r - 1) / h.nr_c2r, lds_bytes(h.Nx, h.nr_c2r * nc));
+        else if (!h.plane_inv && !h.plane_all) add(PH_C2R, (rows + h.nr_c2r - 1) / h.nr_c2r, lds_bytes(h.Nx, h.nr_c2r * nc));
         add(PH_KPROPS, h.nchunk > 0 ? h.nchunk : 1, 0);
     }
     // Deposit block size: 512 threads when the set's tiles hold ~600 beads or more on
@@ -772,7 +766,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
     // records; for the FFT passes adjacent column batches, whose rows share cache lines
     // that a single L2 then fetches once.
     for (Phase ph : {PH_PART, PH_TCOUNT, PH_SPREADA, PH_TILE, PH_XA, PH_XP, PH_MIDY_H, PH_MIDY_G, PH_MIDY_GR,
-                     PH_MIDZ_H, PH_PY, PH_LAST, PH_LASTR, PH_LASTR4, PH_LASTRW, PH_C2R, PH_C2RR, PH_PLANEF, PH_PLANER, PH_PLANEI, PH_PLANEIW}) {
+                     PH_MIDZ_H, PH_PY, PH_LAST, PH_LASTR, PH_LASTR4, PH_LASTRW, PH_C2R, PH_C2RR, PH_PLANEF, PH_PLANER, PH_PLANERECT, PH_YFWD, PH_PLANEI, PH_PLANEA, PH_PLANEAW}) {
         std::vector<WorkItem>& v = maps[ph].host;
         const size_t n = v.size(), q = n / kXcds, rm = n % kXcds;
         if (n < 2 * (size_t)kXcds) continue;
@@ -785,7 +779,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
     }
     for (int p = 0; p < PH_COUNT; ++p) {
         maps[p].n = (int)maps[p].host.size();
-        if (maps[p].lds > ((p == PH_PLANEF || p == PH_PLANER || p == PH_PLANEI || p == PH_PLANEIW || p == PH_LAST || p == PH_LASTR || p == PH_LASTR4 || p == PH_LASTRW) ? kPlaneLds : (size_t)kMaxLds)) { err = "pass needs more LDS than a block may use"; return -TILD_ERR_UNSUPPORTED; }
+        if (maps[p].lds > ((p == PH_PLANEF || p == PH_PLANER || p == PH_PLANERECT || p == PH_PLANEI || p == PH_PLANEA || p == PH_PLANEAW || p == PH_LAST || p == PH_LASTR || p == PH_LASTR4 || p == PH_LASTRW) ? kPlaneLds : (size_t)kMaxLds)) { err = "pass needs more LDS than a block may use"; return -TILD_ERR_UNSUPPORTED; }
         if (maps[p].dev && (!reorder_only || maps[p].cap < maps[p].n)) {
             // reused buffers are last read by the previous reorder's launches
             HIPCHK(hipStreamSynchronize(stream_));
@@ -1098,6 +1092,8 @@ int Batch::enqueue_steps(SetMaps& m, int nsteps, bool integrate, bool write_forc
         HIPCHK(launch_tile_deposit(ctx(PH_TILE), k));
         HIPCHK(launch_plane_r2c(ctx(PH_PLANEF)));
         HIPCHK(launch_plane_reg(ctx(PH_PLANER)));
+        HIPCHK(launch_plane_rect(ctx(PH_PLANERECT)));
+        HIPCHK(launch_yfwd_reg(ctx(PH_YFWD)));
         HIPCHK(launch_mid(ctx(PH_MIDY_H), 1, 0, 0, 0, nullptr));
         HIPCHK(launch_last_fused(ctx(PH_LAST), 0, k));
         HIPCHK(launch_last_reg(ctx(PH_LASTR), k, 0));
@@ -1107,8 +1103,9 @@ int Batch::enqueue_steps(SetMaps& m, int nsteps, bool integrate, bool write_forc
         HIPCHK(launch_grad_reg(ctx(PH_MIDY_GR)));
         HIPCHK(launch_x_c2r(ctx(PH_C2R), true, 0, nullptr, nullptr));
         HIPCHK(launch_c2r_reg(ctx(PH_C2RR)));
-        HIPCHK(launch_plane_inv(ctx(PH_PLANEI), false));
-        HIPCHK(launch_plane_inv(ctx(PH_PLANEIW), true));
+        HIPCHK(launch_plane_inv(ctx(PH_PLANEI)));
+        HIPCHK(launch_plane_all(ctx(PH_PLANEA), false));
+        HIPCHK(launch_plane_all(ctx(PH_PLANEAW), true));
         // integrating steps claim the next step's records; a force evaluation leaves
         // positions and records as they are
         HIPCHK(launch_particles(ctx(PH_PART), integrate, write_forces ? 1 : 0, k, integrate));
@@ -1221,7 +1218,7 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
     // phases 0-7 are kernels, timed by events bound to each launch's own start and stop
     // (a mixed set runs several kernels per phase, one per form); phase 8,
     // the spatial reorders, by an event pair around them
-    constexpr int kSlots = 4, kKernelPhases = kProfPhases - 1;
+    constexpr int kSlots = 5, kKernelPhases = kProfPhases - 1;
     hipEvent_t ev[kKernelPhases][kSlots][2], rv[2];
     for (auto& a : ev) for (auto& b : a) for (auto& e : b) HIPCHK(hipEventCreate(&e));
     for (auto& e : rv) HIPCHK(hipEventCreate(&e));
@@ -1244,6 +1241,8 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
         ok(launch_tile_deposit(ctx(PH_TILE, 1, 1), 0));
         ok(launch_plane_r2c(ctx(PH_PLANEF, 2, 0)));
         ok(launch_plane_reg(ctx(PH_PLANER, 2, 2)));
+        ok(launch_plane_rect(ctx(PH_PLANERECT, 2, 3)));
+        ok(launch_yfwd_reg(ctx(PH_YFWD, 2, 4)));
         ok(launch_mid(ctx(PH_MIDY_H, 2, 1), 1, 0, 0, 0, nullptr));
         ok(launch_last_fused(ctx(PH_LAST, 3, 0), 0, 0));
         ok(launch_last_reg(ctx(PH_LASTR, 3, 1), 0, 0));
@@ -1253,8 +1252,9 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
         ok(launch_grad_reg(ctx(PH_MIDY_GR, 4, 1)));
         ok(launch_x_c2r(ctx(PH_C2R, 5, 0), true, 0, nullptr, nullptr));
         ok(launch_c2r_reg(ctx(PH_C2RR, 5, 3)));
-        ok(launch_plane_inv(ctx(PH_PLANEI, 5, 1), false));
-        ok(launch_plane_inv(ctx(PH_PLANEIW, 5, 2), true));
+        ok(launch_plane_inv(ctx(PH_PLANEI, 5, 1)));
+        ok(launch_plane_all(ctx(PH_PLANEA, 5, 2), false));
+        ok(launch_plane_all(ctx(PH_PLANEAW, 5, 4), true));
         ok(launch_particles(ctx(PH_PART, 6, 0), true, 0, 0, true));
         ok(launch_advance(stream_, d_reps_, m->d_ids, m->nids, 1, ev[7][0][0], ev[7][0][1]));
         used[7][0] = m->nids > 0;

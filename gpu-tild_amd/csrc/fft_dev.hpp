@@ -21,7 +21,7 @@ __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(
 __device__ __forceinline__ float2 mul_mi(float2 a) { return make_float2(a.y, -a.x); }   // a * (-i)
 __device__ __forceinline__ float2 conjf2(float2 a) { return make_float2(a.x, -a.y); }
 
-// Forward DFT of small sizes (2-10, 12, 15, 16), in place on v[0..R-1].
+// Forward DFT of small sizes (2, 3, 4, 5, 7, 8, 10, 16), in place on v[0..R-1].
 template <int R> struct Dft;
 
 template <> struct Dft<2> {
@@ -158,68 +158,6 @@ template <> struct Dft<10> {
         }
     }
 };
-// N = A B with A and B coprime by the prime-factor mapping, as Dft<10>: inputs
-// n = (B n1 + A n2) mod N, A-point transforms over n1, B-point ones over n2, outputs
-// k = (EA k1 + EB k2) mod N with EA = 1 mod A, 0 mod B and EB = 0 mod A, 1 mod B.
-template <int A, int B, int EA, int EB> struct DftPfa {
-    static_assert(EA % A == 1 && EA % B == 0 && EB % A == 0 && EB % B == 1, "prime-factor output map");
-    __device__ __forceinline__ static void run(float2* v) {
-        constexpr int N = A * B;
-        float2 y[A][B];
-#pragma unroll
-        for (int n2 = 0; n2 < B; ++n2) {
-            float2 a[A];
-#pragma unroll
-            for (int n1 = 0; n1 < A; ++n1) a[n1] = v[(B * n1 + A * n2) % N];
-            Dft<A>::run(a);
-#pragma unroll
-            for (int k1 = 0; k1 < A; ++k1) y[k1][n2] = a[k1];
-        }
-#pragma unroll
-        for (int k1 = 0; k1 < A; ++k1) {
-            Dft<B>::run(y[k1]);
-#pragma unroll
-            for (int k2 = 0; k2 < B; ++k2) v[(EA * k1 + EB * k2) % N] = y[k1][k2];
-        }
-    }
-};
-template <> struct Dft<6> {
-    __device__ __forceinline__ static void run(float2* v) { DftPfa<2, 3, 3, 4>::run(v); }
-};
-template <> struct Dft<12> {
-    __device__ __forceinline__ static void run(float2* v) { DftPfa<3, 4, 4, 9>::run(v); }
-};
-template <> struct Dft<15> {
-    __device__ __forceinline__ static void run(float2* v) { DftPfa<3, 5, 10, 6>::run(v); }
-};
-// 9 = 3 x 3: three DFT-3 over the stride-3 subsequences, twiddles w9^(n2 k1), three DFT-3
-// across them; output k1 + 3 k2.
-template <> struct Dft<9> {
-    __device__ __forceinline__ static void run(float2* v) {
-        float2 y[3][3];
-#pragma unroll
-        for (int n2 = 0; n2 < 3; ++n2) {
-            float2 a[3] = {v[n2], v[n2 + 3], v[n2 + 6]};
-            Dft<3>::run(a);
-#pragma unroll
-            for (int k1 = 0; k1 < 3; ++k1) y[k1][n2] = a[k1];
-        }
-        // w9^m = (cos(2 pi m / 9), -sin(2 pi m / 9)), m = 1, 2, 4
-        const float2 w1 = make_float2(0.76604444311897803520f, -0.64278760968653932632f);
-        const float2 w2 = make_float2(0.17364817766693034885f, -0.98480775301220805937f);
-        const float2 w4 = make_float2(-0.93969262078590838405f, -0.34202014332566873304f);
-        y[1][1] = cmul(y[1][1], w1);
-        y[1][2] = cmul(y[1][2], w2);
-        y[2][1] = cmul(y[2][1], w2);
-        y[2][2] = cmul(y[2][2], w4);
-#pragma unroll
-        for (int k1 = 0; k1 < 3; ++k1) {
-            Dft<3>::run(y[k1]);
-#pragma unroll
-            for (int k2 = 0; k2 < 3; ++k2) v[k1 + 3 * k2] = y[k1][k2];
-        }
-    }
-};
 template <> struct Dft<7> {
     __device__ __forceinline__ static void run(float2* v) {
         const float c[4] = {1.f, 0.62348980185873353053f, -0.22252093395631440429f, -0.90096886790241912624f};
@@ -322,12 +260,8 @@ __device__ __forceinline__ float2* lds_fft(float2* A, float2* B, int ldb, int nb
             case 3: fft_stage<3, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
             case 4: fft_stage<4, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
             case 5: fft_stage<5, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
-            case 6: fft_stage<6, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
             case 7: fft_stage<7, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
-            case 9: fft_stage<9, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
             case 10: fft_stage<10, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
-            case 12: fft_stage<12, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
-            case 15: fft_stage<15, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
             case 16: fft_stage<16, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
             default: fft_stage<8, NT>(src, dst, ldb, nb, pl.N, p, tw); break;
         }

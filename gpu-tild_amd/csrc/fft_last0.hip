@@ -1,4 +1,4 @@
-// fft_last0.hip -- k_last_reg for short axes, one or two types.
+// fft_last0.hip -- k_last_reg for axes up to 100 points, one or two types.
 #include "fft_last.hpp"
 
 namespace tild {

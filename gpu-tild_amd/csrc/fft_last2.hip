@@ -1,4 +1,4 @@
-// fft_last2.hip -- k_last_reg for longer axes (R1 >= 12), one or two types.
+// fft_last2.hip -- k_last_reg for longer axes, one or two types.
 #include "fft_last.hpp"
 
 namespace tild {

@@ -14,17 +14,18 @@
 
 namespace tild {
 
-namespace {
-
-bool reg_plan_pair(int k) {   // k = R1 * 32 + R2
-    switch (k) {
-#define TILD_CASE(A, B) case A * 32 + B: return true;
+RegDims reg_dims(const AxisPlan& pl) {
+    if (pl.nst < 2 || pl.nst > 4) return RegDims{0, 0, 0, 0};
+    int key = pl.rad[0];
+    for (int s = 1; s < pl.nst; ++s) key = key * 32 + pl.rad[s];
+    switch (key) {
+#define TILD_CASE(A0, A1, B0, B1) \
+    case reg_plan_key(A0, A1, B0, B1): return RegDims{key, (A0) * (A1), (B0) * (B1), A1 > 1 ? 2 : 1};
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
-        default: return false;
+        default: return RegDims{0, 0, 0, 0};
     }
 }
-}  // namespace
 
 // ------------------------------------------------------------------ y inverse (3D)
 // The y-axis inverse of the gradient spectra (the operation of k_mid_grad, kernels.hip)
@@ -37,21 +38,19 @@ bool reg_plan_pair(int k) {   // k = R1 * 32 + R2
 // One barrier.  A block reads its columns of slots 0 and 2 before it writes any slot,
 // and no other block touches them.
 namespace {
-template <int R1, int R2, int NT>
+template <class P, int NT>
 __device__ __forceinline__ void grad_reg_block(const RepDev& r, int blk, float2* lds) {
-    constexpr int N = R1 * R2, NB = NT / R1, ld = 3 * NB + 1, NT1 = R1 * (R2 - 1);
+    constexpr int R1 = P::R1, R2 = P::R2, N = P::N, NB = NT / P::RM, ld = 3 * NB + 1;
     const int Nxh = r.Nxh;
     const int nchunk = (Nxh + NB - 1) / NB;
     const int o = blk / nchunk, c = blk - o * nchunk;   // o = f Nz + z
     const int f = o / r.Nz, z = o - f * r.Nz;
     const int b0 = c * NB, nb = min(NB, Nxh - b0);
     float2* X1 = lds;                 // N x ld
-    float2* TW1 = X1 + N * ld;        // w_Ny^{i r}, i < R1, 1 <= r < R2
+    float2* TW1 = X1 + N * ld;        // the second group's twiddles
     const int b = (int)threadIdx.x % NB, i = (int)threadIdx.x / NB;
-    {
-        const float2* tw1 = r.reg_tw[1];
-        for (int t = threadIdx.x; t < NT1; t += NT) TW1[t] = gld(tw1 + t);
-    }
+    const float2* const tw = r.reg_tw[1];
+    for (int t = threadIdx.x; t < P::NTW; t += NT) TW1[t] = gld(tw + t);
     // element (n, column b) of slot s: 32-bit offsets from the uniform base
     const uint32_t Mhu = (uint32_t)r.Mh, Nxu = (uint32_t)Nxh;
     const uint32_t plane = (uint32_t)z * (uint32_t)N * Nxu + (uint32_t)(b0 + b);
@@ -77,7 +76,7 @@ __device__ __forceinline__ void grad_reg_block(const RepDev& r, int blk, float2*
         }
 #pragma unroll
         for (int l = 0; l < 3; ++l) {
-            Dft<R1>::run(L[l]);
+            plan_first<P>(L[l], tw);
 #pragma unroll
             for (int q = 0; q < R1; ++q) X1[(i * R1 + q) * ld + l * NB + b] = L[l][q];
         }
@@ -86,20 +85,56 @@ __device__ __forceinline__ void grad_reg_block(const RepDev& r, int blk, float2*
     if (i < R1 && b < nb) {
         float2 t[R2];
 #pragma unroll
-        for (int rr = 1; rr < R2; ++rr) t[rr] = TW1[i * (R2 - 1) + rr - 1];
+        for (int m = 1; m < R2; ++m) t[m] = TW1[tw2_index<P>(i, m)];
 #pragma unroll
         for (int l = 0; l < 3; ++l) {
             float2 w[R2];
 #pragma unroll
             for (int rr = 0; rr < R2; ++rr) w[rr] = X1[(i + R1 * rr) * ld + l * NB + b];
-#pragma unroll
-            for (int rr = 1; rr < R2; ++rr) w[rr] = cmul(w[rr], t[rr]);
-            Dft<R2>::run(w);
+            plan_second<P, !P::KEPT>(w, [&](int m) { return t[m]; });
             const uint32_t s0 = l == 0 ? sU : (l == 1 ? sY : sV);
 #pragma unroll
             for (int q = 0; q < R2; ++q)
                 gst(at32(r.Gk, s0 + (uint32_t)(i + R1 * q) * Nxu), conjf2(w[q]));
         }
+    }
+}
+
+// Forward y FFT of the half spectra of one (field, z) plane's columns in place (the
+// operation of k_mid, kernels.hip), where no plane pass runs it (odd sides); the same
+// blocks, one line per column.
+template <class P, int NT>
+__device__ __forceinline__ void yfwd_reg_block(const RepDev& r, int blk, float2* lds) {
+    constexpr int R1 = P::R1, R2 = P::R2, N = P::N, NB = NT / P::RM, ld = NB + 1;
+    const int Nxh = r.Nxh;
+    const int nchunk = (Nxh + NB - 1) / NB;
+    const int o = blk / nchunk, c = blk - o * nchunk;   // o = f Nz + z
+    const int b0 = c * NB, nb = min(NB, Nxh - b0);
+    float2* X1 = lds;                 // N x ld
+    float2* TW1 = X1 + N * ld;
+    const int b = (int)threadIdx.x % NB, i = (int)threadIdx.x / NB;
+    const float2* const tw = r.reg_tw[1];
+    const uint32_t Nxu = (uint32_t)Nxh, s0 = (uint32_t)o * (uint32_t)N * Nxu + (uint32_t)(b0 + b);
+    float2 v[R1];
+    const bool live = i < R2 && b < nb;
+    if (live) {
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) v[rr] = gld(at32((const float2*)r.H, s0 + (uint32_t)(i + R2 * rr) * Nxu));
+    }
+    for (int t = threadIdx.x; t < P::NTW; t += NT) TW1[t] = gld(tw + t);
+    if (live) {
+        plan_first<P>(v, tw);
+#pragma unroll
+        for (int q = 0; q < R1; ++q) X1[(i * R1 + q) * ld + b] = v[q];
+    }
+    __syncthreads();
+    if (i < R1 && b < nb) {
+        float2 w[R2];
+#pragma unroll
+        for (int rr = 0; rr < R2; ++rr) w[rr] = X1[(i + R1 * rr) * ld + b];
+        plan_second_lds<P, true>(w, TW1, i);
+#pragma unroll
+        for (int q = 0; q < R2; ++q) gst(at32(r.H, s0 + (uint32_t)(i + R1 * q) * Nxu), w[q]);
     }
 }
 }  // namespace
@@ -111,7 +146,27 @@ __global__ void __launch_bounds__(NT) k_grad_reg(const RepDev* __restrict__ reps
     const RepDev& r = reps[wi.rep];
     warm_desc<0, 1, 6, 7>(r);
     switch (r.reg_key[1]) {   // uniform per block
-#define TILD_CASE(A, B) case A * 32 + B: grad_reg_block<A, B, NT>(r, wi.blk, lds); break;
+#define TILD_CASE(A0, A1, B0, B1)          \
+    case reg_plan_key(A0, A1, B0, B1):     \
+        if constexpr ((A0) * (A1) <= 16) grad_reg_block<RegPlan<A0, A1, B0, B1>, NT>(r, wi.blk, lds); \
+        break;
+        TILD_REG_PLANS(TILD_CASE)
+#undef TILD_CASE
+        default: break;   // excluded by grad_reg_plan on the host
+    }
+}
+
+template <int NT>
+__global__ void __launch_bounds__(NT) k_yfwd_reg(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
+    extern __shared__ float2 lds[];
+    const WorkItem wi = wmap[blockIdx.x];
+    const RepDev& r = reps[wi.rep];
+    warm_desc<0, 1, 6, 7>(r);
+    switch (r.reg_key[1]) {   // uniform per block
+#define TILD_CASE(A0, A1, B0, B1)          \
+    case reg_plan_key(A0, A1, B0, B1):     \
+        if constexpr ((A0) * (A1) <= 16) yfwd_reg_block<RegPlan<A0, A1, B0, B1>, NT>(r, wi.blk, lds); \
+        break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
         default: break;   // excluded by grad_reg_plan on the host
@@ -120,9 +175,8 @@ __global__ void __launch_bounds__(NT) k_grad_reg(const RepDev* __restrict__ reps
 
 // ------------------------------------------------------------------ plane forward (3D)
 // x R2C and y FFT of one (field, z) density plane (the operation of k_plane_r2c,
-// kernels.hip) for square planes Nx = Ny with a two-stage plan R1 x R2:
-//   A  task (pair j, i < R2): rows 2j and 2j+1 at x = i + R2 r as one complex line (an odd
-//      side's last row with zeros), DFT_R1;
+// kernels.hip) for even square planes Nx = Ny with a kept two-stage plan R1 x R2:
+//   A  task (pair j, i < R2): rows 2j and 2j+1 at x = i + R2 r as one complex line, DFT_R1;
 //   B  task (j, i < R1): twiddles, DFT_R2 -> Z_j(k), k = i + R1 q; exchange;
 //   C  task (column k < Nxh, i < R2): the half spectra of rows y = i + R2 r unpacked on
 //      the fly from Z_{y/2}(k) and Z_{y/2}(N - k), DFT_R1;
@@ -130,14 +184,9 @@ __global__ void __launch_bounds__(NT) k_grad_reg(const RepDev* __restrict__ reps
 // Three barriers, where the staged pass has seven; loads and stores go straight to and
 // from registers.
 namespace {
-__device__ __forceinline__ float half_of(float a) {
-#pragma clang fp contract(off)
-    return 0.5f * a;
-}
-
 template <int R1, int R2, int NT>
 __device__ __forceinline__ void plane_reg_block(const RepDev& r, int blk, float2* lds) {
-    constexpr int N = R1 * R2, NP = (N + 1) / 2, NXH = N / 2 + 1, ldp = NP | 1, ldc = NXH | 1;
+    constexpr int N = R1 * R2, NP = N / 2, NXH = N / 2 + 1, ldp = NP | 1, ldc = NXH | 1;
     constexpr int NT1 = R1 * (R2 - 1), LDA = (N * ldp > N * ldc) ? N * ldp : N * ldc;
     const int z = blk % r.Nz, f = blk / r.Nz;
     float2* Xa = lds;                  // x stage-1 output, later the y stage-1 output (N x ldc)
@@ -157,9 +206,7 @@ __device__ __forceinline__ void plane_reg_block(const RepDev& r, int blk, float2
 #pragma unroll
         for (int rr = 0; rr < R1; ++rr) {
             const uint32_t o = pbase + (uint32_t)(2 * j * N + i + R2 * rr);
-            const float a = G(at32((const float*)r.rho, o))[0];
-            const float c = N % 2 == 0 || 2 * j + 1 < N ? G(at32((const float*)r.rho, o + N))[0] : 0.f;
-            v[rr] = make_float2(a, c);
+            v[rr] = make_float2(G(at32((const float*)r.rho, o))[0], G(at32((const float*)r.rho, o + N))[0]);
         }
         Dft<R1>::run(v);
 #pragma unroll
@@ -221,10 +268,124 @@ __global__ void __launch_bounds__(NT) k_plane_reg(const RepDev* __restrict__ rep
     const RepDev& r = reps[wi.rep];
     warm_desc<0, 1, 6, 7>(r);
     switch (r.reg_key[0]) {   // uniform per block
-#define TILD_CASE(A, B) case A * 32 + B: plane_reg_block<A, B, NT>(r, wi.blk, lds); break;
+#define TILD_CASE(A0, A1, B0, B1)          \
+    case reg_plan_key(A0, A1, B0, B1):     \
+        if constexpr (reg_plan_kept(A0 * A1 * B0 * B1) && A0 * B0 % 2 == 0 && A0 * B0 <= 128) plane_reg_block<A0, B0, NT>(r, wi.blk, lds); \
+        break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
         default: break;   // excluded by plane_reg_plan on the host
+    }
+}
+
+// The same for any even plane of compiled plans (sides of equal or unequal plans): the x
+// phases compiled per x plan, the y phases per y plan, bit for bit the LDS-staged pass.
+namespace {
+template <class P, int NT>
+__device__ __forceinline__ void plane_rect_x(const RepDev& r, uint32_t pbase, float2* Xa, float2* Xb, const float2* TW) {
+    constexpr int R1 = P::R1, R2 = P::R2, N = P::N;
+    const int np = r.Ny / 2, ldp = np | 1;
+    const float2* const tw = r.reg_tw[0];
+    // A: pairs of rows as complex lines, first group of the x plan
+    for (int task = threadIdx.x; task < np * R2; task += NT) {
+        const int i = task % R2, j = task / R2;
+        float2 v[R1];
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) {
+            const uint32_t o = pbase + (uint32_t)(2 * j * N + i + R2 * rr);
+            v[rr] = make_float2(G(at32((const float*)r.rho, o))[0], G(at32((const float*)r.rho, o + N))[0]);
+        }
+        plan_first<P>(v, tw);
+#pragma unroll
+        for (int q = 0; q < R1; ++q) Xa[(i * R1 + q) * ldp + j] = v[q];
+    }
+    __syncthreads();
+    // B: second group -> Z_j(k)
+    const FastDiv dnp(np);
+    for (int task = threadIdx.x; task < np * R1; task += NT) {
+        int j;
+        const int i = dnp.div(task, j);
+        float2 v[R2];
+#pragma unroll
+        for (int rr = 0; rr < R2; ++rr) v[rr] = Xa[(i + R1 * rr) * ldp + j];
+        plan_second_lds<P, true>(v, TW, i);
+#pragma unroll
+        for (int q = 0; q < R2; ++q) Xb[(i + R1 * q) * ldp + j] = v[q];
+    }
+    __syncthreads();
+}
+
+template <class P, int NT>
+__device__ __forceinline__ void plane_rect_y(const RepDev& r, uint32_t hbase, float2* Xa, const float2* Xb, const float2* TW) {
+    constexpr int R1 = P::R1, R2 = P::R2, N = P::N;
+    const int Nx = r.Nx, nxh = r.Nxh, ldp = (N / 2) | 1, ldc = nxh | 1;
+    const float2* const tw = r.reg_tw[1];
+    const FastDiv dnx(nxh);
+    // C: unpack rows y = i + R2 r of column k, first group of the y plan
+    for (int task = threadIdx.x; task < nxh * R2; task += NT) {
+        int k;
+        const int i = dnx.div(task, k);
+        const int km = k == 0 ? 0 : Nx - k;
+        float2 v[R1];
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) {
+            const int y = i + R2 * rr, j = y >> 1;
+            const float2 Zk = Xb[k * ldp + j], Zm = Xb[km * ldp + j];
+            v[rr] = (y & 1) == 0 ? make_float2(half_of(Zk.x + Zm.x), half_of(Zk.y - Zm.y))
+                                 : make_float2(half_of(Zk.y + Zm.y), half_of(Zm.x - Zk.x));
+        }
+        plan_first<P>(v, tw);
+#pragma unroll
+        for (int q = 0; q < R1; ++q) Xa[(i * R1 + q) * ldc + k] = v[q];
+    }
+    __syncthreads();
+    // D: second group -> H(y, k)
+    for (int task = threadIdx.x; task < nxh * R1; task += NT) {
+        int k;
+        const int i = dnx.div(task, k);
+        float2 v[R2];
+#pragma unroll
+        for (int rr = 0; rr < R2; ++rr) v[rr] = Xa[(i + R1 * rr) * ldc + k];
+        plan_second_lds<P, true>(v, TW, i);
+#pragma unroll
+        for (int q = 0; q < R2; ++q) gst(at32(r.H, hbase + (uint32_t)((i + R1 * q) * nxh + k)), v[q]);
+    }
+}
+}  // namespace
+
+template <int NT>
+__global__ void __launch_bounds__(NT) k_plane_rect(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
+    extern __shared__ float2 lds[];
+    const WorkItem wi = wmap[blockIdx.x];
+    const RepDev& r = reps[wi.rep];
+    warm_desc<0, 1, 6, 7>(r);
+    const int Nx = r.Nx, Ny = r.Ny, nxh = r.Nxh, ldp = (Ny / 2) | 1, ldc = nxh | 1;
+    const int z = wi.blk % r.Nz, f = wi.blk / r.Nz;
+    float2* Xa = lds;                                   // x first-group output, later the y one
+    float2* Xb = Xa + max(Nx * ldp, Ny * ldc);          // Z: x transforms of the row pairs
+    float2* TWx = Xb + Nx * ldp;
+    float2* TWy = TWx + Nx;
+    // second groups' twiddles: fewer than N of each (N - R1), visible after the first barrier
+    {
+        const int nx = reg_ntw(r.reg_key[0], Nx), ny = reg_ntw(r.reg_key[1], Ny);
+        for (int t = threadIdx.x; t < nx; t += NT) TWx[t] = gld(r.reg_tw[0] + t);
+        for (int t = threadIdx.x; t < ny; t += NT) TWy[t] = gld(r.reg_tw[1] + t);
+    }
+    const uint32_t pbase = (uint32_t)f * (uint32_t)r.M + (uint32_t)z * (uint32_t)(Nx * Ny);
+    const uint32_t hbase = ((uint32_t)f * (uint32_t)r.Nz + (uint32_t)z) * (uint32_t)(Ny * nxh);
+    switch (r.reg_key[0]) {   // uniform per block
+#define TILD_CASE(A0, A1, B0, B1) \
+    case reg_plan_key(A0, A1, B0, B1): plane_rect_x<RegPlan<A0, A1, B0, B1>, NT>(r, pbase, Xa, Xb, TWx); break;
+        TILD_REG_PLANS(TILD_CASE)
+#undef TILD_CASE
+        default: break;   // compiled plans only
+    }
+    switch (r.reg_key[1]) {
+#define TILD_CASE(A0, A1, B0, B1) \
+    case reg_plan_key(A0, A1, B0, B1): plane_rect_y<RegPlan<A0, A1, B0, B1>, NT>(r, hbase, Xa, Xb, TWy); break;
+        TILD_REG_PLANS(TILD_CASE)
+#undef TILD_CASE
+        default: break;
     }
 }
 
@@ -412,11 +573,183 @@ __global__ void __launch_bounds__(NT) k_plane_inv(const RepDev* __restrict__ rep
     const RepDev& r = reps[wi.rep];
     warm_desc<0, 1, 3, 6, 7>(r);
     switch (r.reg_key[1]) {   // uniform per block
-#define TILD_CASE(A, B) \
-    case A * 32 + B: if constexpr (plane_inv_threads(A, B) == NT) plane_inv_block<A, B, NT>(r, wi.blk, lds); break;
+#define TILD_CASE(A0, A1, B0, B1)          \
+    case reg_plan_key(A0, A1, B0, B1):     \
+        if constexpr (reg_plan_kept(A0 * A1 * B0 * B1) && (A0 * B0 / 2 + 1) * (A0 > B0 ? A0 : B0) <= NT) \
+            plane_inv_block<A0, B0, NT>(r, wi.blk, lds);                                                 \
+        break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
         default: break;   // excluded by plane_inv_plan on the host
+    }
+}
+
+// The inverse plane pass for the other square plans: all NF fields of one z plane in one
+// block, the x lines paired as the separate x pass pairs them (real lines f 3 + d of a
+// row, two to a complex line), so that the records are bit for bit those of the y inverse
+// and the x pass.  The phases of plane_inv_block; an odd count of lines pairs the last
+// with zeros.
+namespace {
+template <class P, int NT, int NF>
+__device__ __forceinline__ void plane_all_block(const RepDev& r, int z, float2* lds) {
+    constexpr int R1 = P::R1, R2 = P::R2, N = P::N, NXH = N / 2 + 1;
+    constexpr int LA = (3 * NXH) | 1;             // row stride of a field's y inverses: [f][y][line][k]
+    constexpr int NL = 3 * NF, NC = (NL + 1) / 2; // real and complex x lines per row
+    constexpr int NCL = N * NC, LC = NCL | 1;     // x lines, row stride of the x exchange
+    constexpr int CT = (NCL * R2 + NT - 1) / NT, DT = (NCL * R1 + NT - 1) / NT;
+    constexpr int NE = plane_all_elems(N, NF);
+    static_assert(NF * N * LA <= NE && N * LC <= NE && 3 * NF * N * N <= 2 * NE, "plane_all_block: buffer");
+    float2* X = lds;                              // NF x N x LA, then the x exchange (N x LC), then the records
+    float2* TW = X + NE;                          // the second group's twiddles (one plan on x and y)
+    const float2* const twx = r.reg_tw[0];
+    const float2* const twy = r.reg_tw[1];
+    for (int t = threadIdx.x; t < P::NTW; t += NT) TW[t] = gld(twy + t);
+    const uint32_t Mhu = (uint32_t)r.Mh;
+    const uint32_t plane = (uint32_t)z * (uint32_t)(N * NXH);
+    const float kfy = r.kfac[1], kfx = r.kfac[0];
+    // A: y first group of the three lines of column k
+    for (int task = threadIdx.x; task < NF * NXH * R2; task += NT) {
+        const int k = task % NXH, rest = task / NXH, i = rest % R2, f = rest / R2;
+        const uint32_t sU = (uint32_t)(f * 3) * Mhu + plane, sV = sU + 2u * Mhu;
+        float2 u[R1], v[R1];
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) {
+            const uint32_t o = (uint32_t)((i + R2 * rr) * NXH + k);
+            u[rr] = gld(at32((const float2*)r.Gk, sU + o));
+            v[rr] = gld(at32((const float2*)r.Gk, sV + o));
+        }
+        float2* Xf = X + f * (N * LA) + k;
+        float2 L[R1];
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+#pragma unroll
+            for (int rr = 0; rr < R1; ++rr) {
+                const int n = i + R2 * rr;
+                const float ky = 2 * n == N ? 0.f : kfy * (float)(2 * n < N ? n : n - N);
+                // lines of the conj(FFT(conj)) inverse: conj(u), conj(-i ky u), conj(v)
+                L[rr] = l == 0 ? make_float2(u[rr].x, -u[rr].y)
+                               : (l == 1 ? grad_line(ky, u[rr]) : make_float2(v[rr].x, -v[rr].y));
+            }
+            plan_first<P>(L, twy);
+#pragma unroll
+            for (int q = 0; q < R1; ++q) Xf[(i * R1 + q) * LA + l * NXH] = L[q];
+        }
+    }
+    __syncthreads();
+    // B: y second group; Y_l(y, k) = conj of the result, over the rows the task read
+    for (int task = threadIdx.x; task < NF * NXH * R1; task += NT) {
+        const int k = task % NXH, rest = task / NXH, i = rest % R1, f = rest / R1;
+        float2* Xf = X + f * (N * LA) + k;
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+            float2 w[R2];
+#pragma unroll
+            for (int rr = 0; rr < R2; ++rr) w[rr] = Xf[(i + R1 * rr) * LA + l * NXH];
+            plan_second_lds<P, true>(w, TW, i);
+#pragma unroll
+            for (int q = 0; q < R2; ++q) Xf[(i + R1 * q) * LA + l * NXH] = conjf2(w[q]);
+        }
+    }
+    __syncthreads();
+    // C: x first group of complex line (row y, j): real lines 2j and 2j + 1 = f 3 + d
+    float2 hold[CT][R1];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        const int task = (int)threadIdx.x + ct * NT;
+        if (task >= NCL * R2) break;
+        const int c = task % NCL, i = task / NCL, y = c / NC, j = c - y * NC;
+        const int la = 2 * j, lb = la + 1, fa = la / 3, da = la - 3 * fa, fb = lb / 3, db = lb - 3 * fb;
+        const float2* pa = X + fa * (N * LA) + y * LA + da * NXH;
+        const float2* pb = X + (lb < NL ? fb * (N * LA) + y * LA + db * NXH : 0);
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) {
+            const int kn = i + R2 * rr;                 // full-spectrum index
+            const bool upper = kn >= NXH;
+            const int kk = upper ? N - kn : kn;         // its half-spectrum column
+            float2 A = pa[kk], B = lb < NL ? pb[kk] : make_float2(0.f, 0.f);
+            const bool self = kk == 0 || 2 * kk == N;
+            const float kx = self && kk != 0 ? 0.f : kfx * (float)kk;
+            if (da == 0) A = x_gradient(kx, A);
+            if (db == 0) B = x_gradient(kx, B);
+            if (self) { A.y = 0.f; B.y = 0.f; }
+            hold[ct][rr] = upper ? make_float2(A.x + B.y, A.y - B.x) : make_float2(A.x - B.y, -(A.y + B.x));
+        }
+        plan_first<P>(hold[ct], twx);
+        settle<R1>(hold[ct]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        const int task = (int)threadIdx.x + ct * NT;
+        if (task >= NCL * R2) break;
+        const int c = task % NCL, i = task / NCL;
+#pragma unroll
+        for (int q = 0; q < R1; ++q) X[(i * R1 + q) * LC + c] = hold[ct][q];
+    }
+    __syncthreads();
+    // D: x second group -> the real lines at x = i + R1 q, held across a barrier and laid out
+    // as the fields' records [f][y][x](g_x, g_y, g_z)
+    float2 out[DT][R2];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        const int task = (int)threadIdx.x + dt * NT;
+        if (task >= NCL * R1) break;
+        const int i = task % R1, c = task / R1;   // adjacent lanes: adjacent x
+#pragma unroll
+        for (int rr = 0; rr < R2; ++rr) out[dt][rr] = X[(i + R1 * rr) * LC + c];
+        plan_second_lds<P, true>(out[dt], TW, i);
+        settle<R2>(out[dt]);
+    }
+    __syncthreads();
+    float* rec = (float*)X;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        const int task = (int)threadIdx.x + dt * NT;
+        if (task >= NCL * R1) break;
+        const int i = task % R1, c = task / R1, y = c / NC, j = c - y * NC;
+        const int la = 2 * j, lb = la + 1, fa = la / 3, da = la - 3 * fa, fb = lb / 3, db = lb - 3 * fb;
+#pragma unroll
+        for (int q = 0; q < R2; ++q) {
+            const int x = i + R1 * q;
+            rec[((fa * N + y) * N + x) * 3 + da] = out[dt][q].x;
+            if (lb < NL) rec[((fb * N + y) * N + x) * 3 + db] = -out[dt][q].y;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        const uint32_t rec0 = (uint32_t)f * (uint32_t)r.M + (uint32_t)z * (uint32_t)(N * N);
+        const float* src = rec + f * 3 * N * N;
+        if constexpr (N % 2 == 0) {   // 12 rec0 bytes, 16-byte aligned
+            float4* dst = (float4*)((char*)r.G3 + ((rec0 << 3) + (rec0 << 2)));
+            for (int t = threadIdx.x; t < 3 * N * N / 4; t += NT) gst(dst + t, ((const float4*)src)[t]);
+        } else {
+            float* dst = (float*)((char*)r.G3 + ((rec0 << 3) + (rec0 << 2)));
+            for (int t = threadIdx.x; t < 3 * N * N; t += NT) G(dst)[t] = src[t];
+        }
+    }
+}
+}  // namespace
+
+template <int NT>
+__global__ void __launch_bounds__(NT) k_plane_all(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
+    extern __shared__ float2 lds[];
+    const WorkItem wi = wmap[blockIdx.x];
+    const RepDev& r = reps[wi.rep];
+    warm_desc<0, 1, 3, 6, 7>(r);
+    switch (r.reg_key[1] * 2 + (r.nf == 2 ? 1 : 0)) {   // uniform per block
+#define TILD_CASE(A0, A1, B0, B1)                                                                          \
+    case reg_plan_key(A0, A1, B0, B1) * 2:                                                                 \
+        if constexpr (!reg_plan_kept(A0 * A1 * B0 * B1) && A0 * A1 <= 16 && plane_all_threads(A0 * A1 * B0 * B1, 1) == NT) \
+            plane_all_block<RegPlan<A0, A1, B0, B1>, NT, 1>(r, wi.blk, lds);                               \
+        break;                                                                                             \
+    case reg_plan_key(A0, A1, B0, B1) * 2 + 1:                                                             \
+        if constexpr (!reg_plan_kept(A0 * A1 * B0 * B1) && A0 * A1 <= 16 && plane_all_threads(A0 * A1 * B0 * B1, 2) == NT) \
+            plane_all_block<RegPlan<A0, A1, B0, B1>, NT, 2>(r, wi.blk, lds);                               \
+        break;
+        TILD_REG_PLANS(TILD_CASE)
+#undef TILD_CASE
+        default: break;   // excluded by plane_all_plan on the host
     }
 }
 
@@ -432,14 +765,9 @@ __global__ void __launch_bounds__(NT) k_plane_inv(const RepDev* __restrict__ rep
 // reads each half-spectrum value twice (the second time from cache), which is why grids of
 // many planes take the plane pass instead.
 namespace {
-__device__ __forceinline__ float2 x_gradient(float kx, float2 a) {   // -i k_x a
-#pragma clang fp contract(off)
-    return make_float2(kx * a.y, -kx * a.x);
-}
-
-template <int R1, int R2, int NT>
+template <class P, int NT>
 __device__ __forceinline__ void c2r_reg_block(const RepDev& r, int blk, float2* lds) {
-    constexpr int N = R1 * R2, NXH = N / 2 + 1, NT1 = R1 * (R2 - 1);
+    constexpr int R1 = P::R1, R2 = P::R2, N = P::N, NXH = N / 2 + 1, NT1 = P::NTW;
     static_assert(NT1 <= NT, "c2r_reg_block: one twiddle per thread");
     const int D = r.dim, NL = r.nf * D, nc = (NL + 1) / 2;
     const int nrows = r.M / N;                 // rows of one field
@@ -488,7 +816,7 @@ __device__ __forceinline__ void c2r_reg_block(const RepDev& r, int blk, float2* 
             const float re = fuse ? __builtin_fmaf(kx, A[rr].y, -c.y) : a.x - c.y;
             v[rr] = upper ? make_float2(a.x + c.y, a.y - c.x) : make_float2(re, -(a.y + c.x));
         }
-        Dft<R1>::run(v);
+        plan_first<P>(v, r.reg_tw[0]);
 #pragma unroll
         for (int q = 0; q < R1; ++q) X[(i * R1 + q) * ldb + b] = v[q];
     }
@@ -501,9 +829,7 @@ __device__ __forceinline__ void c2r_reg_block(const RepDev& r, int blk, float2* 
         float2 w[R2];
 #pragma unroll
         for (int rr = 0; rr < R2; ++rr) w[rr] = X[(i + R1 * rr) * ldb + b];
-#pragma unroll
-        for (int rr = 1; rr < R2; ++rr) w[rr] = cmul(w[rr], lds_twiddle(TW + i * (R2 - 1) + rr - 1));
-        Dft<R2>::run(w);
+        plan_second_lds<P, true>(w, TW, i);
 #pragma unroll
         for (int q = 0; q < R2; ++q) X[(i + R1 * q) * ldb + b] = w[q];
     }
@@ -535,7 +861,8 @@ __global__ void __launch_bounds__(NT) k_c2r_reg(const RepDev* __restrict__ reps,
     const RepDev& r = reps[wi.rep];
     warm_desc<0, 1, 3, 6, 7, 8>(r);
     switch (r.reg_key[0]) {   // uniform per block
-#define TILD_CASE(A, B) case A * 32 + B: c2r_reg_block<A, B, NT>(r, wi.blk, lds); break;
+#define TILD_CASE(A0, A1, B0, B1) \
+    case reg_plan_key(A0, A1, B0, B1): c2r_reg_block<RegPlan<A0, A1, B0, B1>, NT>(r, wi.blk, lds); break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
         default: break;   // reg_key holds compiled plans only
@@ -549,27 +876,44 @@ hipError_t launch_c2r_reg(const LaunchCtx& c) {
 }
 
 bool plane_inv_plan(const AxisPlan& px, const AxisPlan& py) {
-    if (!(px.N == py.N && grad_reg_plan(py))) return false;
-    return plane_inv_threads(py.rad[0], py.rad[1]) > 0;
+    if (!(px.N == py.N && reg_dims(py).key && reg_plan_kept(py.N))) return false;
+    const int rmax = py.rad[0] > py.rad[1] ? py.rad[0] : py.rad[1];
+    return (py.N / 2 + 1) * rmax <= kPlaneInvThreads && plane_inv_lds_bytes(py) <= kPlaneLds / 2;
 }
 
-hipError_t launch_plane_inv(const LaunchCtx& c, bool wide) {
+bool plane_all_plan(const AxisPlan& px, const AxisPlan& py, int nf) {
+    const RegDims d = reg_dims(py);
+    return px.N == py.N && d.key && d.R1 <= 16 && !reg_plan_kept(py.N) && nf <= 2 && plane_all_threads(py.N, nf) > 0;
+}
+
+hipError_t launch_plane_inv(const LaunchCtx& c) {
     if (!c.n) return hipSuccess;
-    if (wide) TILD_LAUNCH(c, k_plane_inv<kPlaneInvWide>, dim3(c.n), dim3(kPlaneInvWide), c.lds, c.reps, c.wmap);
-    else TILD_LAUNCH(c, k_plane_inv<kPlaneInvThreads>, dim3(c.n), dim3(kPlaneInvThreads), c.lds, c.reps, c.wmap);
+    TILD_LAUNCH(c, k_plane_inv<kPlaneInvThreads>, dim3(c.n), dim3(kPlaneInvThreads), c.lds, c.reps, c.wmap);
     return hipGetLastError();
 }
 
-hipError_t configure_plane_inv() {
-    hipError_t e = hipFuncSetAttribute((const void*)k_plane_inv<kPlaneInvThreads>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kPlaneLds / 2));
-    if (e != hipSuccess) return e;
-    return hipFuncSetAttribute((const void*)k_plane_inv<kPlaneInvWide>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)kPlaneLds);
+hipError_t launch_plane_all(const LaunchCtx& c, bool wide) {
+    if (!c.n) return hipSuccess;
+    if (wide) TILD_LAUNCH(c, k_plane_all<kPlaneInvWide>, dim3(c.n), dim3(kPlaneInvWide), c.lds, c.reps, c.wmap);
+    else TILD_LAUNCH(c, k_plane_all<kPlaneInvThreads>, dim3(c.n), dim3(kPlaneInvThreads), c.lds, c.reps, c.wmap);
+    return hipGetLastError();
 }
 
+static hipError_t allow_lds(const void* kernel, size_t bytes) {
+    return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
+hipError_t configure_plane_inv() {
+    for (hipError_t e : {allow_lds((const void*)k_plane_inv<kPlaneInvThreads>, kPlaneLds / 2),
+                         allow_lds((const void*)k_plane_all<kPlaneInvThreads>, kPlaneLds / 2),
+                         allow_lds((const void*)k_plane_all<kPlaneInvWide>, kPlaneLds)})
+        if (e != hipSuccess) return e;
+    return hipSuccess;
+}
+
+// the kept square plans
 bool plane_reg_plan(const AxisPlan& px, const AxisPlan& py) {
-    return px.N == py.N && grad_reg_plan(px);
+    return px.N == py.N && reg_dims(px).key && reg_plan_kept(px.N);
 }
 
 hipError_t launch_plane_reg(const LaunchCtx& c) {
@@ -578,15 +922,20 @@ hipError_t launch_plane_reg(const LaunchCtx& c) {
     return hipGetLastError();
 }
 
+hipError_t launch_plane_rect(const LaunchCtx& c) {
+    if (!c.n) return hipSuccess;
+    TILD_LAUNCH(c, k_plane_rect<kPlaneRegThreads>, dim3(c.n), dim3(kPlaneRegThreads), c.lds, c.reps, c.wmap);
+    return hipGetLastError();
+}
+
 hipError_t configure_plane_reg() {
-    return hipFuncSetAttribute((const void*)k_plane_reg<kPlaneRegThreads>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)kPlaneLds);
+    const hipError_t e = allow_lds((const void*)k_plane_reg<kPlaneRegThreads>, kPlaneLds);
+    return e != hipSuccess ? e : allow_lds((const void*)k_plane_rect<kPlaneRegThreads>, kPlaneLds);
 }
 
 bool grad_reg_plan(const AxisPlan& pl) {
-    if (pl.nst != 2) return false;
-    const int k = pl.rad[0] * 32 + pl.rad[1];
-    return reg_plan_pair(k);
+    const RegDims d = reg_dims(pl);
+    return d.key && d.R1 <= 16;
 }
 
 hipError_t launch_grad_reg(const LaunchCtx& c) {
@@ -595,11 +944,16 @@ hipError_t launch_grad_reg(const LaunchCtx& c) {
     return hipGetLastError();
 }
 
+hipError_t launch_yfwd_reg(const LaunchCtx& c) {
+    if (!c.n) return hipSuccess;
+    TILD_LAUNCH(c, k_yfwd_reg<kGradRegThreads>, dim3(c.n), dim3(kGradRegThreads), c.lds, c.reps, c.wmap);
+    return hipGetLastError();
+}
+
 bool last_reg_plan(const AxisPlan& pl, int ntypes, int nf) {
-    if (pl.nst != 2 || ntypes < 1 || ntypes > 4 || nf > ntypes + 1) return false;
-    if (!last_reg_variant(pl.rad[0], pl.rad[1], ntypes, nf - ntypes)) return false;
-    const int k = pl.rad[0] * 32 + pl.rad[1];
-    return reg_plan_pair(k);
+    const RegDims d = reg_dims(pl);
+    if (!d.key || ntypes < 1 || ntypes > 4 || nf > ntypes + 1) return false;
+    return last_reg_variant(pl.rad[0], d.R1, d.R2, pl.nst == 2, ntypes) && last_reg_cols(d.R1, d.R2, nf) >= 1;
 }
 
 hipError_t launch_last_reg(const LaunchCtx& c, int koff, int cls) {

@@ -92,33 +92,58 @@ constexpr int kGradThreads = 256;                       // block of the y invers
 constexpr int kC2rThreads = 256;                        // block of the inverse x pass (records)
 constexpr size_t kPlaneLds = 163840;                    // LDS one block may use (MI355X)
 hipError_t launch_mid_grad(const LaunchCtx& c);
-// Two-stage Stockham plans R1 x R2 the register-resident passes are compiled for: the
-// 5-smooth lengths from 24 to 256 that two radices up to 16 make (as the planner splits
-// them), and 21, 28, 35 and 63 points.
-#define TILD_REG_PLANS(X) \
-    X(8, 3) X(5, 5) X(9, 3) X(10, 3) X(8, 4) X(6, 6) X(8, 5) X(9, 5) X(16, 3) X(10, 5) X(9, 6) X(10, 6) X(8, 8) \
-    X(9, 8) X(15, 5) X(10, 8) X(10, 9) X(12, 8) X(10, 10) X(12, 9) X(12, 10) X(16, 8) X(12, 12) X(15, 10) \
-    X(16, 10) X(15, 12) X(16, 12) X(15, 15) X(16, 15) X(16, 16) X(7, 3) X(7, 4) X(7, 5) X(9, 7)
+// Stockham plans the register-resident passes are compiled for, as two groups of stages
+// (A0 A1) (B0 B1) (1: no second stage): a thread runs a group's stages on the R1 = A0 A1
+// and then on the R2 = B0 B1 values it holds, so that a plan of three or four stages takes
+// one exchange through LDS like one of two.  The radices and their order are the planner's.
+#define TILD_REG_PLANS(X)                                                                            \
+    X(8, 1, 3, 1) X(5, 1, 5, 1) X(10, 1, 3, 1) X(8, 1, 4, 1) X(8, 1, 5, 1) X(16, 1, 3, 1)            \
+    X(10, 1, 5, 1) X(8, 1, 8, 1) X(10, 1, 8, 1) X(16, 1, 8, 1) X(16, 1, 10, 1) /* 24 ... 160 */      \
+    X(7, 1, 3, 1) X(7, 1, 4, 1) X(7, 1, 5, 1) X(10, 1, 10, 1)                  /* 21 28 35 100 */     \
+    X(3, 1, 3, 3) X(4, 1, 3, 3) X(5, 1, 3, 3) X(7, 1, 3, 3) X(5, 1, 4, 3)      /* 27 36 45 63 60 */   \
+    X(8, 1, 3, 3) X(5, 1, 5, 3) X(10, 1, 3, 3) X(8, 1, 4, 3) X(8, 1, 5, 3)     /* 72 75 90 96 120 */  \
+    X(5, 1, 5, 5) X(16, 1, 3, 3) X(10, 1, 5, 3) X(8, 1, 8, 3) X(8, 1, 5, 5)    /* 125 144 150 192 200 */ \
+    X(10, 1, 8, 3) X(3, 3, 3, 2) X(4, 3, 3, 3) X(5, 4, 3, 3) X(8, 3, 3, 3)     /* 240 54 108 180 216 */ \
+    X(5, 5, 3, 3)                                                              /* 225 */
+// the radices in order, five bits each
+__host__ __device__ constexpr int reg_plan_key(int a0, int a1, int b0, int b1) {
+    int k = a0;
+    if (a1 > 1) k = k * 32 + a1;
+    k = k * 32 + b0;
+    return b1 > 1 ? k * 32 + b1 : k;
+}
+// Plans of the first two lines: the fused z pass, the y inverse and the plane passes have
+// run these in registers all along, with products and sums fused as the compiler chose
+// there; every other register pass fuses them as the LDS-staged pass it stands for, so that
+// no length's results depend on which of the two runs.
+__host__ __device__ constexpr bool reg_plan_kept(int n) {
+    return n == 24 || n == 25 || n == 30 || n == 32 || n == 40 || n == 48 || n == 50 || n == 64 || n == 80 || n == 128 ||
+           n == 160;
+}
+// key, group sizes and first stage of the second group of an axis plan (key 0: not compiled)
+struct RegDims {
+    int key, R1, R2, group2;
+};
+RegDims reg_dims(const AxisPlan& pl);
 // Fused last-axis pass with register-resident columns (fft_last.hpp): last axes with one
-// of those plans, at most four types (two on axes whose first radix is 12 or more) plus
-// charges.  Blocks of kLastRegThreads threads hold nl_last = last_reg_cols
-// columns; results agree with k_last_fused to rounding.
+// of those plans, at most four types (two on axes above 100 points or of first radix 16)
+// plus charges.  Blocks of kLastRegThreads threads hold nl_last = last_reg_cols columns.
 constexpr int kLastRegThreads = 256;
-// the variants compiled in (plan R1 x R2, types, charge field): a thread of the middle
-// stage holds a coupling coefficient per type for each of its R2 values, at most 40
-__host__ __device__ constexpr bool last_reg_variant(int R1, int R2, int TT, int CH) {
-    return TT <= (R1 >= 12 ? 2 : 4) && TT * R2 <= 40;
+// Plans of two stages run the inverse reversed (RepDev::axr), others as they are; a thread
+// of the coupling stage holds a coefficient per type for each of its R2 (R1) values, at
+// most 50.
+__host__ __device__ constexpr bool last_reg_variant(int A0, int R1, int R2, bool rev, int TT) {
+    return TT <= (R1 * R2 > 100 || A0 == 16 ? 2 : 4) && TT * (rev ? R2 : R1) <= 50;
 }
-// the kernel instantiation of a variant: plans of short axes with up to two types (class 0)
-// or three and four (class 1), and those with R1 >= 12 of the longer axes (class 2); 16 x 3
-// is with the short ones, so that a sweep of sides up to 50 launches one class
-__host__ __device__ constexpr int last_reg_class(int R1, int R2, int TT) {
-    return R1 * R2 > 64 && R1 >= 12 ? 2 : (TT >= 3 ? 1 : 0);
-}
+// the kernel instantiation of a variant: axes up to 100 points with up to two types (class
+// 0) or three and four (class 1), and longer axes (class 2)
+__host__ __device__ constexpr int last_reg_class(int N, int TT) { return N > 100 ? 2 : (TT >= 3 ? 1 : 0); }
 bool last_reg_plan(const AxisPlan& pl, int ntypes, int nf);
-// columns of a block: one middle-stage thread per (column, i < R1, field)
-__host__ __device__ constexpr int last_reg_cols(int R1, int nf) { return kLastRegThreads / (R1 * nf); }
-inline int last_reg_lines(const AxisPlan& pl, int nf) { return last_reg_cols(pl.rad[0], nf); }
+// columns of a block: one thread per (column, index of the larger group, field)
+__host__ __device__ constexpr int last_reg_cols(int R1, int R2, int nf) {
+    return kLastRegThreads / ((R1 > R2 ? R1 : R2) * nf);
+}
+inline int last_reg_lines(const AxisPlan& pl, int nf) { return last_reg_cols(reg_dims(pl).R1, reg_dims(pl).R2, nf); }
 // the two exchange buffers, the inverse stage's twiddles and the ramp weights
 inline size_t last_reg_lds_bytes(const AxisPlan& pl, int nf) {
     const size_t N = (size_t)pl.N, nl = (size_t)last_reg_lines(pl, nf);
@@ -131,46 +156,67 @@ hipError_t launch_last_reg_2(const LaunchCtx& c, int koff);
 hipError_t configure_last_reg_0();
 hipError_t configure_last_reg_1();
 hipError_t configure_last_reg_2();
-// The y inverse of the gradient spectra with register-resident columns (3D, two-stage
-// y plans as above): blocks of kGradRegThreads threads, grad_reg_lines(plan) columns
-// each, grad_reg_chunks per (field, z) plane.
+// The y inverse of the gradient spectra with register-resident columns (3D, y plans as
+// above with R1 <= 16): blocks of kGradRegThreads threads, grad_reg_lines(plan) columns
+// each, grad_reg_chunks per (field, z) plane.  The forward y pass of the half spectra
+// (k_yfwd_reg) has the same blocks.
 constexpr int kGradRegThreads = 128;
 bool grad_reg_plan(const AxisPlan& pl);
-inline int grad_reg_lines(const AxisPlan& pl) { return kGradRegThreads / pl.rad[0]; }
+inline int grad_reg_lines(const AxisPlan& pl) {
+    const RegDims d = reg_dims(pl);
+    return kGradRegThreads / (d.R1 > d.R2 ? d.R1 : d.R2);
+}
 inline int grad_reg_chunks(const AxisPlan& pl, int Nxh) { return (Nxh + grad_reg_lines(pl) - 1) / grad_reg_lines(pl); }
 inline size_t grad_reg_lds_bytes(const AxisPlan& pl) {
     return ((size_t)pl.N * (3 * (size_t)grad_reg_lines(pl) + 1) + (size_t)pl.N) * sizeof(float2);
 }
+inline size_t yfwd_reg_lds_bytes(const AxisPlan& pl) {
+    return ((size_t)pl.N * ((size_t)grad_reg_lines(pl) + 1) + (size_t)pl.N) * sizeof(float2);
+}
 hipError_t launch_grad_reg(const LaunchCtx& c);
-// The forward plane pass with register-resident columns (square planes, two-stage
-// plans as above): one block of kPlaneRegThreads threads per (field, z) plane.
+hipError_t launch_yfwd_reg(const LaunchCtx& c);
+// The forward plane pass with register-resident columns: one block of kPlaneRegThreads
+// threads per (field, z) plane.  k_plane_reg: square planes of the kept two-stage plans;
+// k_plane_rect: any other plane of compiled plans.
 constexpr int kPlaneRegThreads = 512;
 bool plane_reg_plan(const AxisPlan& px, const AxisPlan& py);
 inline size_t plane_reg_lds_bytes(const AxisPlan& pl) {
-    const size_t N = (size_t)pl.N, ldp = (size_t)(((pl.N + 1) / 2) | 1), ldc = (size_t)((pl.N / 2 + 1) | 1);
+    const size_t N = (size_t)pl.N, ldp = (size_t)((pl.N / 2) | 1), ldc = (size_t)((pl.N / 2 + 1) | 1);
     return (N * (ldp > ldc ? ldp : ldc) + N * ldp + 2 * N) * sizeof(float2);
 }
+inline size_t plane_rect_lds_bytes(int Nx, int Ny) {
+    const size_t a = (size_t)Nx * (size_t)((Ny / 2) | 1), b = (size_t)Ny * (size_t)((Nx / 2 + 1) | 1);
+    return ((a > b ? a : b) + a + (size_t)Nx + (size_t)Ny) * sizeof(float2);
+}
 hipError_t launch_plane_reg(const LaunchCtx& c);
+hipError_t launch_plane_rect(const LaunchCtx& c);
 hipError_t configure_plane_reg();
 // Register-resident inverse plane pass (y inverse + x C2R into the gather records) of
-// square planes with a two-stage plan: one block of kPlaneInvThreads threads per (field,
-// z) plane, two blocks to a CU; planes whose y stages outgrow those threads or whose LDS
-// leaves one block to a CU (75 to 108 points a side) take kPlaneInvWide threads, which
-// fill the CU.
+// square planes with a kept two-stage plan: one block of kPlaneInvThreads threads per
+// (field, z) plane, two blocks to a CU.
 constexpr int kPlaneInvThreads = 512, kPlaneInvWide = 1024;
-__host__ __device__ constexpr size_t plane_inv_lds(int R1, int R2) {
-    const size_t N = (size_t)R1 * R2, la = (3 * (N / 2 + 1)) | 1;
-    return (N * la + (size_t)R1 * (R2 - 1)) * sizeof(float2);
+inline size_t plane_inv_lds_bytes(const AxisPlan& pl) {
+    const size_t N = (size_t)pl.N, la = (size_t)((3 * (pl.N / 2 + 1)) | 1);
+    return (N * la + (size_t)pl.rad[0] * (pl.rad[1] - 1)) * sizeof(float2);
 }
-// the block size of a plan (0: no such pass)
-__host__ __device__ constexpr int plane_inv_threads(int R1, int R2) {
-    const int tasks = (R1 * R2 / 2 + 1) * (R1 > R2 ? R1 : R2);
-    return tasks <= kPlaneInvThreads && plane_inv_lds(R1, R2) <= kPlaneLds / 2 ? kPlaneInvThreads
-           : (tasks <= kPlaneInvWide && plane_inv_lds(R1, R2) <= kPlaneLds ? kPlaneInvWide : 0);
-}
-inline size_t plane_inv_lds_bytes(const AxisPlan& pl) { return plane_inv_lds(pl.rad[0], pl.rad[1]); }
 bool plane_inv_plan(const AxisPlan& px, const AxisPlan& py);
-hipError_t launch_plane_inv(const LaunchCtx& c, bool wide);
+// The same for the other plans, all (one or two) fields of a z plane in one block, its x
+// lines paired across them as the separate x pass pairs them; kPlaneInvWide threads where
+// the LDS leaves one block to a CU.
+// the larger of the y inverses (rows of three half spectra per field) and the x exchange
+__host__ __device__ constexpr int plane_all_elems(int N, int nf) {
+    return N * (nf * ((3 * (N / 2 + 1)) | 1) > ((N * ((3 * nf + 1) / 2)) | 1) ? nf * ((3 * (N / 2 + 1)) | 1)
+                                                                             : ((N * ((3 * nf + 1) / 2)) | 1));
+}
+__host__ __device__ constexpr size_t plane_all_lds(int N, int nf) {
+    return ((size_t)plane_all_elems(N, nf) + N) * sizeof(float2);
+}
+__host__ __device__ constexpr int plane_all_threads(int N, int nf) {
+    return plane_all_lds(N, nf) <= kPlaneLds / 2 ? kPlaneInvThreads : (plane_all_lds(N, nf) <= kPlaneLds ? kPlaneInvWide : 0);
+}
+bool plane_all_plan(const AxisPlan& px, const AxisPlan& py, int nf);
+hipError_t launch_plane_inv(const LaunchCtx& c);
+hipError_t launch_plane_all(const LaunchCtx& c, bool wide);
 hipError_t configure_plane_inv();
 hipError_t configure_last_reg();
 hipError_t launch_plane_r2c(const LaunchCtx& c);

@@ -405,18 +405,18 @@ __device__ __forceinline__ void load_srec4(const RepDev& r, int j0, int total, c
     }
 }
 
-// Densities of a tile's rows and their x R2C for axes with a two-stage plan R1 x R2, row
+// Densities of a tile's rows and their x R2C for axes with a compiled plan, row
 // pairs as complex lines with columns in registers between the stages (the transform of
 // the LDS-staged form, in three phases instead of five):
 //   A  task (pair j, i < R2): rows 2j and 2j + 1 at x = i + R2 r from the fixed-point
-//      rows, written to rho on the way; DFT_R1; exchange;
-//   B  task (j, i < R1): twiddles, DFT_R2 -> Z_j(k), over the values the task read;
+//      rows, written to rho on the way; first group; exchange;
+//   B  task (j, i < R1): second group -> Z_j(k), over the values the task read;
 //   C  the two rows' half spectra from Z_k and Z_{N-k}, stored.
-// X: N x ldb exchange; TW: w_N^{i r}; rowid: global row (f, z, y) of each tile row.
-template <int R1, int R2, int NT>
+// X: N x ldb exchange; TW: the second group's twiddles; rowid: global row (f, z, y) of each tile row.
+template <class P, int NT>
 __device__ __forceinline__ void deposit_xfft(const RepDev& r, const unsigned long long* patch, float2* X, const float2* TW,
                                              const int* rowid, int rows, int trows) {
-    constexpr int N = R1 * R2, NXH = N / 2 + 1;
+    constexpr int R1 = P::R1, R2 = P::R2, N = P::N, NXH = N / 2 + 1;
     const int npairs = (rows + 1) / 2, ldb = npairs | 1;
     const double inv_t = r.fix_inv, inv_q = r.fixq_inv;
     float* const rho = r.rho;
@@ -438,7 +438,7 @@ __device__ __forceinline__ void deposit_xfft(const RepDev& r, const unsigned lon
                 G(at32(rho, ob + (uint32_t)n))[0] = v[rr].y;
             }
         }
-        Dft<R1>::run(v);
+        plan_first<P>(v, r.reg_tw[0]);
 #pragma unroll
         for (int q = 0; q < R1; ++q) X[(i * R1 + q) * ldb + j] = v[q];
     }
@@ -450,9 +450,7 @@ __device__ __forceinline__ void deposit_xfft(const RepDev& r, const unsigned lon
         float2 w[R2];
 #pragma unroll
         for (int rr = 0; rr < R2; ++rr) w[rr] = X[(i + R1 * rr) * ldb + j];
-#pragma unroll
-        for (int rr = 1; rr < R2; ++rr) w[rr] = cmul(w[rr], lds_twiddle(TW + i * (R2 - 1) + rr - 1));
-        Dft<R2>::run(w);
+        plan_second_lds<P, true>(w, TW, i);
 #pragma unroll
         for (int q = 0; q < R2; ++q) X[(i + R1 * q) * ldb + j] = w[q];
     }
@@ -531,7 +529,7 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
     float2* const xtw = fbuf + (size_t)Nx * (((rows + 1) / 2) | 1);
     int* const rowid = (int*)(xtw + Nx);
     if (XFFT && xreg) {
-        const int ntw = Nx - (r.reg_key[0] >> 5);   // R1 (R2 - 1)
+        const int ntw = reg_ntw(r.reg_key[0], Nx);
         for (int k = threadIdx.x; k < ntw; k += kDepositThreads) xtw[k] = gld(r.reg_tw[0] + k);
         for (int rr = threadIdx.x; rr < rows; rr += kDepositThreads) {
             const int ly = rr % By, lz = (rr / By) % Bz, f = rr / (By * Bz);
@@ -610,7 +608,9 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
     // densities of the tile rows -> rho and the x-axis R2C (pairs of rows)
     if (XFFT && xreg) {
         switch (r.reg_key[0]) {   // uniform
-#define TILD_CASE(A, B) case A * 32 + B: deposit_xfft<A, B, kDepositThreads>(r, patch, fbuf, xtw, rowid, rows, T * By * Bz); break;
+#define TILD_CASE(A0, A1, B0, B1)      \
+    case reg_plan_key(A0, A1, B0, B1): \
+        deposit_xfft<RegPlan<A0, A1, B0, B1>, kDepositThreads>(r, patch, fbuf, xtw, rowid, rows, T * By * Bz); break;
             TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
             default: break;   // reg_key holds compiled plans only
