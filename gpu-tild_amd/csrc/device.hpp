@@ -116,7 +116,7 @@ struct alignas(64) RepDev {
     int c2r_reg;   // 1: the x C2R runs register-resident (k_c2r_reg)
     int plane_rect;   // 1: the forward plane pass of other planes runs register-resident (k_plane_rect)
     int yfwd_reg;  // 1: the forward y pass runs register-resident (k_yfwd_reg)
-    int plane_all; // 1: y inverse and x C2R of all fields run as one plane pass (k_plane_all)
+    int plane_pair; // > 0: y inverse and x C2R run as one pass (k_plane_inv), this many pairs of lines a block
     // FFT plans (x, y, z)
     AxisPlan ax[3];
     AxisPlan axr;  // inverse plan of the last axis: a two-stage plan reversed, else ax[dim - 1]

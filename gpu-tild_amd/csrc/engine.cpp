@@ -513,19 +513,18 @@ int Batch::add_plain(const System& S, uint32_t seed, std::string& err) {
     // compiled plans; without a plane pass the y transform alone
     h.plane_reg = h.plane_fwd && !tune_.staged && h.grid_off32 && plane_reg_plan(h.ax[0], h.ax[1]) &&
                   plane_reg_lds_bytes(h.ax[0]) <= kPlaneLds ? 1 : 0;
-    h.plane_rect = h.plane_fwd && !h.plane_reg && h.grid_off32 && h.reg_key[0] && h.reg_key[1] &&
-                   plane_rect_lds_bytes(h.Nx, h.Ny) <= kPlaneLds ? 1 : 0;
-    h.yfwd_reg = D == 3 && !h.plane_fwd && h.grid_off32 && h.reg_key[1] && grad_reg_plan(h.ax[1]) ? 1 : 0;
+    h.plane_rect = h.plane_fwd && !h.plane_reg && !tune_.staged && h.grid_off32 && plane_rect_plan(h.ax[0], h.ax[1]) ? 1 : 0;
+    h.yfwd_reg = D == 3 && !h.plane_fwd && !tune_.staged && h.grid_off32 && yfwd_reg_plan(h.ax[1]) ? 1 : 0;
     // the y inverse and the x C2R as one pass per (field, z) plane: square planes with an
     // even two-stage plan, no field phases (whose records need the densities)
     h.plane_inv = D == 3 && !tune_.staged && h.grid_off32 && !h.FPtab && plane_inv_plan(h.ax[0], h.ax[1]) &&
                   h.ax[0].rad[0] == h.ax[1].rad[0] && h.ax[0].rad[1] == h.ax[1].rad[1] ? 1 : 0;
-    h.plane_all = D == 3 && !tune_.staged && h.grid_off32 && !h.FPtab && h.grad_reg && plane_all_plan(h.ax[0], h.ax[1], h.nf) ? 1 : 0;
+    h.plane_pair = D == 3 && !tune_.staged && h.grid_off32 && !h.FPtab && !h.plane_inv ? plane_pairs(h.ax[0], h.ax[1], h.nf) : 0;
 
     // the register form of the x C2R into the records, where the plane pass does not run: one
     // stage-B task per thread, and no more rows per block than leave a block for every CU
     // (a small launch is bound by one block's chain of phases)
-    h.c2r_reg = h.reg_key[0] && h.grid_off32 && !h.FPtab && !h.plane_inv && !h.plane_all ? 1 : 0;
+    h.c2r_reg = h.reg_key[0] && h.grid_off32 && !h.FPtab && !h.plane_inv && !h.plane_pair ? 1 : 0;
     if (h.c2r_reg) {
         const RegDims rd = reg_dims(h.ax[0]);
         int nr = std::max(1, kC2rRegThreads / (nc * std::max(rd.R1, rd.R2)));
@@ -705,9 +704,10 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         if (h.spread_mode == 2) {
             add(PH_TCOUNT, (h.ns + kCountBlock - 1) / kCountBlock, 0);
             add(PH_SCAN, 1, 0);
-            add(PH_TILE, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd, h.reg_key[0] && h.grid_off32));
-            maps[PH_TILE].xfft = maps[PH_TILE].xfft || !h.plane_fwd;
-            maps[PH_TILE].anyrec = maps[PH_TILE].anyrec || !h.srec;
+            const Phase dep = h.plane_fwd ? PH_TILE : PH_TILEX;
+            add(dep, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd, h.reg_key[0] && h.grid_off32));
+            maps[dep].anyrec = maps[dep].anyrec || !h.srec;
+            maps[PH_TILEX].xfft = true;
             if (R.reorder_every > 0) add(PH_RTILE, h.ntiles, 0);
         } else {
             add(PH_SPREADA, R.nblk_part, 0);
@@ -716,16 +716,17 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         {
             MidGeom g = mid_geom(h, 1, h.nf);
             add(PH_PY, g.nouter * g.nchunk, lds_bytes(g.N, g.nl));
+            maps[PH_PLANER].anyrec = maps[PH_PLANER].anyrec || h.plane_rect || h.yfwd_reg;
             if (D == 3 && h.plane_reg) add(PH_PLANER, h.nf * h.Nz, plane_reg_lds_bytes(h.ax[0]));
-            else if (D == 3 && h.plane_rect) add(PH_PLANERECT, h.nf * h.Nz, plane_rect_lds_bytes(h.Nx, h.Ny));
-            else if (D == 3 && h.yfwd_reg) add(PH_YFWD, h.nf * h.Nz * grad_reg_chunks(h.ax[1], h.Nxh), yfwd_reg_lds_bytes(h.ax[1]));
+            else if (D == 3 && h.plane_rect) add(PH_PLANER, h.nf * h.Nz, plane_rect_lds_bytes(h.Nx, h.Ny));
+            else if (D == 3 && h.yfwd_reg) add(PH_PLANER, yfwd_reg_blocks(h.ax[1], h.Nxh, h.nf * h.Nz), yfwd_reg_lds_bytes(h.ax[1]));
             else if (D == 3 && h.plane_fwd) add(PH_PLANEF, h.nf * h.Nz, plane_r2c_lds(h));
             else if (D == 3) add(PH_MIDY_H, g.nouter * g.nchunk, lds_bytes(g.N, g.nl));
         }
         if (D == 3) {
             MidGeom g = mid_grad_geom(h);
             if (h.plane_inv) add(PH_PLANEI, h.nf * h.Nz, plane_inv_lds_bytes(h.ax[1]));
-            else if (h.plane_all) add(plane_all_threads(h.Ny, h.nf) == kPlaneInvWide ? PH_PLANEAW : PH_PLANEA, h.Nz, plane_all_lds(h.Ny, h.nf));
+            else if (h.plane_pair) add(PH_PLANEI, h.Nz * ((3 * h.nf + 2 * h.plane_pair - 1) / (2 * h.plane_pair)), plane_pair_lds_bytes(h.Nx, h.Ny, h.plane_pair));
             else if (h.grad_reg) add(PH_MIDY_GR, h.nf * h.Nz * grad_reg_chunks(h.ax[1], h.Nxh), grad_reg_lds_bytes(h.ax[1]));
             else add(PH_MIDY_G, g.nouter * g.nchunk, lds_bytes(g.N, 3 * g.nl));
             MidGeom gz = mid_geom(h, 2, h.nf);
@@ -740,33 +741,33 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         else add(PH_LAST, (Q + h.nl_last - 1) / h.nl_last, last_lds_bytes(Nla, h.nf, h.last_dirs, h.nl_last));
         const int nc = (h.nf * D + 1) / 2;
         if (h.c2r_reg) add(PH_C2RR, (rows + h.nr_c2r - 1) / h.nr_c2r, c2r_reg_lds_bytes(h.Nx, h.nr_c2r * nc));
-        else if (!h.plane_inv && !h.plane_all) add(PH_C2R, (rows + h.nr_c2r - 1) / h.nr_c2r, lds_bytes(h.Nx, h.nr_c2r * nc));
+        else if (!h.plane_inv && !h.plane_pair) add(PH_C2R, (rows + h.nr_c2r - 1) / h.nr_c2r, lds_bytes(h.Nx, h.nr_c2r * nc));
         add(PH_KPROPS, h.nchunk > 0 ? h.nchunk : 1, 0);
     }
     // Deposit block size: 512 threads when the set's tiles hold ~600 beads or more on
     // average (one or two records per thread), else 256 (small tiles leave most of a
     // larger block idle, and the deposit of a sweep of small replicas took twice as long).
     // A bead of a higher order counts by its nodes against order 1's.
-    {
+    for (Phase dep : {PH_TILE, PH_TILEX}) {
         long long beads = 0, tiles = 0;
-        int want = -1;   // the block size the set's tiled replicas ask for, if they agree
+        int want = -1;   // the block size the launch's replicas ask for, if they agree
         for (int id : ids)
-            if (reps_[id]->h.spread_mode == 2) {
+            if (reps_[id]->h.spread_mode == 2 && (dep == PH_TILE) == (reps_[id]->h.plane_fwd != 0)) {
                 const long long np = std::max(reps_[id]->h.P, 1) + 1, d = reps_[id]->dim;
                 beads += (long long)reps_[id]->ns * (d == 3 ? np * np * np / 8 : np * np / 4);
                 tiles += reps_[id]->h.ntiles;
                 const int w = reps_[id]->dep_threads;
                 want = want == -1 ? w : (want == w ? want : 0);
             }
-        maps[PH_TILE].threads = want == 256 || want == 512 ? want : (tiles > 0 && beads >= 600 * tiles ? 512 : 256);
+        maps[dep].threads = want == 256 || want == 512 ? want : (tiles > 0 && beads >= 600 * tiles ? 512 : 256);
     }
     // Workgroups go to the 8 XCDs round-robin (launch block w runs on XCD w % 8).  Every
     // pass hands each XCD a contiguous run of work items: for the particle-order passes
     // one slab of a spatially ordered replica, so that its L2 holds that slab's grid
     // records; for the FFT passes adjacent column batches, whose rows share cache lines
     // that a single L2 then fetches once.
-    for (Phase ph : {PH_PART, PH_TCOUNT, PH_SPREADA, PH_TILE, PH_XA, PH_XP, PH_MIDY_H, PH_MIDY_G, PH_MIDY_GR,
-                     PH_MIDZ_H, PH_PY, PH_LAST, PH_LASTR, PH_LASTR4, PH_LASTRW, PH_C2R, PH_C2RR, PH_PLANEF, PH_PLANER, PH_PLANERECT, PH_YFWD, PH_PLANEI, PH_PLANEA, PH_PLANEAW}) {
+    for (Phase ph : {PH_PART, PH_TCOUNT, PH_SPREADA, PH_TILE, PH_TILEX, PH_XA, PH_XP, PH_MIDY_H, PH_MIDY_G, PH_MIDY_GR,
+                     PH_MIDZ_H, PH_PY, PH_LAST, PH_LASTR, PH_LASTR4, PH_LASTRW, PH_C2R, PH_C2RR, PH_PLANEF, PH_PLANER, PH_PLANEI}) {
         std::vector<WorkItem>& v = maps[ph].host;
         const size_t n = v.size(), q = n / kXcds, rm = n % kXcds;
         if (n < 2 * (size_t)kXcds) continue;
@@ -779,7 +780,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
     }
     for (int p = 0; p < PH_COUNT; ++p) {
         maps[p].n = (int)maps[p].host.size();
-        if (maps[p].lds > ((p == PH_PLANEF || p == PH_PLANER || p == PH_PLANERECT || p == PH_PLANEI || p == PH_PLANEA || p == PH_PLANEAW || p == PH_LAST || p == PH_LASTR || p == PH_LASTR4 || p == PH_LASTRW) ? kPlaneLds : (size_t)kMaxLds)) { err = "pass needs more LDS than a block may use"; return -TILD_ERR_UNSUPPORTED; }
+        if (maps[p].lds > ((p == PH_PLANEF || p == PH_PLANER || p == PH_PLANEI || p == PH_LAST || p == PH_LASTR || p == PH_LASTR4 || p == PH_LASTRW) ? kPlaneLds : (size_t)kMaxLds)) { err = "pass needs more LDS than a block may use"; return -TILD_ERR_UNSUPPORTED; }
         if (maps[p].dev && (!reorder_only || maps[p].cap < maps[p].n)) {
             // reused buffers are last read by the previous reorder's launches
             HIPCHK(hipStreamSynchronize(stream_));
@@ -1090,10 +1091,9 @@ int Batch::enqueue_steps(SetMaps& m, int nsteps, bool integrate, bool write_forc
         HIPCHK(launch_spread(ctx(PH_SPREADA), k));
         HIPCHK(launch_x_r2c(ctx(PH_XA), true, 0, nullptr, nullptr));
         HIPCHK(launch_tile_deposit(ctx(PH_TILE), k));
+        HIPCHK(launch_tile_deposit(ctx(PH_TILEX), k));
         HIPCHK(launch_plane_r2c(ctx(PH_PLANEF)));
         HIPCHK(launch_plane_reg(ctx(PH_PLANER)));
-        HIPCHK(launch_plane_rect(ctx(PH_PLANERECT)));
-        HIPCHK(launch_yfwd_reg(ctx(PH_YFWD)));
         HIPCHK(launch_mid(ctx(PH_MIDY_H), 1, 0, 0, 0, nullptr));
         HIPCHK(launch_last_fused(ctx(PH_LAST), 0, k));
         HIPCHK(launch_last_reg(ctx(PH_LASTR), k, 0));
@@ -1104,8 +1104,6 @@ int Batch::enqueue_steps(SetMaps& m, int nsteps, bool integrate, bool write_forc
         HIPCHK(launch_x_c2r(ctx(PH_C2R), true, 0, nullptr, nullptr));
         HIPCHK(launch_c2r_reg(ctx(PH_C2RR)));
         HIPCHK(launch_plane_inv(ctx(PH_PLANEI)));
-        HIPCHK(launch_plane_all(ctx(PH_PLANEA), false));
-        HIPCHK(launch_plane_all(ctx(PH_PLANEAW), true));
         // integrating steps claim the next step's records; a force evaluation leaves
         // positions and records as they are
         HIPCHK(launch_particles(ctx(PH_PART), integrate, write_forces ? 1 : 0, k, integrate));
@@ -1239,10 +1237,9 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
             e0 = hipErrorUnknown;
         ok(launch_x_r2c(ctx(PH_XA, 1, 0), true, 0, nullptr, nullptr));
         ok(launch_tile_deposit(ctx(PH_TILE, 1, 1), 0));
+        ok(launch_tile_deposit(ctx(PH_TILEX, 1, 3), 0));
         ok(launch_plane_r2c(ctx(PH_PLANEF, 2, 0)));
         ok(launch_plane_reg(ctx(PH_PLANER, 2, 2)));
-        ok(launch_plane_rect(ctx(PH_PLANERECT, 2, 3)));
-        ok(launch_yfwd_reg(ctx(PH_YFWD, 2, 4)));
         ok(launch_mid(ctx(PH_MIDY_H, 2, 1), 1, 0, 0, 0, nullptr));
         ok(launch_last_fused(ctx(PH_LAST, 3, 0), 0, 0));
         ok(launch_last_reg(ctx(PH_LASTR, 3, 1), 0, 0));
@@ -1253,8 +1250,6 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
         ok(launch_x_c2r(ctx(PH_C2R, 5, 0), true, 0, nullptr, nullptr));
         ok(launch_c2r_reg(ctx(PH_C2RR, 5, 3)));
         ok(launch_plane_inv(ctx(PH_PLANEI, 5, 1)));
-        ok(launch_plane_all(ctx(PH_PLANEA, 5, 2), false));
-        ok(launch_plane_all(ctx(PH_PLANEAW, 5, 4), true));
         ok(launch_particles(ctx(PH_PART, 6, 0), true, 0, 0, true));
         ok(launch_advance(stream_, d_reps_, m->d_ids, m->nids, 1, ev[7][0][0], ev[7][0][1]));
         used[7][0] = m->nids > 0;

@@ -175,14 +175,14 @@ __device__ __forceinline__ void last_reg_block(const RepDev& r, int blk, float2*
                 for (int q = 0; q < R1; ++q) Y1[(i * R1 + q) * ldy + line * NB + b] = z[q];
             }
         };
+        const float fi = (float)i;
         float2 z[RC];
 #pragma unroll
         for (int q = 0; q < RC; ++q) z[q] = make_float2(w[q].x, -w[q].y);
         inverse_first(z, f);
 #pragma unroll
         for (int q = 0; q < RC; ++q) {
-            const int n = i + KS * q;
-            const float kl = 2 * n == N ? 0.f : r.kfac[la] * (float)(2 * n < N ? n : n - N);
+            const float kl = r.kfac[la] * freq_of<KS, N>(i, fi, q);
             z[q] = grad_line(kl, w[q]);
         }
         inverse_first(z, NF + f);

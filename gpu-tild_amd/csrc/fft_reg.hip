@@ -65,10 +65,10 @@ __device__ __forceinline__ void grad_reg_block(const RepDev& r, int blk, float2*
             v[rr] = gld(at32((const float2*)r.Gk, sV + n));
         }
         float2 L[3][R1];
+        const float fi = (float)i;
 #pragma unroll
         for (int rr = 0; rr < R1; ++rr) {
-            const int n = i + R2 * rr;
-            const float ky = 2 * n == N ? 0.f : r.kfac[1] * (float)(2 * n < N ? n : n - N);
+            const float ky = r.kfac[1] * freq_of<R2, N>(i, fi, rr);
             // lines of the conj(FFT(conj)) inverse: conj(u), conj(-i ky u), conj(v)
             L[0][rr] = make_float2(u[rr].x, -u[rr].y);
             L[1][rr] = grad_line(ky, u[rr]);
@@ -100,43 +100,6 @@ __device__ __forceinline__ void grad_reg_block(const RepDev& r, int blk, float2*
     }
 }
 
-// Forward y FFT of the half spectra of one (field, z) plane's columns in place (the
-// operation of k_mid, kernels.hip), where no plane pass runs it (odd sides); the same
-// blocks, one line per column.
-template <class P, int NT>
-__device__ __forceinline__ void yfwd_reg_block(const RepDev& r, int blk, float2* lds) {
-    constexpr int R1 = P::R1, R2 = P::R2, N = P::N, NB = NT / P::RM, ld = NB + 1;
-    const int Nxh = r.Nxh;
-    const int nchunk = (Nxh + NB - 1) / NB;
-    const int o = blk / nchunk, c = blk - o * nchunk;   // o = f Nz + z
-    const int b0 = c * NB, nb = min(NB, Nxh - b0);
-    float2* X1 = lds;                 // N x ld
-    float2* TW1 = X1 + N * ld;
-    const int b = (int)threadIdx.x % NB, i = (int)threadIdx.x / NB;
-    const float2* const tw = r.reg_tw[1];
-    const uint32_t Nxu = (uint32_t)Nxh, s0 = (uint32_t)o * (uint32_t)N * Nxu + (uint32_t)(b0 + b);
-    float2 v[R1];
-    const bool live = i < R2 && b < nb;
-    if (live) {
-#pragma unroll
-        for (int rr = 0; rr < R1; ++rr) v[rr] = gld(at32((const float2*)r.H, s0 + (uint32_t)(i + R2 * rr) * Nxu));
-    }
-    for (int t = threadIdx.x; t < P::NTW; t += NT) TW1[t] = gld(tw + t);
-    if (live) {
-        plan_first<P>(v, tw);
-#pragma unroll
-        for (int q = 0; q < R1; ++q) X1[(i * R1 + q) * ld + b] = v[q];
-    }
-    __syncthreads();
-    if (i < R1 && b < nb) {
-        float2 w[R2];
-#pragma unroll
-        for (int rr = 0; rr < R2; ++rr) w[rr] = X1[(i + R1 * rr) * ld + b];
-        plan_second_lds<P, true>(w, TW1, i);
-#pragma unroll
-        for (int q = 0; q < R2; ++q) gst(at32(r.H, s0 + (uint32_t)(i + R1 * q) * Nxu), w[q]);
-    }
-}
 }  // namespace
 
 template <int NT>
@@ -149,23 +112,6 @@ __global__ void __launch_bounds__(NT) k_grad_reg(const RepDev* __restrict__ reps
 #define TILD_CASE(A0, A1, B0, B1)          \
     case reg_plan_key(A0, A1, B0, B1):     \
         if constexpr ((A0) * (A1) <= 16) grad_reg_block<RegPlan<A0, A1, B0, B1>, NT>(r, wi.blk, lds); \
-        break;
-        TILD_REG_PLANS(TILD_CASE)
-#undef TILD_CASE
-        default: break;   // excluded by grad_reg_plan on the host
-    }
-}
-
-template <int NT>
-__global__ void __launch_bounds__(NT) k_yfwd_reg(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
-    extern __shared__ float2 lds[];
-    const WorkItem wi = wmap[blockIdx.x];
-    const RepDev& r = reps[wi.rep];
-    warm_desc<0, 1, 6, 7>(r);
-    switch (r.reg_key[1]) {   // uniform per block
-#define TILD_CASE(A0, A1, B0, B1)          \
-    case reg_plan_key(A0, A1, B0, B1):     \
-        if constexpr ((A0) * (A1) <= 16) yfwd_reg_block<RegPlan<A0, A1, B0, B1>, NT>(r, wi.blk, lds); \
         break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
@@ -261,23 +207,6 @@ __device__ __forceinline__ void plane_reg_block(const RepDev& r, int blk, float2
 }
 }  // namespace
 
-template <int NT>
-__global__ void __launch_bounds__(NT) k_plane_reg(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
-    extern __shared__ float2 lds[];
-    const WorkItem wi = wmap[blockIdx.x];
-    const RepDev& r = reps[wi.rep];
-    warm_desc<0, 1, 6, 7>(r);
-    switch (r.reg_key[0]) {   // uniform per block
-#define TILD_CASE(A0, A1, B0, B1)          \
-    case reg_plan_key(A0, A1, B0, B1):     \
-        if constexpr (reg_plan_kept(A0 * A1 * B0 * B1) && A0 * B0 % 2 == 0 && A0 * B0 <= 128) plane_reg_block<A0, B0, NT>(r, wi.blk, lds); \
-        break;
-        TILD_REG_PLANS(TILD_CASE)
-#undef TILD_CASE
-        default: break;   // excluded by plane_reg_plan on the host
-    }
-}
-
 // The same for any even plane of compiled plans (sides of equal or unequal plans): the x
 // phases compiled per x plan, the y phases per y plan, bit for bit the LDS-staged pass.
 namespace {
@@ -351,16 +280,11 @@ __device__ __forceinline__ void plane_rect_y(const RepDev& r, uint32_t hbase, fl
         for (int q = 0; q < R2; ++q) gst(at32(r.H, hbase + (uint32_t)((i + R1 * q) * nxh + k)), v[q]);
     }
 }
-}  // namespace
 
 template <int NT>
-__global__ void __launch_bounds__(NT) k_plane_rect(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
-    extern __shared__ float2 lds[];
-    const WorkItem wi = wmap[blockIdx.x];
-    const RepDev& r = reps[wi.rep];
-    warm_desc<0, 1, 6, 7>(r);
+__device__ __forceinline__ void plane_rect_block(const RepDev& r, int blk, float2* lds) {
     const int Nx = r.Nx, Ny = r.Ny, nxh = r.Nxh, ldp = (Ny / 2) | 1, ldc = nxh | 1;
-    const int z = wi.blk % r.Nz, f = wi.blk / r.Nz;
+    const int z = blk % r.Nz, f = blk / r.Nz;
     float2* Xa = lds;                                   // x first-group output, later the y one
     float2* Xb = Xa + max(Nx * ldp, Ny * ldc);          // Z: x transforms of the row pairs
     float2* TWx = Xb + Nx * ldp;
@@ -374,18 +298,103 @@ __global__ void __launch_bounds__(NT) k_plane_rect(const RepDev* __restrict__ re
     const uint32_t pbase = (uint32_t)f * (uint32_t)r.M + (uint32_t)z * (uint32_t)(Nx * Ny);
     const uint32_t hbase = ((uint32_t)f * (uint32_t)r.Nz + (uint32_t)z) * (uint32_t)(Ny * nxh);
     switch (r.reg_key[0]) {   // uniform per block
-#define TILD_CASE(A0, A1, B0, B1) \
-    case reg_plan_key(A0, A1, B0, B1): plane_rect_x<RegPlan<A0, A1, B0, B1>, NT>(r, pbase, Xa, Xb, TWx); break;
+#define TILD_CASE(A0, A1, B0, B1)          \
+    case reg_plan_key(A0, A1, B0, B1):     \
+        if constexpr ((A0) * (A1) <= 16 && (B0) * (B1) <= 16) plane_rect_x<RegPlan<A0, A1, B0, B1>, NT>(r, pbase, Xa, Xb, TWx); \
+        break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
-        default: break;   // compiled plans only
+        default: break;   // excluded by plane_rect_plan on the host
     }
     switch (r.reg_key[1]) {
-#define TILD_CASE(A0, A1, B0, B1) \
-    case reg_plan_key(A0, A1, B0, B1): plane_rect_y<RegPlan<A0, A1, B0, B1>, NT>(r, hbase, Xa, Xb, TWy); break;
+#define TILD_CASE(A0, A1, B0, B1)          \
+    case reg_plan_key(A0, A1, B0, B1):     \
+        if constexpr ((A0) * (A1) <= 16 && (B0) * (B1) <= 16) plane_rect_y<RegPlan<A0, A1, B0, B1>, NT>(r, hbase, Xa, Xb, TWy); \
+        break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
         default: break;
+    }
+}
+
+// Forward y FFT of the half spectra of a (field, z) plane's columns in place (the operation
+// of k_mid, kernels.hip), where the deposit transforms x (odd sides): kYfwdThreads threads
+// take NB columns, so that a block takes several such pieces; live: the piece exists.
+template <class P>
+__device__ __forceinline__ void yfwd_piece(const RepDev& r, int piece, bool live, float2* lds) {
+    constexpr int R1 = P::R1, R2 = P::R2, N = P::N, NB = kYfwdThreads / P::RM, ld = NB + 1;
+    const int Nxh = r.Nxh, nchunk = (Nxh + NB - 1) / NB;
+    const int o = piece / nchunk, c = piece - o * nchunk;   // o = f Nz + z
+    const int b0 = c * NB, nb = live ? min(NB, Nxh - b0) : 0;
+    float2* X1 = lds;                 // N x ld
+    float2* TW1 = X1 + N * ld;
+    const int tid = (int)threadIdx.x % kYfwdThreads, b = tid % NB, i = tid / NB;
+    const float2* const tw = r.reg_tw[1];
+    const uint32_t Nxu = (uint32_t)Nxh, s0 = (uint32_t)o * (uint32_t)N * Nxu + (uint32_t)(b0 + b);
+    float2 v[R1];
+    if (i < R2 && b < nb) {
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) v[rr] = gld(at32((const float2*)r.H, s0 + (uint32_t)(i + R2 * rr) * Nxu));
+    }
+    for (int t = tid; t < P::NTW; t += kYfwdThreads) TW1[t] = gld(tw + t);
+    if (i < R2 && b < nb) {
+        plan_first<P>(v, tw);
+#pragma unroll
+        for (int q = 0; q < R1; ++q) X1[(i * R1 + q) * ld + b] = v[q];
+    }
+    __syncthreads();
+    if (i < R1 && b < nb) {
+        float2 w[R2];
+#pragma unroll
+        for (int rr = 0; rr < R2; ++rr) w[rr] = X1[(i + R1 * rr) * ld + b];
+        plan_second_lds<P, true>(w, TW1, i);
+#pragma unroll
+        for (int q = 0; q < R2; ++q) gst(at32(r.H, s0 + (uint32_t)(i + R1 * q) * Nxu), w[q]);
+    }
+}
+}  // namespace
+
+// ANY: some replica of the set takes one of the two other forms; without them the kernel
+// holds the kept squares only, and its registers (74 against 128).
+template <int NT, bool ANY>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) k_plane_reg(const RepDev* __restrict__ reps,
+                                                                                        const WorkItem* __restrict__ wmap) {
+    extern __shared__ float2 lds[];
+    const WorkItem wi = wmap[blockIdx.x];
+    const RepDev& r = reps[wi.rep];
+    if (ANY) warm_desc<0, 1, 6, 7, 8>(r);
+    else warm_desc<0, 1, 6, 7>(r);
+    if constexpr (ANY) {   // uniform per block, like the switches
+        if (r.plane_rect) {
+            plane_rect_block<NT>(r, wi.blk, lds);
+            return;
+        }
+        if (r.yfwd_reg) {
+            const int sub = (int)threadIdx.x / kYfwdThreads, piece = wi.blk * (NT / kYfwdThreads) + sub;
+            switch (r.reg_key[1]) {
+#define TILD_CASE(A0, A1, B0, B1)                                                                    \
+    case reg_plan_key(A0, A1, B0, B1):                                                               \
+        if constexpr ((A0) * (A1) <= 16 && (B0) * (B1) <= 16) {                                      \
+            using P = RegPlan<A0, A1, B0, B1>;                                                       \
+            constexpr int NB = kYfwdThreads / P::RM, elems = P::N * (NB + 2);                        \
+            yfwd_piece<P>(r, piece, piece < r.nf * r.Nz * ((r.Nxh + NB - 1) / NB), lds + sub * elems); \
+        }                                                                                            \
+        break;
+                TILD_REG_PLANS(TILD_CASE)
+#undef TILD_CASE
+                default: break;   // excluded by yfwd_reg_plan on the host
+            }
+            return;
+        }
+    }
+    switch (r.reg_key[0]) {
+#define TILD_CASE(A0, A1, B0, B1)          \
+    case reg_plan_key(A0, A1, B0, B1):     \
+        if constexpr (reg_plan_kept(A0 * A1 * B0 * B1) && A0 * B0 % 2 == 0 && A0 * B0 <= 128) plane_reg_block<A0, B0, NT>(r, wi.blk, lds); \
+        break;
+        TILD_REG_PLANS(TILD_CASE)
+#undef TILD_CASE
+        default: break;   // excluded by plane_reg_plan on the host
     }
 }
 
@@ -441,10 +450,10 @@ __device__ __forceinline__ void plane_inv_block(const RepDev& r, int blk, float2
             v[rr] = gld(at32((const float2*)r.Gk, sV + o));
         }
         float2 L[3][R1];
+        const float fi = (float)i;
 #pragma unroll
         for (int rr = 0; rr < R1; ++rr) {
-            const int n = i + R2 * rr;
-            const float ky = 2 * n == N ? 0.f : kfy * (float)(2 * n < N ? n : n - N);
+            const float ky = kfy * freq_of<R2, N>(i, fi, rr);
             // lines of the conj(FFT(conj)) inverse: conj(u), conj(-i ky u), conj(v)
             L[0][rr] = make_float2(u[rr].x, -u[rr].y);
             L[1][rr] = grad_line(ky, u[rr]);
@@ -490,20 +499,18 @@ __device__ __forceinline__ void plane_inv_block(const RepDev& r, int blk, float2
         const bool rowline = c < N;
         const int ya = rowline ? c : 2 * (c - N), yb = rowline ? c : ya + 1;
         const int la = rowline ? 0 : 2, lb = rowline ? 1 : 2;
+        const float fi = (float)i;
 #pragma unroll
         for (int rr = 0; rr < R1; ++rr) {
-            const int kn = i + R2 * rr;                 // full-spectrum index
-            const bool upper = kn >= NXH;
-            const int kk = upper ? N - kn : kn;         // its half-spectrum column
-            float2 A = X[ya * LA + la * NXH + kk];
-            float2 B = yb < N ? X[yb * LA + lb * NXH + kk] : make_float2(0.f, 0.f);
-            const bool self = kk == 0 || 2 * kk == N;
+            const HalfEntry e = half_entry<R2, N>(i, fi, rr);   // of the full-spectrum index
+            float2 A = X[ya * LA + la * NXH + e.kk];
+            float2 B = yb < N ? X[yb * LA + lb * NXH + e.kk] : make_float2(0.f, 0.f);
             if (rowline) {   // the x derivative: -i k_x (0 on the Nyquist column)
-                const float kx = self && kk != 0 ? 0.f : kfx * (float)kk;
+                const float kx = kfx * e.k;
                 A = make_float2(kx * A.y, -kx * A.x);
             }
-            if (self) { A.y = 0.f; B.y = 0.f; }
-            hold[ct][rr] = upper ? make_float2(A.x + B.y, A.y - B.x) : make_float2(A.x - B.y, -(A.y + B.x));
+            if (e.self) { A.y = 0.f; B.y = 0.f; }
+            hold[ct][rr] = e.upper ? make_float2(A.x + B.y, A.y - B.x) : make_float2(A.x - B.y, -(A.y + B.x));
         }
         Dft<R1>::run(hold[ct]);
     }
@@ -566,13 +573,173 @@ __device__ __forceinline__ void plane_inv_block(const RepDev& r, int blk, float2
 }
 }  // namespace
 
+// The inverse plane pass of any other plane of compiled plans, bit for bit the y inverse
+// and the x pass it stands for.  That x pass takes the real lines of a row (line f 3 + d of
+// field f's component d) two to a complex line, so a block takes one such pair of lines of
+// a z plane (more where that leaves threads idle, plane_pairs): their y inverses over the
+// plane's columns, the paired x transform of its rows, and their components of the records.
+// One pair of 96 x 96 points fits half a CU's LDS where a field's three lines do not.
+namespace {
+template <class P, int NT>
+__device__ __forceinline__ void plane_pair_y(const RepDev& r, int z, int l0, int nl, int la, float2* X, const float2* TW) {
+    constexpr int R1 = P::R1, R2 = P::R2, N = P::N;
+    const int nxh = r.Nxh;   // rows: [line][k]
+    const float2* const tw = r.reg_tw[1];
+    const uint32_t Mhu = (uint32_t)r.Mh, plane = (uint32_t)z * (uint32_t)(N * nxh);
+    const FastDiv dnx(nxh);
+    // A: first group of column k of line l0 + s
+    for (int task = threadIdx.x; task < nl * nxh * R2; task += NT) {
+        int k;
+        const int rest = dnx.div(task, k), i = rest % R2, s = rest / R2;
+        const int l = l0 + s, f = l / 3, d = l - 3 * f;
+        const uint32_t src = (uint32_t)(f * 3 + (d == 2 ? 2 : 0)) * Mhu + plane + (uint32_t)k;
+        float2 v[R1];
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) v[rr] = gld(at32((const float2*)r.Gk, src + (uint32_t)((i + R2 * rr) * nxh)));
+        const float fi = (float)i;
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) {
+            // lines of the conj(FFT(conj)) inverse: conj(u), conj(-i ky u), conj(v)
+            v[rr] = pick(d == 1, grad_line(r.kfac[1] * freq_of<R2, N>(i, fi, rr), v[rr]), make_float2(v[rr].x, -v[rr].y));
+        }
+        plan_first<P>(v, tw);
+#pragma unroll
+        for (int q = 0; q < R1; ++q) X[(i * R1 + q) * la + s * nxh + k] = v[q];
+    }
+    __syncthreads();
+    // B: second group over the rows the task read; conj of the result
+    for (int task = threadIdx.x; task < nl * nxh * R1; task += NT) {
+        int k;
+        const int rest = dnx.div(task, k), i = rest % R1, s = rest / R1;
+        float2* Xc = X + s * nxh + k;
+        float2 w[R2];
+#pragma unroll
+        for (int rr = 0; rr < R2; ++rr) w[rr] = Xc[(i + R1 * rr) * la];
+        plan_second_lds<P, true>(w, TW, i);
+#pragma unroll
+        for (int q = 0; q < R2; ++q) Xc[(i + R1 * q) * la] = conjf2(w[q]);
+    }
+    __syncthreads();
+}
+
+template <class P, int NT>
+__device__ __forceinline__ void plane_pair_x(const RepDev& r, int z, int l0, int nl, int la, float2* X, const float2* TW) {
+    constexpr int R1 = P::R1, R2 = P::R2, N = P::N, NXH = N / 2 + 1;
+    constexpr int CT = plane_pair_hold(R1);      // tasks of a thread
+    const int ny = r.Ny, np = (nl + 1) / 2, ncl = ny * np, lc = ncl | 1;   // complex lines (row y, pair j)
+    const float2* const tw = r.reg_tw[0];
+    const float kf = r.kfac[0];
+    const FastDiv dncl(ncl), dnp(np);
+    // C: first group of line c, held across a barrier: the exchange takes the rows' place
+    float2 hold[CT][R1];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        const int task = (int)threadIdx.x + ct * NT;
+        if (task >= ncl * R2) break;
+        int c, j;
+        const int i = dncl.div(task, c), y = dnp.div(c, j);
+        const int la0 = l0 + 2 * j, d0 = la0 - 3 * (la0 / 3), d1 = d0 == 2 ? 0 : d0 + 1;
+        const bool two = 2 * j + 1 < nl;
+        const float2* ra = X + y * la + 2 * j * NXH;
+        const float2* rb = ra + (two ? NXH : 0);
+        const float fi = (float)i;
+        float2 a[R1], b[R1];
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) {
+            const int kk = half_entry<R2, N>(i, fi, rr).kk;
+            a[rr] = ra[kk];
+            b[rr] = rb[kk];
+        }
+#pragma unroll
+        for (int rr = 0; rr < R1; ++rr) {
+            const HalfEntry e = half_entry<R2, N>(i, fi, rr);   // of the full-spectrum index
+            const float kx = kf * e.k;
+            float2 A = pick(d0 == 0, x_gradient(kx, a[rr]), a[rr]), B = pick(d1 == 0, x_gradient(kx, b[rr]), b[rr]);
+            if (!two) B = make_float2(0.f, 0.f);
+            if (e.self) { A.y = 0.f; B.y = 0.f; }
+            hold[ct][rr] = e.upper ? make_float2(A.x + B.y, A.y - B.x) : make_float2(A.x - B.y, -(A.y + B.x));
+        }
+        plan_first<P>(hold[ct], tw);
+        settle<R1>(hold[ct]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        const int task = (int)threadIdx.x + ct * NT;
+        if (task >= ncl * R2) break;
+        int c;
+        const int i = dncl.div(task, c);
+#pragma unroll
+        for (int q = 0; q < R1; ++q) X[(i * R1 + q) * lc + c] = hold[ct][q];
+    }
+    __syncthreads();
+    // D: second group -> the pairs' components of the records at x = i + R1 q (adjacent
+    // lanes: adjacent x)
+    const uint32_t M3 = 3u * (uint32_t)r.M, base = 3u * (uint32_t)(z * N * ny);
+    for (int task = threadIdx.x; task < ncl * R1; task += NT) {
+        const int i = task % R1, c = task / R1;
+        int j;
+        const int y = dnp.div(c, j);
+        const int la0 = l0 + 2 * j, f0 = la0 / 3, d0 = la0 - 3 * f0;
+        float2 w[R2];
+#pragma unroll
+        for (int rr = 0; rr < R2; ++rr) w[rr] = X[(i + R1 * rr) * lc + c];
+        plan_second_lds<P, true>(w, TW, i);
+        settle<R2>(w);
+        const uint32_t o = base + 3u * (uint32_t)(y * N + i) + (uint32_t)f0 * M3;
+        const uint32_t p0 = o + (uint32_t)d0, p1 = d0 == 2 ? o + M3 : p0 + 1;
+#pragma unroll
+        for (int q = 0; q < R2; ++q) G(at32((float*)r.G3, p0 + 3u * R1 * q))[0] = w[q].x;
+        if (2 * j + 1 < nl) {
+#pragma unroll
+            for (int q = 0; q < R2; ++q) G(at32((float*)r.G3, p1 + 3u * R1 * q))[0] = -w[q].y;
+        }
+    }
+}
+
 template <int NT>
-__global__ void __launch_bounds__(NT) k_plane_inv(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
+__device__ __forceinline__ void plane_pair_block(const RepDev& r, int blk, float2* lds) {
+    const int nlines = 3 * r.nf, per = 2 * r.plane_pair, nb = (nlines + per - 1) / per;
+    const int z = blk / nb, l0 = per * (blk - z * nb), nl = min(per, nlines - l0), la = (per * r.Nxh) | 1;
+    float2* TWy = lds + plane_pair_elems(r.Nx, r.Ny, r.plane_pair);   // second groups' twiddles
+    float2* TWx = TWy + r.Ny;
+    {
+        const int ny = reg_ntw(r.reg_key[1], r.Ny), nx = reg_ntw(r.reg_key[0], r.Nx);
+        for (int t = threadIdx.x; t < ny; t += NT) TWy[t] = gld(r.reg_tw[1] + t);
+        for (int t = threadIdx.x; t < nx; t += NT) TWx[t] = gld(r.reg_tw[0] + t);
+    }
+    switch (r.reg_key[1]) {   // uniform per block
+#define TILD_CASE(A0, A1, B0, B1)          \
+    case reg_plan_key(A0, A1, B0, B1):     \
+        if constexpr ((A0) * (A1) <= 16 && (B0) * (B1) <= 16) plane_pair_y<RegPlan<A0, A1, B0, B1>, NT>(r, z, l0, nl, la, lds, TWy); \
+        break;
+        TILD_REG_PLANS(TILD_CASE)
+#undef TILD_CASE
+        default: break;   // excluded by plane_pairs on the host
+    }
+    switch (r.reg_key[0]) {
+#define TILD_CASE(A0, A1, B0, B1)          \
+    case reg_plan_key(A0, A1, B0, B1):     \
+        if constexpr ((A0) * (A1) <= 16 && (B0) * (B1) <= 16) plane_pair_x<RegPlan<A0, A1, B0, B1>, NT>(r, z, l0, nl, la, lds, TWx); \
+        break;
+        TILD_REG_PLANS(TILD_CASE)
+#undef TILD_CASE
+        default: break;
+    }
+}
+}  // namespace
+
+template <int NT>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) k_plane_inv(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
     extern __shared__ float2 lds[];
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
-    warm_desc<0, 1, 3, 6, 7>(r);
-    switch (r.reg_key[1]) {   // uniform per block
+    warm_desc<0, 1, 3, 6, 7, 8>(r);
+    if (r.plane_pair) {   // uniform per block, like the switch
+        plane_pair_block<NT>(r, wi.blk, lds);
+        return;
+    }
+    switch (r.reg_key[1]) {
 #define TILD_CASE(A0, A1, B0, B1)          \
     case reg_plan_key(A0, A1, B0, B1):     \
         if constexpr (reg_plan_kept(A0 * A1 * B0 * B1) && (A0 * B0 / 2 + 1) * (A0 > B0 ? A0 : B0) <= NT) \
@@ -581,175 +748,6 @@ __global__ void __launch_bounds__(NT) k_plane_inv(const RepDev* __restrict__ rep
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
         default: break;   // excluded by plane_inv_plan on the host
-    }
-}
-
-// The inverse plane pass for the other square plans: all NF fields of one z plane in one
-// block, the x lines paired as the separate x pass pairs them (real lines f 3 + d of a
-// row, two to a complex line), so that the records are bit for bit those of the y inverse
-// and the x pass.  The phases of plane_inv_block; an odd count of lines pairs the last
-// with zeros.
-namespace {
-template <class P, int NT, int NF>
-__device__ __forceinline__ void plane_all_block(const RepDev& r, int z, float2* lds) {
-    constexpr int R1 = P::R1, R2 = P::R2, N = P::N, NXH = N / 2 + 1;
-    constexpr int LA = (3 * NXH) | 1;             // row stride of a field's y inverses: [f][y][line][k]
-    constexpr int NL = 3 * NF, NC = (NL + 1) / 2; // real and complex x lines per row
-    constexpr int NCL = N * NC, LC = NCL | 1;     // x lines, row stride of the x exchange
-    constexpr int CT = (NCL * R2 + NT - 1) / NT, DT = (NCL * R1 + NT - 1) / NT;
-    constexpr int NE = plane_all_elems(N, NF);
-    static_assert(NF * N * LA <= NE && N * LC <= NE && 3 * NF * N * N <= 2 * NE, "plane_all_block: buffer");
-    float2* X = lds;                              // NF x N x LA, then the x exchange (N x LC), then the records
-    float2* TW = X + NE;                          // the second group's twiddles (one plan on x and y)
-    const float2* const twx = r.reg_tw[0];
-    const float2* const twy = r.reg_tw[1];
-    for (int t = threadIdx.x; t < P::NTW; t += NT) TW[t] = gld(twy + t);
-    const uint32_t Mhu = (uint32_t)r.Mh;
-    const uint32_t plane = (uint32_t)z * (uint32_t)(N * NXH);
-    const float kfy = r.kfac[1], kfx = r.kfac[0];
-    // A: y first group of the three lines of column k
-    for (int task = threadIdx.x; task < NF * NXH * R2; task += NT) {
-        const int k = task % NXH, rest = task / NXH, i = rest % R2, f = rest / R2;
-        const uint32_t sU = (uint32_t)(f * 3) * Mhu + plane, sV = sU + 2u * Mhu;
-        float2 u[R1], v[R1];
-#pragma unroll
-        for (int rr = 0; rr < R1; ++rr) {
-            const uint32_t o = (uint32_t)((i + R2 * rr) * NXH + k);
-            u[rr] = gld(at32((const float2*)r.Gk, sU + o));
-            v[rr] = gld(at32((const float2*)r.Gk, sV + o));
-        }
-        float2* Xf = X + f * (N * LA) + k;
-        float2 L[R1];
-#pragma unroll
-        for (int l = 0; l < 3; ++l) {
-#pragma unroll
-            for (int rr = 0; rr < R1; ++rr) {
-                const int n = i + R2 * rr;
-                const float ky = 2 * n == N ? 0.f : kfy * (float)(2 * n < N ? n : n - N);
-                // lines of the conj(FFT(conj)) inverse: conj(u), conj(-i ky u), conj(v)
-                L[rr] = l == 0 ? make_float2(u[rr].x, -u[rr].y)
-                               : (l == 1 ? grad_line(ky, u[rr]) : make_float2(v[rr].x, -v[rr].y));
-            }
-            plan_first<P>(L, twy);
-#pragma unroll
-            for (int q = 0; q < R1; ++q) Xf[(i * R1 + q) * LA + l * NXH] = L[q];
-        }
-    }
-    __syncthreads();
-    // B: y second group; Y_l(y, k) = conj of the result, over the rows the task read
-    for (int task = threadIdx.x; task < NF * NXH * R1; task += NT) {
-        const int k = task % NXH, rest = task / NXH, i = rest % R1, f = rest / R1;
-        float2* Xf = X + f * (N * LA) + k;
-#pragma unroll
-        for (int l = 0; l < 3; ++l) {
-            float2 w[R2];
-#pragma unroll
-            for (int rr = 0; rr < R2; ++rr) w[rr] = Xf[(i + R1 * rr) * LA + l * NXH];
-            plan_second_lds<P, true>(w, TW, i);
-#pragma unroll
-            for (int q = 0; q < R2; ++q) Xf[(i + R1 * q) * LA + l * NXH] = conjf2(w[q]);
-        }
-    }
-    __syncthreads();
-    // C: x first group of complex line (row y, j): real lines 2j and 2j + 1 = f 3 + d
-    float2 hold[CT][R1];
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-        const int task = (int)threadIdx.x + ct * NT;
-        if (task >= NCL * R2) break;
-        const int c = task % NCL, i = task / NCL, y = c / NC, j = c - y * NC;
-        const int la = 2 * j, lb = la + 1, fa = la / 3, da = la - 3 * fa, fb = lb / 3, db = lb - 3 * fb;
-        const float2* pa = X + fa * (N * LA) + y * LA + da * NXH;
-        const float2* pb = X + (lb < NL ? fb * (N * LA) + y * LA + db * NXH : 0);
-#pragma unroll
-        for (int rr = 0; rr < R1; ++rr) {
-            const int kn = i + R2 * rr;                 // full-spectrum index
-            const bool upper = kn >= NXH;
-            const int kk = upper ? N - kn : kn;         // its half-spectrum column
-            float2 A = pa[kk], B = lb < NL ? pb[kk] : make_float2(0.f, 0.f);
-            const bool self = kk == 0 || 2 * kk == N;
-            const float kx = self && kk != 0 ? 0.f : kfx * (float)kk;
-            if (da == 0) A = x_gradient(kx, A);
-            if (db == 0) B = x_gradient(kx, B);
-            if (self) { A.y = 0.f; B.y = 0.f; }
-            hold[ct][rr] = upper ? make_float2(A.x + B.y, A.y - B.x) : make_float2(A.x - B.y, -(A.y + B.x));
-        }
-        plan_first<P>(hold[ct], twx);
-        settle<R1>(hold[ct]);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-        const int task = (int)threadIdx.x + ct * NT;
-        if (task >= NCL * R2) break;
-        const int c = task % NCL, i = task / NCL;
-#pragma unroll
-        for (int q = 0; q < R1; ++q) X[(i * R1 + q) * LC + c] = hold[ct][q];
-    }
-    __syncthreads();
-    // D: x second group -> the real lines at x = i + R1 q, held across a barrier and laid out
-    // as the fields' records [f][y][x](g_x, g_y, g_z)
-    float2 out[DT][R2];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-        const int task = (int)threadIdx.x + dt * NT;
-        if (task >= NCL * R1) break;
-        const int i = task % R1, c = task / R1;   // adjacent lanes: adjacent x
-#pragma unroll
-        for (int rr = 0; rr < R2; ++rr) out[dt][rr] = X[(i + R1 * rr) * LC + c];
-        plan_second_lds<P, true>(out[dt], TW, i);
-        settle<R2>(out[dt]);
-    }
-    __syncthreads();
-    float* rec = (float*)X;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-        const int task = (int)threadIdx.x + dt * NT;
-        if (task >= NCL * R1) break;
-        const int i = task % R1, c = task / R1, y = c / NC, j = c - y * NC;
-        const int la = 2 * j, lb = la + 1, fa = la / 3, da = la - 3 * fa, fb = lb / 3, db = lb - 3 * fb;
-#pragma unroll
-        for (int q = 0; q < R2; ++q) {
-            const int x = i + R1 * q;
-            rec[((fa * N + y) * N + x) * 3 + da] = out[dt][q].x;
-            if (lb < NL) rec[((fb * N + y) * N + x) * 3 + db] = -out[dt][q].y;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        const uint32_t rec0 = (uint32_t)f * (uint32_t)r.M + (uint32_t)z * (uint32_t)(N * N);
-        const float* src = rec + f * 3 * N * N;
-        if constexpr (N % 2 == 0) {   // 12 rec0 bytes, 16-byte aligned
-            float4* dst = (float4*)((char*)r.G3 + ((rec0 << 3) + (rec0 << 2)));
-            for (int t = threadIdx.x; t < 3 * N * N / 4; t += NT) gst(dst + t, ((const float4*)src)[t]);
-        } else {
-            float* dst = (float*)((char*)r.G3 + ((rec0 << 3) + (rec0 << 2)));
-            for (int t = threadIdx.x; t < 3 * N * N; t += NT) G(dst)[t] = src[t];
-        }
-    }
-}
-}  // namespace
-
-template <int NT>
-__global__ void __launch_bounds__(NT) k_plane_all(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
-    extern __shared__ float2 lds[];
-    const WorkItem wi = wmap[blockIdx.x];
-    const RepDev& r = reps[wi.rep];
-    warm_desc<0, 1, 3, 6, 7>(r);
-    switch (r.reg_key[1] * 2 + (r.nf == 2 ? 1 : 0)) {   // uniform per block
-#define TILD_CASE(A0, A1, B0, B1)                                                                          \
-    case reg_plan_key(A0, A1, B0, B1) * 2:                                                                 \
-        if constexpr (!reg_plan_kept(A0 * A1 * B0 * B1) && A0 * A1 <= 16 && plane_all_threads(A0 * A1 * B0 * B1, 1) == NT) \
-            plane_all_block<RegPlan<A0, A1, B0, B1>, NT, 1>(r, wi.blk, lds);                               \
-        break;                                                                                             \
-    case reg_plan_key(A0, A1, B0, B1) * 2 + 1:                                                             \
-        if constexpr (!reg_plan_kept(A0 * A1 * B0 * B1) && A0 * A1 <= 16 && plane_all_threads(A0 * A1 * B0 * B1, 2) == NT) \
-            plane_all_block<RegPlan<A0, A1, B0, B1>, NT, 2>(r, wi.blk, lds);                               \
-        break;
-        TILD_REG_PLANS(TILD_CASE)
-#undef TILD_CASE
-        default: break;   // excluded by plane_all_plan on the host
     }
 }
 
@@ -790,31 +788,28 @@ __device__ __forceinline__ void c2r_reg_block(const RepDev& r, int blk, float2* 
         const bool two = lb < NL;
         const bool xa = D == 3 ? la % 3 == 0 : true, xb = D == 3 && lb % 3 == 0;   // x derivatives (2D: every even line)
         const uint32_t o = (uint32_t)la * line + (uint32_t)(row0 + rr0) * (uint32_t)NXH;
+        const float fi = (float)i;
         float2 A[R1], B[R1];
 #pragma unroll
         for (int rr = 0; rr < R1; ++rr) {
-            const int kn = i + R2 * rr;
-            const uint32_t kk = (uint32_t)(kn >= NXH ? N - kn : kn);
+            const uint32_t kk = (uint32_t)half_entry<R2, N>(i, fi, rr).kk;
             A[rr] = gld(at32((const float2*)r.Gk, o + kk));
-            B[rr] = two ? gld(at32((const float2*)r.Gk, o + line + kk)) : make_float2(0.f, 0.f);
+            B[rr] = gld(at32((const float2*)r.Gk, o + (two ? line : 0u) + kk));
         }
         float2 v[R1];
 #pragma unroll
         for (int rr = 0; rr < R1; ++rr) {
-            const int kn = i + R2 * rr;
-            const bool upper = kn >= NXH;
-            const int kk = upper ? N - kn : kn;
-            const bool self = kk == 0 || 2 * kk == N;             // self-conjugate column
-            const float kx = self && kk != 0 ? 0.f : kf * (float)kk;
-            float2 a = A[rr], c = B[rr];
-            if (xa) a = x_gradient(kx, a);
-            if (xb) c = x_gradient(kx, c);
-            if (self) { a.y = 0.f; c.y = 0.f; }
+            const HalfEntry e = half_entry<R2, N>(i, fi, rr);
+            const float kx = kf * e.k;
+            float2 a = A[rr], c = two ? B[rr] : make_float2(0.f, 0.f);
+            a = pick(xa, x_gradient(kx, a), a);
+            c = pick(xb, x_gradient(kx, c), c);
+            if (e.self) { a.y = 0.f; c.y = 0.f; }
             // conj(Z) is transformed (the inverse as conj(FFT(conj))); products round before
             // they are added, as in the staged form, except where that form fuses them: the
             // lower half's real part with two fields in 2D
             const float re = fuse ? __builtin_fmaf(kx, A[rr].y, -c.y) : a.x - c.y;
-            v[rr] = upper ? make_float2(a.x + c.y, a.y - c.x) : make_float2(re, -(a.y + c.x));
+            v[rr] = e.upper ? make_float2(a.x + c.y, a.y - c.x) : make_float2(re, -(a.y + c.x));
         }
         plan_first<P>(v, r.reg_tw[0]);
 #pragma unroll
@@ -881,9 +876,18 @@ bool plane_inv_plan(const AxisPlan& px, const AxisPlan& py) {
     return (py.N / 2 + 1) * rmax <= kPlaneInvThreads && plane_inv_lds_bytes(py) <= kPlaneLds / 2;
 }
 
-bool plane_all_plan(const AxisPlan& px, const AxisPlan& py, int nf) {
-    const RegDims d = reg_dims(py);
-    return px.N == py.N && d.key && d.R1 <= 16 && !reg_plan_kept(py.N) && nf <= 2 && plane_all_threads(py.N, nf) > 0;
+// Pairs of lines to a block: as many as leave a task of the largest phase to every thread,
+// spread evenly over the plane's blocks.
+int plane_pairs(const AxisPlan& px, const AxisPlan& py, int nf) {
+    const RegDims x = reg_dims(px), y = reg_dims(py);
+    if (!x.key || !y.key || x.R1 > 16 || y.R1 > 16 || x.R2 > 16 || y.R2 > 16) return 0;
+    const int np = (3 * nf + 1) / 2, nxh = px.N / 2 + 1;
+    const int tasks = std::max(2 * nxh * std::max(y.R1, y.R2), py.N * std::max(x.R1, x.R2));
+    int g = std::max(1, std::min(np, kPlaneInvThreads / tasks));
+    const int nb = (np + g - 1) / g;
+    g = (np + nb - 1) / nb;
+    return g * py.N * x.R2 <= plane_pair_hold(x.R1) * kPlaneInvThreads && plane_pair_lds_bytes(px.N, py.N, g) <= kPlaneLds / 2
+               ? g : 0;
 }
 
 hipError_t launch_plane_inv(const LaunchCtx& c) {
@@ -892,23 +896,12 @@ hipError_t launch_plane_inv(const LaunchCtx& c) {
     return hipGetLastError();
 }
 
-hipError_t launch_plane_all(const LaunchCtx& c, bool wide) {
-    if (!c.n) return hipSuccess;
-    if (wide) TILD_LAUNCH(c, k_plane_all<kPlaneInvWide>, dim3(c.n), dim3(kPlaneInvWide), c.lds, c.reps, c.wmap);
-    else TILD_LAUNCH(c, k_plane_all<kPlaneInvThreads>, dim3(c.n), dim3(kPlaneInvThreads), c.lds, c.reps, c.wmap);
-    return hipGetLastError();
-}
-
 static hipError_t allow_lds(const void* kernel, size_t bytes) {
     return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
 hipError_t configure_plane_inv() {
-    for (hipError_t e : {allow_lds((const void*)k_plane_inv<kPlaneInvThreads>, kPlaneLds / 2),
-                         allow_lds((const void*)k_plane_all<kPlaneInvThreads>, kPlaneLds / 2),
-                         allow_lds((const void*)k_plane_all<kPlaneInvWide>, kPlaneLds)})
-        if (e != hipSuccess) return e;
-    return hipSuccess;
+    return allow_lds((const void*)k_plane_inv<kPlaneInvThreads>, kPlaneLds / 2);
 }
 
 // the kept square plans
@@ -916,21 +909,27 @@ bool plane_reg_plan(const AxisPlan& px, const AxisPlan& py) {
     return px.N == py.N && reg_dims(px).key && reg_plan_kept(px.N);
 }
 
-hipError_t launch_plane_reg(const LaunchCtx& c) {
-    if (!c.n) return hipSuccess;
-    TILD_LAUNCH(c, k_plane_reg<kPlaneRegThreads>, dim3(c.n), dim3(kPlaneRegThreads), c.lds, c.reps, c.wmap);
-    return hipGetLastError();
+bool plane_rect_plan(const AxisPlan& px, const AxisPlan& py) {
+    const RegDims x = reg_dims(px), y = reg_dims(py);
+    return x.key && y.key && std::max(std::max(x.R1, x.R2), std::max(y.R1, y.R2)) <= 16 &&
+           plane_rect_lds_bytes(px.N, py.N) <= kPlaneLds;
 }
 
-hipError_t launch_plane_rect(const LaunchCtx& c) {
+bool yfwd_reg_plan(const AxisPlan& pl) {
+    const RegDims d = reg_dims(pl);
+    return d.key && d.R1 <= 16 && d.R2 <= 16 && yfwd_reg_lds_bytes(pl) <= kPlaneLds;
+}
+
+hipError_t launch_plane_reg(const LaunchCtx& c) {
     if (!c.n) return hipSuccess;
-    TILD_LAUNCH(c, k_plane_rect<kPlaneRegThreads>, dim3(c.n), dim3(kPlaneRegThreads), c.lds, c.reps, c.wmap);
+    if (c.anyrec) TILD_LAUNCH(c, (k_plane_reg<kPlaneRegThreads, true>), dim3(c.n), dim3(kPlaneRegThreads), c.lds, c.reps, c.wmap);
+    else TILD_LAUNCH(c, (k_plane_reg<kPlaneRegThreads, false>), dim3(c.n), dim3(kPlaneRegThreads), c.lds, c.reps, c.wmap);
     return hipGetLastError();
 }
 
 hipError_t configure_plane_reg() {
-    const hipError_t e = allow_lds((const void*)k_plane_reg<kPlaneRegThreads>, kPlaneLds);
-    return e != hipSuccess ? e : allow_lds((const void*)k_plane_rect<kPlaneRegThreads>, kPlaneLds);
+    const hipError_t e = allow_lds((const void*)k_plane_reg<kPlaneRegThreads, false>, kPlaneLds);
+    return e != hipSuccess ? e : allow_lds((const void*)k_plane_reg<kPlaneRegThreads, true>, kPlaneLds);
 }
 
 bool grad_reg_plan(const AxisPlan& pl) {
@@ -941,12 +940,6 @@ bool grad_reg_plan(const AxisPlan& pl) {
 hipError_t launch_grad_reg(const LaunchCtx& c) {
     if (!c.n) return hipSuccess;
     TILD_LAUNCH(c, k_grad_reg<kGradRegThreads>, dim3(c.n), dim3(kGradRegThreads), c.lds, c.reps, c.wmap);
-    return hipGetLastError();
-}
-
-hipError_t launch_yfwd_reg(const LaunchCtx& c) {
-    if (!c.n) return hipSuccess;
-    TILD_LAUNCH(c, k_yfwd_reg<kGradRegThreads>, dim3(c.n), dim3(kGradRegThreads), c.lds, c.reps, c.wmap);
     return hipGetLastError();
 }
 

@@ -134,6 +134,40 @@ __device__ __forceinline__ void plan_second_lds(float2* w, const float2* TW, int
     plan_second<P, FUSED>(w, [&](int m) { return TW[tw2_index<P>(i, m)]; });
 }
 
+// Frequency of n = i + S r, i < S (fi = (float)i), on an axis of N points, 0 at N/2.  Which
+// side of N/2 the S values of one r lie on is known when the loop over r is unrolled, but
+// for the r that holds N/2: spelled out, since i's bound is not visible to the compiler and
+// the selects, conversions and address terms of every element were most of a short phase.
+template <int S, int N>
+__device__ __forceinline__ float freq_of(int i, float fi, int r) {
+    const int lo = S * r, hi = lo + S - 1;
+    if (2 * hi < N) return fi + (float)lo;
+    if (2 * lo > N) return fi + (float)(lo - N);
+    const int n2 = 2 * (i + lo);
+    const float f = 2 * lo == N || n2 > N ? fi + (float)(lo - N) : fi + (float)lo;
+    return N % 2 == 0 && n2 == N ? 0.f : f;
+}
+// The same n as an entry of a half spectrum: column kk = n, or N - n with the conjugate
+// (upper; N/2 as either), self: its own conjugate, k: the frequency kk, 0 at N/2.
+struct HalfEntry {
+    bool upper, self;
+    int kk;
+    float k;
+};
+template <int S, int N>
+__device__ __forceinline__ HalfEntry half_entry(int i, float fi, int r) {
+    const int lo = S * r, hi = lo + S - 1;
+    const bool mid = 2 * lo <= N && N <= 2 * hi;   // N/2 is among the S values
+    const bool nyq = N % 2 == 0 && mid && 2 * (i + lo) == N;
+    HalfEntry e;
+    e.upper = 2 * hi <= N ? false : (2 * lo >= N ? true : 2 * (i + lo) > N);
+    e.kk = e.upper ? (N - lo) - i : i + lo;
+    e.k = e.upper ? (float)(N - lo) - fi : fi + (float)lo;
+    if (nyq) e.k = 0.f;
+    e.self = (r == 0 && i == 0) || nyq;
+    return e;
+}
+
 // Products that the LDS-staged passes write to LDS before a later stage adds them: kept
 // out of FMA contraction with those additions, as they are there.
 __device__ __forceinline__ float2 scaled(float s, float2 a) {
@@ -147,6 +181,12 @@ __device__ __forceinline__ float2 grad_line(float k, float2 a) {
 __device__ __forceinline__ float2 x_gradient(float kx, float2 a) {   // -i k_x a
 #pragma clang fp contract(off)
     return make_float2(kx * a.y, -kx * a.x);
+}
+// on ? a : b, with both computed: a select, where the compiler branches around the products
+// of every element and waits for its loads one by one
+__device__ __forceinline__ float2 pick(bool on, float2 a, float2 b) {
+    settle<1>(&a);
+    return make_float2(on ? a.x : b.x, on ? a.y : b.y);
 }
 __device__ __forceinline__ float half_of(float a) {
 #pragma clang fp contract(off)

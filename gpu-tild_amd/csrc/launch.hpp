@@ -158,8 +158,7 @@ hipError_t configure_last_reg_1();
 hipError_t configure_last_reg_2();
 // The y inverse of the gradient spectra with register-resident columns (3D, y plans as
 // above with R1 <= 16): blocks of kGradRegThreads threads, grad_reg_lines(plan) columns
-// each, grad_reg_chunks per (field, z) plane.  The forward y pass of the half spectra
-// (k_yfwd_reg) has the same blocks.
+// each, grad_reg_chunks per (field, z) plane.
 constexpr int kGradRegThreads = 128;
 bool grad_reg_plan(const AxisPlan& pl);
 inline int grad_reg_lines(const AxisPlan& pl) {
@@ -170,14 +169,10 @@ inline int grad_reg_chunks(const AxisPlan& pl, int Nxh) { return (Nxh + grad_reg
 inline size_t grad_reg_lds_bytes(const AxisPlan& pl) {
     return ((size_t)pl.N * (3 * (size_t)grad_reg_lines(pl) + 1) + (size_t)pl.N) * sizeof(float2);
 }
-inline size_t yfwd_reg_lds_bytes(const AxisPlan& pl) {
-    return ((size_t)pl.N * ((size_t)grad_reg_lines(pl) + 1) + (size_t)pl.N) * sizeof(float2);
-}
 hipError_t launch_grad_reg(const LaunchCtx& c);
-hipError_t launch_yfwd_reg(const LaunchCtx& c);
-// The forward plane pass with register-resident columns: one block of kPlaneRegThreads
-// threads per (field, z) plane.  k_plane_reg: square planes of the kept two-stage plans;
-// k_plane_rect: any other plane of compiled plans.
+// The forward plane pass with register-resident columns: blocks of kPlaneRegThreads
+// threads.  plane_reg: a (field, z) plane of the kept two-stage plans, square; plane_rect:
+// any other of compiled plans; yfwd: columns of planes whose deposit transforms x.
 constexpr int kPlaneRegThreads = 512;
 bool plane_reg_plan(const AxisPlan& px, const AxisPlan& py);
 inline size_t plane_reg_lds_bytes(const AxisPlan& pl) {
@@ -189,34 +184,43 @@ inline size_t plane_rect_lds_bytes(int Nx, int Ny) {
     return ((a > b ? a : b) + a + (size_t)Nx + (size_t)Ny) * sizeof(float2);
 }
 hipError_t launch_plane_reg(const LaunchCtx& c);
-hipError_t launch_plane_rect(const LaunchCtx& c);
+bool plane_rect_plan(const AxisPlan& px, const AxisPlan& py);
+// yfwd: pieces of kYfwdThreads threads, their exchange and twiddles side by side
+constexpr int kYfwdThreads = 128, kYfwdPieces = kPlaneRegThreads / kYfwdThreads;
+inline int yfwd_reg_lines(const AxisPlan& pl) {
+    const RegDims d = reg_dims(pl);
+    return kYfwdThreads / (d.R1 > d.R2 ? d.R1 : d.R2);
+}
+inline int yfwd_reg_blocks(const AxisPlan& pl, int Nxh, int planes) {
+    const int nl = yfwd_reg_lines(pl);
+    return (planes * ((Nxh + nl - 1) / nl) + kYfwdPieces - 1) / kYfwdPieces;
+}
+inline size_t yfwd_reg_lds_bytes(const AxisPlan& pl) {
+    return (size_t)kYfwdPieces * (size_t)pl.N * (size_t)(yfwd_reg_lines(pl) + 2) * sizeof(float2);
+}
+bool yfwd_reg_plan(const AxisPlan& pl);
 hipError_t configure_plane_reg();
 // Register-resident inverse plane pass (y inverse + x C2R into the gather records) of
 // square planes with a kept two-stage plan: one block of kPlaneInvThreads threads per
 // (field, z) plane, two blocks to a CU.
-constexpr int kPlaneInvThreads = 512, kPlaneInvWide = 1024;
+constexpr int kPlaneInvThreads = 512;
 inline size_t plane_inv_lds_bytes(const AxisPlan& pl) {
     const size_t N = (size_t)pl.N, la = (size_t)((3 * (pl.N / 2 + 1)) | 1);
     return (N * la + (size_t)pl.rad[0] * (pl.rad[1] - 1)) * sizeof(float2);
 }
 bool plane_inv_plan(const AxisPlan& px, const AxisPlan& py);
-// The same for the other plans, all (one or two) fields of a z plane in one block, its x
-// lines paired across them as the separate x pass pairs them; kPlaneInvWide threads where
-// the LDS leaves one block to a CU.
-// the larger of the y inverses (rows of three half spectra per field) and the x exchange
-__host__ __device__ constexpr int plane_all_elems(int N, int nf) {
-    return N * (nf * ((3 * (N / 2 + 1)) | 1) > ((N * ((3 * nf + 1) / 2)) | 1) ? nf * ((3 * (N / 2 + 1)) | 1)
-                                                                             : ((N * ((3 * nf + 1) / 2)) | 1));
+// The same for any other plane of compiled plans with R1, R2 <= 16, in the same kernel: one
+// block per z plane and plane_pairs pairs of the x pass' lines, two blocks to a CU.  A thread
+// holds plane_pair_hold(R1) first groups, 24 values, at once.
+__host__ __device__ constexpr int plane_pair_hold(int R1) { return R1 > 24 ? 1 : 24 / R1; }
+__host__ __device__ constexpr int plane_pair_elems(int Nx, int Ny, int g) {   // the rows' half spectra, or the x exchange
+    return Ny * ((2 * g * (Nx / 2 + 1)) | 1) > Nx * ((Ny * g) | 1) ? Ny * ((2 * g * (Nx / 2 + 1)) | 1) : Nx * ((Ny * g) | 1);
 }
-__host__ __device__ constexpr size_t plane_all_lds(int N, int nf) {
-    return ((size_t)plane_all_elems(N, nf) + N) * sizeof(float2);
+inline size_t plane_pair_lds_bytes(int Nx, int Ny, int g) {
+    return (size_t)(plane_pair_elems(Nx, Ny, g) + Nx + Ny) * sizeof(float2);
 }
-__host__ __device__ constexpr int plane_all_threads(int N, int nf) {
-    return plane_all_lds(N, nf) <= kPlaneLds / 2 ? kPlaneInvThreads : (plane_all_lds(N, nf) <= kPlaneLds ? kPlaneInvWide : 0);
-}
-bool plane_all_plan(const AxisPlan& px, const AxisPlan& py, int nf);
+int plane_pairs(const AxisPlan& px, const AxisPlan& py, int nf);   // 0: no such pass
 hipError_t launch_plane_inv(const LaunchCtx& c);
-hipError_t launch_plane_all(const LaunchCtx& c, bool wide);
 hipError_t configure_plane_inv();
 hipError_t configure_last_reg();
 hipError_t launch_plane_r2c(const LaunchCtx& c);
