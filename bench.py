@@ -75,9 +75,9 @@ def phase_bytes(ns, D, M, Mh, nf, T, gjf, charged, ncoef, reorder_every, plane_i
 
 # the kernel of each profiled phase on the default (tiled, forward-plane) path, as named
 # in the rocprofv3 summaries
-PHASE_KERNEL = {"claim": "k_tile_claim", "deposit": "k_tile_deposit<512>", "plane_r2c": "k_plane_reg<512>",
-                "last_fused": "k_last_reg<256, 0>", "y_ifft": "k_grad_reg<128>", "x_c2r": "k_x_c2r<true, 256>",
-                "particles": "k_particles<true, true>",
+PHASE_KERNEL = {"claim": "k_tile_claim", "deposit": "k_tile_deposit<512, false, false>", "plane_r2c": "k_plane_reg<512, false>",
+                "last_fused": "k_last_reg<256, 2>", "y_ifft": "k_grad_reg<128>", "x_c2r": "k_x_c2r<true, 256>",
+                "particles": "k_particles<true, true, false>",
                 "advance": "k_advance", "reorder": None}
 # with the inverse plane pass (square x-y planes)
 PHASE_KERNEL_PLANE_INV = dict(PHASE_KERNEL, y_ifft=None, x_c2r="k_plane_inv<512>")

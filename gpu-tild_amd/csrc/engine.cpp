@@ -515,8 +515,9 @@ int Batch::add_plain(const System& S, uint32_t seed, std::string& err) {
                   plane_reg_lds_bytes(h.ax[0]) <= kPlaneLds ? 1 : 0;
     h.plane_rect = h.plane_fwd && !h.plane_reg && !tune_.staged && h.grid_off32 && plane_rect_plan(h.ax[0], h.ax[1]) ? 1 : 0;
     h.yfwd_reg = D == 3 && !h.plane_fwd && !tune_.staged && h.grid_off32 && yfwd_reg_plan(h.ax[1]) ? 1 : 0;
-    // the y inverse and the x C2R as one pass per (field, z) plane: square planes with an
-    // even two-stage plan, no field phases (whose records need the densities)
+    // the y inverse and the x C2R as one pass per (field, z) plane: square planes of the
+    // kept plans, or per z plane and pairs of lines: other compiled plans; no field phases
+    // (whose records need the densities)
     h.plane_inv = D == 3 && !tune_.staged && h.grid_off32 && !h.FPtab && plane_inv_plan(h.ax[0], h.ax[1]) &&
                   h.ax[0].rad[0] == h.ax[1].rad[0] && h.ax[0].rad[1] == h.ax[1].rad[1] ? 1 : 0;
     h.plane_pair = D == 3 && !tune_.staged && h.grid_off32 && !h.FPtab && !h.plane_inv ? plane_pairs(h.ax[0], h.ax[1], h.nf) : 0;
@@ -704,6 +705,9 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         if (h.spread_mode == 2) {
             add(PH_TCOUNT, (h.ns + kCountBlock - 1) / kCountBlock, 0);
             add(PH_SCAN, 1, 0);
+            // deposits that transform x apart: their registers (128 against 52) and LDS
+            // would bound the others' blocks per CU (sweep of 24 replicas, 10 of them of odd
+            // sides: 23.7 us a step in one launch, 21.7 in two)
             const Phase dep = h.plane_fwd ? PH_TILE : PH_TILEX;
             add(dep, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd, h.reg_key[0] && h.grid_off32));
             maps[dep].anyrec = maps[dep].anyrec || !h.srec;

@@ -30,7 +30,9 @@ constexpr int kProfPhases = 9;   // claim, deposit, forward plane, last_fused, y
 // of stored spectra for properties (every replica: it is the last axis in 2D).
 // PLANE: y-inverse + x C2R of 3D replicas whose planes fit one block's LDS (they
 // skip MIDY_G and C2R); PLANEF: x R2C + y FFT of tiled 3D replicas with even Ny
-// (their deposit writes densities only and they skip MIDY_H).
+// (their deposit writes densities only and they skip MIDY_H; PLANER: its register forms and
+// the forward y pass of the others); PLANEI: inverse plane pass; TILE, TILEX: deposits
+// without and with the x transform; LASTR, LASTR4, LASTRW: classes of the fused z pass.
 enum Phase { PH_PART = 0, PH_SPREADA, PH_XA, PH_XP, PH_SCAN, PH_TILE, PH_MIDY_H, PH_MIDY_G,
              PH_MIDZ_H, PH_PY, PH_LAST, PH_C2R, PH_PLANEF, PH_TCOUNT, PH_KPROPS, PH_RTILE, PH_LASTR, PH_MIDY_GR, PH_PLANER, PH_LASTR4, PH_LASTRW, PH_PLANEI, PH_C2RR, PH_TILEX, PH_COUNT };
 

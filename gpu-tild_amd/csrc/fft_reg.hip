@@ -1,12 +1,11 @@
 // fft_reg.hip -- FFT passes of the step with register-resident columns (CDNA4 / gfx950):
 // the forward plane pass (k_plane_reg), the y inverse of the gradient spectra
-// (k_grad_reg) and the inverse plane pass (k_plane_inv); the fused last-axis pass is in
-// fft_last.hpp.  Each takes the axes whose Stockham plan has two stages R1 x R2
-// (R1 >= R2, TILD_REG_PLANS); a thread keeps its columns in registers between the stages,
-// so a pass makes one to three LDS exchanges where the LDS-staged forms (kernels.hip)
-// stage every value through LDS with a barrier after each phase.  (An inverse x transform
-// of its own into the gather records stays LDS-staged: its register forms measured
-// slower.)
+// (k_grad_reg), the inverse plane pass (k_plane_inv) and the inverse x transform into the
+// gather records (k_c2r_reg); the fused last-axis pass is in fft_last.hpp, the x transform
+// of the deposit in spread_tiled.hip.  Each takes axes with a plan of TILD_REG_PLANS, two
+// groups of one or two Stockham stages; a thread keeps its columns in registers through a
+// group, so a pass makes one to three LDS exchanges where the LDS-staged forms
+// (kernels.hip) stage every value through LDS with a barrier after each phase.
 #include "device.hpp"
 #include "fft_dev.hpp"
 #include "fft_reg_dev.hpp"
@@ -29,13 +28,13 @@ RegDims reg_dims(const AxisPlan& pl) {
 
 // ------------------------------------------------------------------ y inverse (3D)
 // The y-axis inverse of the gradient spectra (the operation of k_mid_grad, kernels.hip)
-// for two-stage y plans R1 x R2, columns in registers between the stages: per (field,
-// z) plane and NB = NT / R1 adjacent x columns,
+// for y plans of groups R1 x R2, columns in registers between the groups: per (field,
+// z) plane and NB = NT / max(R1, R2) adjacent x columns,
 //   A  thread (b, i), i < R2: rows i + R2 r of U (slot 0) and V (slot 2), the three
-//      lines conj(U), conj(-i k_y U), conj(V), DFT_R1; exchange;
-//   B  thread (b, i), i < R1: twiddles w_Ny^{i r}, DFT_R2 -> rows i + R1 q of the three
-//      outputs (slots 0, 1, 2).
-// One barrier.  A block reads its columns of slots 0 and 2 before it writes any slot,
+//      lines conj(U), conj(-i k_y U), conj(V), first group; exchange;
+//   B  thread (b, i), i < R1: second group -> rows i + R1 q of the three outputs (slots
+//      0, 1, 2).
+// One barrier; bound by its loads and stores (18.4 us LDS-staged, 9.4 here on 96^3).  A block reads its columns of slots 0 and 2 before it writes any slot,
 // and no other block touches them.
 namespace {
 template <class P, int NT>
@@ -355,7 +354,9 @@ __device__ __forceinline__ void yfwd_piece(const RepDev& r, int piece, bool live
 }  // namespace
 
 // ANY: some replica of the set takes one of the two other forms; without them the kernel
-// holds the kept squares only, and its registers (74 against 128).
+// holds the kept squares only, and its registers (74 against 89, three blocks to a CU
+// against two).  One launch for the forms: the sweep of 24 replicas spends 11.7 us a step
+// here, and 19.3 with a launch for each.
 template <int NT, bool ANY>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) k_plane_reg(const RepDev* __restrict__ reps,
                                                                                         const WorkItem* __restrict__ wmap) {
@@ -402,7 +403,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) k_
 // The y inverse of the gradient spectra and the x C2R into gather records of one
 // (field, z) plane in one block (the operations of k_grad_reg and k_x_c2r, kernels.hip,
 // without the half spectra of the y inverses going through HBM), for square planes
-// Nx = Ny = N with a two-stage plan R1 x R2 (an odd N pairs its last row's z derivative
+// Nx = Ny = N with a kept two-stage plan R1 x R2 (an odd N pairs its last row's z derivative
 // with an all-zero line):
 //   A  task (column k < N/2 + 1, i < R2): rows i + R2 r of U and V (slots 0 and 2),
 //      the lines conj(U), conj(-i k_y U), conj(V), DFT_R1;
@@ -579,6 +580,8 @@ __device__ __forceinline__ void plane_inv_block(const RepDev& r, int blk, float2
 // a z plane (more where that leaves threads idle, plane_pairs): their y inverses over the
 // plane's columns, the paired x transform of its rows, and their components of the records.
 // One pair of 96 x 96 points fits half a CU's LDS where a field's three lines do not.
+// Bound by instruction issue on few waves (96 x 96: 2,700 a wave, two waves per SIMD):
+// 96^3 22.8 us and 45 x 36 x 60 6.8 where the y inverse and the x pass took 26.8 and 9.2.
 namespace {
 template <class P, int NT>
 __device__ __forceinline__ void plane_pair_y(const RepDev& r, int z, int l0, int nl, int la, float2* X, const float2* TW) {
@@ -753,13 +756,14 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) k_
 
 // ------------------------------------------------------------------ x C2R
 // Inverse x transform of the half spectra into the gather records (the operation of
-// k_x_c2r, kernels.hip) for two-stage x plans, where the plane pass does not run (2D, and
-// planes of unequal sides); nr_c2r rows per block, nc complex lines per row:
+// k_x_c2r, kernels.hip) for compiled x plans, where no plane pass runs it (2D, and planes
+// above half a CU's LDS); nr_c2r rows per block, nc complex lines per row:
 //   A  task (line b, i < R2): Z = A + i B at k = i + R2 r of the full spectrum straight
-//      from the half spectra (the upper half by Hermitian symmetry), DFT_R1; exchange;
-//   B  task (b, i < R1): twiddles, DFT_R2 -> the real lines, over the values the task read;
+//      from the half spectra (the upper half by Hermitian symmetry), first group; exchange;
+//   B  task (b, i < R1): second group -> the real lines, over the values the task read;
 //   C  the records (g_x, g_y, g_z), stored in order.
-// Two barriers; the staged form has four and waits for its second stage's twiddles.  It
+// Two barriers; the staged form has four and waits for its second stage's twiddles (film
+// 64^2 5.6 -> 4.3 us, the latency of a launch of few blocks; 192^2 5.2 -> 4.8).  It
 // reads each half-spectrum value twice (the second time from cache), which is why grids of
 // many planes take the plane pass instead.
 namespace {
@@ -877,7 +881,9 @@ bool plane_inv_plan(const AxisPlan& px, const AxisPlan& py) {
 }
 
 // Pairs of lines to a block: as many as leave a task of the largest phase to every thread,
-// spread evenly over the plane's blocks.
+// spread evenly over the plane's blocks (a 21 x 21 x 225 slab with a pair to each of 675
+// blocks of 462 / 3 tasks 9.7 us, with three 6.1; 27^3 alike with one and two).  Groups
+// above 16 would spill the registers of two blocks to a CU.
 int plane_pairs(const AxisPlan& px, const AxisPlan& py, int nf) {
     const RegDims x = reg_dims(px), y = reg_dims(py);
     if (!x.key || !y.key || x.R1 > 16 || y.R1 > 16 || x.R2 > 16 || y.R2 > 16) return 0;

@@ -230,8 +230,8 @@ inline size_t plane_r2c_lds(const RepDev& h) {
     const size_t a = (size_t)h.Nx * (size_t)((h.Ny / 2) | 1), b = (size_t)h.Ny * (size_t)(h.Nxh | 1);
     return 2 * (a > b ? a : b) * sizeof(float2);
 }
-// x C2R into the gather records with register-resident columns (two-stage x plans, no
-// field phases): one exchange buffer and the second stage's twiddles.
+// x C2R into the gather records with register-resident columns (compiled x plans, no
+// field phases): one exchange buffer and the second group's twiddles.
 constexpr int kC2rRegThreads = 256;
 inline size_t c2r_reg_lds_bytes(int N, int nlines) { return fft_buf_bytes(N, nlines) + (size_t)N * sizeof(float2); }
 hipError_t launch_c2r_reg(const LaunchCtx& c);

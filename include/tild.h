@@ -111,14 +111,14 @@ typedef struct {
                             on it. */
     int deposit_threads; /* tiled spread: deposit block size, 256 or 512 (0 = by the
                             beads per tile).  Results do not depend on it. */
-    int fft_staged;      /* nonzero: the forward plane pass, the fused z pass and the y
-                            inverse stage every value through LDS even where their
-                            register-resident forms apply (two-stage plans 16x10, 10x8,
-                            8x8, 8x5 of the axis; the plane pass square planes, the z
-                            pass at most four types, two on a 160-point axis).  The forms agree to rounding (about 1e-7
-                            relative), not bit for bit: the compiler fuses multiplies into
-                            additions where one keeps in registers what the other stages
-                            through LDS. */
+    int fft_staged;      /* nonzero: every FFT pass of the step stages every value through
+                            LDS even where its register-resident form applies (36 axis
+                            lengths of 21 to 240 points; the z pass at most four types,
+                            two above 100 points).  On axes of 24, 25, 30, 32, 40, 48, 50,
+                            64, 80, 128 and 160 points the forms agree to rounding (about
+                            1e-7 relative), not bit for bit: the compiler fuses multiplies
+                            into additions where one keeps in registers what the other
+                            stages through LDS.  On other axes they are identical. */
 } tild_opts;
 
 /* Properties of calc_properties() (calc_properties.cu:20-116): FP64 reductions. */
