@@ -1423,7 +1423,9 @@ static void unpermute(const T* in, T* out, size_t n, const std::vector<int>& pid
 }
 int Batch::to_host(const Replica& R, const float* dev, float* host, std::string& err) {
     const size_t bytes = (size_t)R.ns * R.dim * sizeof(float);
+    std::unique_lock<std::mutex> spare(spare_mu_, std::defer_lock);
     if (R.permuted) {   // a permuted replica has reorder buffers
+        spare.lock();   // until the copy has left the buffer
         HIPCHK(launch_site_order(stream_, dev, R.h.pid, R.h.XO_alt, R.ns, R.dim, true));
         dev = R.h.XO_alt;
     }
@@ -1434,8 +1436,14 @@ int Batch::to_host(const Replica& R, const float* dev, float* host, std::string&
 
 int Batch::to_device(const Replica& R, const float* host, float* dev, std::string& err) {
     const size_t bytes = (size_t)R.ns * R.dim * sizeof(float);
-    HIPCHK(hipMemcpyAsync(R.permuted ? R.h.XO_alt : dev, host, bytes, hipMemcpyHostToDevice, stream_));
-    if (R.permuted) HIPCHK(launch_site_order(stream_, R.h.XO_alt, R.h.pid, dev, R.ns, R.dim, false));
+    if (!R.permuted) {
+        HIPCHK(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, stream_));
+        return 0;
+    }
+    // the buffer's next user is ordered after these two by the stream
+    std::lock_guard<std::mutex> spare(spare_mu_);
+    HIPCHK(hipMemcpyAsync(R.h.XO_alt, host, bytes, hipMemcpyHostToDevice, stream_));
+    HIPCHK(launch_site_order(stream_, R.h.XO_alt, R.h.pid, dev, R.ns, R.dim, false));
     return 0;
 }
 

@@ -9,6 +9,7 @@
 
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -231,7 +232,9 @@ private:
     int fetch_pid(const Replica& R, std::vector<int>& pid, std::string& err);
     // per-bead device array (dim floats) <-> host array in site order.  A permuted replica's
     // beads change order on the device, through the spare buffer of its spatial reorder
-    // (which only the next reorder writes, and the stream orders it after the copy).
+    // (which only the next reorder writes, and the stream orders it after the copy).  The
+    // buffer belongs to one copy at a time: threads that read one engine together wait here.
+    std::mutex spare_mu_;
     int to_host(const Replica& R, const float* dev, float* host, std::string& err);
     int to_device(const Replica& R, const float* host, float* dev, std::string& err);
     void free_maps(PhaseMap* maps);
