@@ -307,8 +307,10 @@ __device__ __forceinline__ void deposit_srec(const SrecTile& c, const float4 rec
 // Round to nearest of w 2^F (|w 2^F| < 2^51) as a 64-bit integer: adding 1.5 2^52 in FP64
 // leaves the integer in the low mantissa bits, ties to even, the same integer as
 // __float2ll_rn of the FP32 product (scaling by a power of two is exact) in a third of its
-// instructions.
+// instructions.  ANY: the conversion itself, for any w.
+template <bool ANY>
 __device__ __forceinline__ unsigned long long round_scaled(float w, double scale) {
+    if constexpr (ANY) return (unsigned long long)__float2ll_rn(w * (float)scale);
     const double magic = 6755399441055744.0;   // 1.5 2^52
     return (unsigned long long)(__double_as_longlong(__builtin_fma((double)w, scale, magic)) - __double_as_longlong(magic));
 }
@@ -318,20 +320,10 @@ __device__ __forceinline__ unsigned long long round_scaled(float w, double scale
 // and are skipped.  Unrolled: with run-time loops a record took 1,300 instructions and more,
 // a third of them in the rounding to 64-bit integers (order 3 on a 48^3 grid, 41,480 beads:
 // 34.7 us).
-template <int NP, int D>
-__device__ __forceinline__ void deposit_posrec(const RepDev& r, const float4 rec, float qi,
-                                               unsigned long long* patch, int y0, int z0, int By, int Bz) {
-    const int Nx = r.Nx, tp = __float_as_int(rec.w);
-    float W[3][5];
-    int n0[3] = {0, 0, 0};
-    W[2][0] = 1.f;
-    n0[0] = stencil_1d(rec.x, r.dx[0], r.idx[0], Nx, NP - 1, W[0]);
-    n0[1] = stencil_1d(rec.y, r.dx[1], r.idx[1], r.Ny, NP - 1, W[1]);
-    if constexpr (D == 3) n0[2] = stencil_1d(rec.z, r.dx[2], r.idx[2], r.Nz, NP - 1, W[2]);
-    // a position that is not a number has weights that are none and deposits nothing, as
-    // where such a weight is converted to an integer
-    const float wsum = W[0][NP - 1] + W[1][NP - 1] + W[2][0] + (rec.x + rec.y + rec.z);
-    if (wsum != wsum) return;
+template <int NP, int D, bool ANY>
+__device__ __forceinline__ void deposit_nodes(const RepDev& r, const float (&W)[3][5], const int (&n0)[3], int tp, float qi,
+                                              unsigned long long* patch, int y0, int z0, int By, int Bz) {
+    const int Nx = r.Nx;
     int xx[NP];
     xx[0] = n0[0];
 #pragma unroll
@@ -357,11 +349,32 @@ __device__ __forceinline__ void deposit_posrec(const RepDev& r, const float4 rec
             for (int ix = 0; ix < NP; ++ix) {
                 // Wx Wy Wz in the reference's product order (device_grid_utils.cu:329)
                 const float w = D == 3 ? W[0][ix] * W[1][iy] * W[2][iz] : W[0][ix] * W[1][iy];
-                atomicAdd(rowp + xx[ix], round_scaled(w, scale));
+                atomicAdd(rowp + xx[ix], round_scaled<ANY>(w, scale));
                 if (charged) atomicAdd(rowq + xx[ix], (unsigned long long)__float2ll_rn((w * qi) * r.fixq_scale));
             }
         }
     }
+}
+
+template <int NP, int D>
+__device__ __forceinline__ void deposit_posrec(const RepDev& r, const float4 rec, float qi,
+                                               unsigned long long* patch, int y0, int z0, int By, int Bz) {
+    const int tp = __float_as_int(rec.w);
+    float W[3][5];
+    int n0[3] = {0, 0, 0};
+    W[2][0] = 1.f;
+    n0[0] = stencil_1d(rec.x, r.dx[0], r.idx[0], r.Nx, NP - 1, W[0]);
+    n0[1] = stencil_1d(rec.y, r.dx[1], r.idx[1], r.Ny, NP - 1, W[1]);
+    if constexpr (D == 3) n0[2] = stencil_1d(rec.z, r.dx[2], r.idx[2], r.Nz, NP - 1, W[2]);
+    // A position's weights sum to 1 per axis.  Those of a coordinate that is not a number,
+    // infinite or beyond FP32's resolution of the grid can be anything: they take the plain
+    // conversion, as in the global-atomic spread (a sum of 4 bounds a product by 2.4, and
+    // round_scaled holds up to 2^51 2^-F >= 2^7).
+    float sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < NP; ++k) sum += fabsf(W[0][k]) + fabsf(W[1][k]) + (D == 3 ? fabsf(W[2][k]) : 0.f);
+    if (sum <= 4.f) deposit_nodes<NP, D, false>(r, W, n0, tp, qi, patch, y0, z0, By, Bz);
+    else deposit_nodes<NP, D, true>(r, W, n0, tp, qi, patch, y0, z0, By, Bz);
 }
 
 template <int D>

@@ -62,3 +62,29 @@ def test_mixed_orders_in_a_batch(tmp_path):
         assert np.array_equal(b.positions(ids[k]), e.positions()), k
         e.close()
     b.close()
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("order", [0, 2, 3, 4])
+def test_positions_without_a_place_deposit_alike(order, dim, tmp_path):
+    # a coordinate that is not a number, infinite, or so large that its FP32 offset from the
+    # node has no meaning still has a node (every index is wrapped) and weights, and both
+    # spreads round those to the same integers, as for any other bead
+    g = (20, 16, 24)[:dim]
+    mk = decks.melt3d if dim == 3 else decks.melt2d
+    text, d = mk(tmp_path, grid=g, box=tuple(0.5 * n for n in g), n_chains=150, pmeorder=order)
+    s = tild.System(text, d)
+    tiled, atomic = tild.Engine(s, device=0, seed=3, spread_mode=2), tild.Engine(s, device=0, seed=3, spread_mode=1)
+    for bad in (np.nan, np.inf, -np.inf, 1e9, -3e7):
+        for axis in range(dim):
+            x = s.positions()
+            x[5, axis] = bad
+            rho = []
+            for e in (tiled, atomic):
+                e.set_positions(x)
+                e.forces()
+                rho.append([e.density(t) for t in range(s.ntypes)])
+            for a, b in zip(*rho):
+                assert np.array_equal(a, b, equal_nan=True), (bad, axis)
+    tiled.close()
+    atomic.close()
