@@ -165,7 +165,7 @@ __device__ __forceinline__ void plane_reg_block(const RepDev& r, int blk, float2
 #pragma unroll
         for (int rr = 0; rr < R2; ++rr) v[rr] = Xa[(i + R1 * rr) * ldp + j];
 #pragma unroll
-        for (int rr = 1; rr < R2; ++rr) v[rr] = cmul(v[rr], TWx[i * (R2 - 1) + rr - 1]);
+        for (int rr = 1; rr < R2; ++rr) v[rr] = cmul_kept(v[rr], TWx[i * (R2 - 1) + rr - 1]);
         Dft<R2>::run(v);
 #pragma unroll
         for (int q = 0; q < R2; ++q) Xb[(i + R1 * q) * ldp + j] = v[q];
@@ -198,7 +198,7 @@ __device__ __forceinline__ void plane_reg_block(const RepDev& r, int blk, float2
 #pragma unroll
         for (int rr = 0; rr < R2; ++rr) v[rr] = Xa[(i + R1 * rr) * ldc + k];
 #pragma unroll
-        for (int rr = 1; rr < R2; ++rr) v[rr] = cmul(v[rr], TWy[i * (R2 - 1) + rr - 1]);
+        for (int rr = 1; rr < R2; ++rr) v[rr] = cmul_kept(v[rr], TWy[i * (R2 - 1) + rr - 1]);
         Dft<R2>::run(v);
 #pragma unroll
         for (int q = 0; q < R2; ++q) gst(at32(r.H, hbase + (uint32_t)((i + R1 * q) * NXH + k)), v[q]);

@@ -39,6 +39,13 @@ __device__ __forceinline__ float2 cmul_fused(float2 a, float2 b) {
     const float yy = a.y * b.y, yx = a.y * b.x;
     return make_float2(__builtin_fmaf(a.x, b.x, -yy), __builtin_fmaf(a.x, b.y, yx));
 }
+// ... those of the kept plans' forward plane pass, which is compiled into two kernels and
+// whose bits may not depend on which of them a set of replicas runs
+__device__ __forceinline__ float2 cmul_kept(float2 a, float2 b) {
+#pragma clang fp contract(off)
+    const float yy = a.y * b.y, xy = a.x * b.y;
+    return make_float2(__builtin_fmaf(a.x, b.x, -yy), __builtin_fmaf(a.y, b.x, xy));
+}
 template <bool FUSED> __device__ __forceinline__ float2 cmul_as(float2 a, float2 b) {
     if constexpr (FUSED) return cmul_fused(a, b);
     else return cmul(a, b);

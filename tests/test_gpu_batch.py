@@ -100,3 +100,22 @@ def test_batched_spatial_reorder_is_invisible(which, tmp_path):
         assert np.array_equal(xa, xb), (which, i)
         assert abs(pa["Upe"] - pb["Upe"]) <= 1e-12 * abs(pb["Upe"]), (which, i)
     print(f"[{which}] {len(systems)} replicas reordered every 3 steps: positions bit-identical to never reordering")
+
+
+def test_square_planes_keep_their_bits_in_a_mixed_set(tmp_path):
+    # with a rectangular or an odd-sided replica in the set, the forward plane pass is a
+    # kernel that holds every form; square planes run the same transform in it
+    grids = [(n, n, 10) for n in (24, 30, 32, 40, 48, 50, 64, 80, 128)] + [(36, 30, 10), (25, 27, 10)]
+    systems = []
+    for k, g in enumerate(grids):
+        t, d = decks.melt3d(tmp_path / str(k), grid=g, box=tuple(0.5 * n for n in g), n_chains=5 * g[0], delt=0.02)
+        systems.append(tild.System(t, d))
+    b = tild.Batch(device=0)
+    ids = [b.add(s, 20 + k) for k, s in enumerate(systems)]
+    b.step(8)
+    for k, s in enumerate(systems):
+        e = tild.Engine(s, device=0, seed=20 + k)
+        e.step(8)
+        assert np.array_equal(b.positions(ids[k]), e.positions()), grids[k]
+        e.close()
+    b.close()
