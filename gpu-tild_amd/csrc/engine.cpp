@@ -560,7 +560,7 @@ int Batch::tile_regions(int id, bool bin_only, std::string& err) {
     if (R.h.spread_mode != 2) return 0;
     if (int rc = unclaim(id, err)) return rc;
     PhaseMap* mp = R.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].anyrec}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].allforms}; };
     HIPCHK(launch_tile_count(ctx(PH_TCOUNT), 0));
     HIPCHK(launch_tile_scan(ctx(PH_SCAN)));
     if (!bin_only) HIPCHK(launch_tile_regions(stream_, d_reps_, id));
@@ -682,7 +682,7 @@ int Batch::upload_desc(int id, std::string& err) {
 
 // ---------------------------------------------------------------- work maps
 int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& err, bool reorder_only) {
-    for (int p = 0; p < PH_COUNT; ++p) { maps[p].host.clear(); maps[p].lds = 0; maps[p].n = 0; maps[p].xfft = false; maps[p].anyrec = false; }
+    for (int p = 0; p < PH_COUNT; ++p) { maps[p].host.clear(); maps[p].lds = 0; maps[p].n = 0; maps[p].xfft = false; maps[p].allforms = false; }
     for (int id : ids) {
         const Replica& R = *reps_[id];
         const RepDev& h = R.h;
@@ -692,7 +692,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
             maps[ph].lds = std::max(maps[ph].lds, lds);
         };
         add(PH_PART, R.nblk_part, 0);
-        maps[PH_PART].anyrec = maps[PH_PART].anyrec || h.P > 1;
+        maps[PH_PART].allforms = maps[PH_PART].allforms || h.P > 1;
         if (reorder_only) {   // the passes of reorder_set (tiled replicas)
             add(PH_TCOUNT, (h.ns + kCountBlock - 1) / kCountBlock, 0);
             add(PH_SCAN, 1, 0);
@@ -710,7 +710,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
             // sides: 23.7 us a step in one launch, 21.7 in two)
             const Phase dep = h.plane_fwd ? PH_TILE : PH_TILEX;
             add(dep, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd, h.reg_key[0] && h.grid_off32));
-            maps[dep].anyrec = maps[dep].anyrec || !h.srec;
+            maps[dep].allforms = maps[dep].allforms || !h.srec;
             maps[PH_TILEX].xfft = true;
             if (R.reorder_every > 0) add(PH_RTILE, h.ntiles, 0);
         } else {
@@ -720,7 +720,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         {
             MidGeom g = mid_geom(h, 1, h.nf);
             add(PH_PY, g.nouter * g.nchunk, lds_bytes(g.N, g.nl));
-            maps[PH_PLANER].anyrec = maps[PH_PLANER].anyrec || h.plane_rect || h.yfwd_reg;
+            maps[PH_PLANER].allforms = maps[PH_PLANER].allforms || h.plane_rect || h.yfwd_reg;
             if (D == 3 && h.plane_reg) add(PH_PLANER, h.nf * h.Nz, plane_reg_lds_bytes(h.ax[0]));
             else if (D == 3 && h.plane_rect) add(PH_PLANER, h.nf * h.Nz, plane_rect_lds_bytes(h.Nx, h.Ny));
             else if (D == 3 && h.yfwd_reg) add(PH_PLANER, yfwd_reg_blocks(h.ax[1], h.Nxh, h.nf * h.Nz), yfwd_reg_lds_bytes(h.ax[1]));
@@ -731,7 +731,10 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
             MidGeom g = mid_grad_geom(h);
             if (h.plane_inv) add(PH_PLANEI, h.nf * h.Nz, plane_inv_lds_bytes(h.ax[1]));
             else if (h.plane_pair) add(PH_PLANEI, h.Nz * ((3 * h.nf + 2 * h.plane_pair - 1) / (2 * h.plane_pair)), plane_pair_lds_bytes(h.Nx, h.Ny, h.plane_pair));
-            else if (h.grad_reg) add(PH_MIDY_GR, h.nf * h.Nz * grad_reg_chunks(h.ax[1], h.Nxh), grad_reg_lds_bytes(h.ax[1]));
+            else if (h.grad_reg) {
+                maps[PH_MIDY_GR].allforms = maps[PH_MIDY_GR].allforms || h.ax[1].nst > 2;
+                add(PH_MIDY_GR, h.nf * h.Nz * grad_reg_chunks(h.ax[1], h.Nxh), grad_reg_lds_bytes(h.ax[1]));
+            }
             else add(PH_MIDY_G, g.nouter * g.nchunk, lds_bytes(g.N, 3 * g.nl));
             MidGeom gz = mid_geom(h, 2, h.nf);
             add(PH_MIDZ_H, gz.nouter * gz.nchunk, lds_bytes(gz.N, gz.nl));
@@ -1090,7 +1093,7 @@ int Batch::build_tables(Replica& R, const System& S, std::string& err) {
 // device step counter plus k, and one launch at the end advances the counter.
 int Batch::enqueue_steps(SetMaps& m, int nsteps, bool integrate, bool write_forces, std::string& err) {
     PhaseMap* mp = m.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].anyrec}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].allforms}; };
     for (int k = 0; k < nsteps; ++k) {
         HIPCHK(launch_spread(ctx(PH_SPREADA), k));
         HIPCHK(launch_x_r2c(ctx(PH_XA), true, 0, nullptr, nullptr));
@@ -1230,7 +1233,7 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
     for (int s = 0; s < n && !rc; ++s) {
         bool used[kKernelPhases][kSlots] = {};
         auto ctx = [&](Phase p, int ph, int slot) {
-            LaunchCtx c{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].anyrec};
+            LaunchCtx c{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].allforms};
             if (c.n > 0) { c.t0 = ev[ph][slot][0]; c.t1 = ev[ph][slot][1]; used[ph][slot] = true; }
             return c;
         };
@@ -1307,7 +1310,7 @@ int Batch::profile(const std::vector<int>& ids, int n, double* ms, int nph, std:
 int Batch::forward_spectra(int id, std::string& err) {
     Replica& R = *reps_[id];
     PhaseMap* mp = R.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].anyrec}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].allforms}; };
     HIPCHK(launch_x_r2c(ctx(PH_XP), false, 0, nullptr, nullptr));
     HIPCHK(launch_mid(ctx(PH_PY), 1, 0, 0, 0, nullptr));
     if (R.dim == 3) HIPCHK(launch_mid(ctx(PH_MIDZ_H), 2, 0, 0, 0, nullptr));
@@ -1321,7 +1324,7 @@ int Batch::properties(int id, tild_props* out, std::string& err) {
     HIPCHK(hipSetDevice(device_));
     if (int rc = forward_spectra(id, err)) return rc;
     PhaseMap* mp = R.maps;
-    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].anyrec}; };
+    auto ctx = [&](Phase p) { return LaunchCtx{d_reps_, mp[p].dev, mp[p].n, mp[p].lds, stream_, nullptr, nullptr, mp[p].threads, mp[p].xfft, mp[p].allforms}; };
     HIPCHK(launch_kprops(ctx(PH_KPROPS), R.nq));
     HIPCHK(launch_reduce_rows(stream_, R.h.partials, R.nq, R.h.nchunk, R.d_results));
     HIPCHK(launch_bond_props(ctx(PH_PART)));

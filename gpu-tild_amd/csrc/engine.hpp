@@ -44,7 +44,7 @@ struct PhaseMap {
     int n = 0;
     int threads = 0;   // block size where a pass has more than one (0: its default)
     bool xfft = true;  // tiled deposit: some replica of the set transforms along x in it
-    bool anyrec = true;   // ... deposits position records; particles: some replica's order is above 1
+    bool allforms = true;   // some replica of the set needs the instantiation of every form (LaunchCtx)
     int cap = 0;       // work items the device buffer holds
 };
 

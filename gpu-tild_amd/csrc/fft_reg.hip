@@ -90,7 +90,7 @@ __device__ __forceinline__ void grad_reg_block(const RepDev& r, int blk, float2*
             float2 w[R2];
 #pragma unroll
             for (int rr = 0; rr < R2; ++rr) w[rr] = X1[(i + R1 * rr) * ld + l * NB + b];
-            plan_second<P, !P::KEPT>(w, [&](int m) { return t[m]; });
+            plan_second<P, true>(w, [&](int m) { return t[m]; });
             const uint32_t s0 = l == 0 ? sU : (l == 1 ? sY : sV);
 #pragma unroll
             for (int q = 0; q < R2; ++q)
@@ -101,7 +101,10 @@ __device__ __forceinline__ void grad_reg_block(const RepDev& r, int blk, float2*
 
 }  // namespace
 
-template <int NT>
+// ALL: some replica of the set has a grouped y plan; without them 121 registers and four waves
+// per SIMD, with them 210 and two (y of 80 points, 160 x 80 x 80: 9.6 us, and 11.5 in the
+// kernel of all plans; 128^3: 21 and 24).
+template <int NT, bool ALL>
 __global__ void __launch_bounds__(NT) k_grad_reg(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap) {
     extern __shared__ float2 lds[];
     const WorkItem wi = wmap[blockIdx.x];
@@ -110,7 +113,8 @@ __global__ void __launch_bounds__(NT) k_grad_reg(const RepDev* __restrict__ reps
     switch (r.reg_key[1]) {   // uniform per block
 #define TILD_CASE(A0, A1, B0, B1)          \
     case reg_plan_key(A0, A1, B0, B1):     \
-        if constexpr ((A0) * (A1) <= 16) grad_reg_block<RegPlan<A0, A1, B0, B1>, NT>(r, wi.blk, lds); \
+        if constexpr ((A0) * (A1) <= 16 && (ALL || !reg_plan_grouped(A1, B1)))     \
+            grad_reg_block<RegPlan<A0, A1, B0, B1>, NT>(r, wi.blk, lds);           \
         break;
         TILD_REG_PLANS(TILD_CASE)
 #undef TILD_CASE
@@ -928,7 +932,7 @@ bool yfwd_reg_plan(const AxisPlan& pl) {
 
 hipError_t launch_plane_reg(const LaunchCtx& c) {
     if (!c.n) return hipSuccess;
-    if (c.anyrec) TILD_LAUNCH(c, (k_plane_reg<kPlaneRegThreads, true>), dim3(c.n), dim3(kPlaneRegThreads), c.lds, c.reps, c.wmap);
+    if (c.allforms) TILD_LAUNCH(c, (k_plane_reg<kPlaneRegThreads, true>), dim3(c.n), dim3(kPlaneRegThreads), c.lds, c.reps, c.wmap);
     else TILD_LAUNCH(c, (k_plane_reg<kPlaneRegThreads, false>), dim3(c.n), dim3(kPlaneRegThreads), c.lds, c.reps, c.wmap);
     return hipGetLastError();
 }
@@ -945,7 +949,8 @@ bool grad_reg_plan(const AxisPlan& pl) {
 
 hipError_t launch_grad_reg(const LaunchCtx& c) {
     if (!c.n) return hipSuccess;
-    TILD_LAUNCH(c, k_grad_reg<kGradRegThreads>, dim3(c.n), dim3(kGradRegThreads), c.lds, c.reps, c.wmap);
+    if (c.allforms) TILD_LAUNCH(c, (k_grad_reg<kGradRegThreads, true>), dim3(c.n), dim3(kGradRegThreads), c.lds, c.reps, c.wmap);
+    else TILD_LAUNCH(c, (k_grad_reg<kGradRegThreads, false>), dim3(c.n), dim3(kGradRegThreads), c.lds, c.reps, c.wmap);
     return hipGetLastError();
 }
 

@@ -1243,13 +1243,13 @@ static void particles_launch(const LaunchCtx& c, int write_forces, int koff) {
 hipError_t launch_particles(const LaunchCtx& c, bool integrate, int write_forces, int koff, bool claim) {
     if (!c.n) return hipSuccess;
     if (integrate && claim) {
-        if (c.anyrec) particles_launch<true, true, true>(c, write_forces, koff);
+        if (c.allforms) particles_launch<true, true, true>(c, write_forces, koff);
         else particles_launch<true, true, false>(c, write_forces, koff);
     } else if (integrate) {
-        if (c.anyrec) particles_launch<true, false, true>(c, write_forces, koff);
+        if (c.allforms) particles_launch<true, false, true>(c, write_forces, koff);
         else particles_launch<true, false, false>(c, write_forces, koff);
     } else {
-        if (c.anyrec) particles_launch<false, false, true>(c, write_forces, koff);
+        if (c.allforms) particles_launch<false, false, true>(c, write_forces, koff);
         else particles_launch<false, false, false>(c, write_forces, koff);
     }
     CHECK_LAUNCH(); return hipSuccess;

@@ -66,7 +66,10 @@ struct LaunchCtx {
     hipEvent_t t0 = nullptr, t1 = nullptr;
     int threads = 0;    // block size where a pass has more than one (0: its default)
     bool xfft = true;   // tiled deposit: some replica of the set transforms along x in it
-    bool anyrec = true; // ... deposits position records; particles: some replica's order is above 1
+    // some replica of the set needs the instantiation that holds every form.  Deposit:
+    // position records; particles: orders above 1; forward plane pass: rectangles and y
+    // columns; y inverse, x C2R: plans with a group of two stages
+    bool allforms = true;
 };
 
 // Launch on c.stream; with c.t0 set, through hipExtLaunchKernel, whose events take
@@ -120,6 +123,9 @@ __host__ __device__ constexpr bool reg_plan_kept(int n) {
     return n == 24 || n == 25 || n == 30 || n == 32 || n == 40 || n == 48 || n == 50 || n == 64 || n == 80 || n == 128 ||
            n == 160;
 }
+// Plans with a group of two stages hold more values a thread (reg_plan_grouped): sets without
+// them run kernels compiled without them, whose registers leave room for more waves.
+__host__ __device__ constexpr bool reg_plan_grouped(int A1, int B1) { return A1 > 1 || B1 > 1; }
 // key, group sizes and first stage of the second group of an axis plan (key 0: not compiled)
 struct RegDims {
     int key, R1, R2, group2;

@@ -748,7 +748,7 @@ hipError_t launch_tile_deposit(const LaunchCtx& c, int koff) {
         deposit_launch<256, false, false>, deposit_launch<256, false, true>, deposit_launch<256, true, false>,
         deposit_launch<256, true, true>,   deposit_launch<512, false, false>, deposit_launch<512, false, true>,
         deposit_launch<512, true, false>,  deposit_launch<512, true, true>};
-    kernels[(c.threads >= 512 ? 4 : 0) + (c.xfft ? 2 : 0) + (c.anyrec ? 1 : 0)](c, koff);
+    kernels[(c.threads >= 512 ? 4 : 0) + (c.xfft ? 2 : 0) + (c.allforms ? 1 : 0)](c, koff);
     CHECK_LAUNCH(); return hipSuccess;
 }
 

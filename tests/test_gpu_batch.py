@@ -119,3 +119,23 @@ def test_square_planes_keep_their_bits_in_a_mixed_set(tmp_path):
         assert np.array_equal(b.positions(ids[k]), e.positions()), grids[k]
         e.close()
     b.close()
+
+
+def test_y_inverse_keeps_its_bits_in_a_mixed_set(tmp_path):
+    # planes without an inverse plane pass: with a y plan of grouped stages in the set the y
+    # inverse is a kernel that holds every plan
+    grids = [(20, n, 9) for n in (24, 25, 30, 32, 40, 48, 50, 64, 80, 128, 160)] + [(20, 36, 9), (20, 125, 9)]
+    systems = []
+    for k, g in enumerate(grids):
+        t, d = decks.melt3d(tmp_path / str(k), grid=g, box=tuple(0.5 * n for n in g), n_chains=4 * g[1], delt=0.02)
+        systems.append(tild.System(t, d))
+    b = tild.Batch(device=0)
+    ids = [b.add(s, 20 + k) for k, s in enumerate(systems)]
+    b.step(8)
+    for k, s in enumerate(systems):
+        e = tild.Engine(s, device=0, seed=20 + k)
+        assert e.geometry()["grad_reg"] == 1
+        e.step(8)
+        assert np.array_equal(b.positions(ids[k]), e.positions()), grids[k]
+        e.close()
+    b.close()
