@@ -139,3 +139,24 @@ def test_y_inverse_keeps_its_bits_in_a_mixed_set(tmp_path):
         assert np.array_equal(b.positions(ids[k]), e.positions()), grids[k]
         e.close()
     b.close()
+
+
+def test_x_c2r_keeps_its_bits_in_a_mixed_set(tmp_path):
+    # films and planes without an inverse plane pass: with an x plan of grouped stages in the
+    # set the x C2R is a kernel that holds every plan
+    grids = [(n, 36) for n in (21, 24, 25, 30, 32, 40, 48, 50, 64, 80, 100, 128, 160)] + [(100, 128, 9), (64, 256, 9)]
+    grids += [(96, 40), (225, 40), (120, 128, 9)]
+    systems = []
+    for k, g in enumerate(grids):
+        mk = decks.melt3d if len(g) == 3 else decks.melt2d
+        t, d = mk(tmp_path / str(k), grid=g, box=tuple(0.5 * n for n in g), n_chains=3 * g[0], delt=0.02)
+        systems.append(tild.System(t, d))
+    b = tild.Batch(device=0)
+    ids = [b.add(s, 20 + k) for k, s in enumerate(systems)]
+    b.step(8)
+    for k, s in enumerate(systems):
+        e = tild.Engine(s, device=0, seed=20 + k)
+        e.step(8)
+        assert np.array_equal(b.positions(ids[k]), e.positions()), grids[k]
+        e.close()
+    b.close()

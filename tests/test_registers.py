@@ -34,7 +34,7 @@ def _vgprs(tmp):
 
 
 # 512 registers per SIMD lane: 128 are four waves, 168 three
-@pytest.mark.parametrize("kernel,limit", [("k_grad_reg", 128)])
+@pytest.mark.parametrize("kernel,limit", [("k_grad_reg", 128), ("k_c2r_reg", 128)])
 def test_the_lean_instantiation_keeps_its_waves(kernel, limit, tmp_path):
     if not pathlib.Path(READELF).exists():
         pytest.skip("no llvm-readelf")
