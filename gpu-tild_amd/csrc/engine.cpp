@@ -683,6 +683,9 @@ int Batch::upload_desc(int id, std::string& err) {
 // ---------------------------------------------------------------- work maps
 int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& err, bool reorder_only) {
     for (int p = 0; p < PH_COUNT; ++p) { maps[p].host.clear(); maps[p].lds = 0; maps[p].n = 0; maps[p].xfft = false; maps[p].allforms = false; }
+    unsigned last_classes = 0;   // of the fused last-axis pass in the set
+    for (int id : ids)
+        if (const RepDev& h = reps_[id]->h; h.last_reg) last_classes |= 1u << last_reg_class(h.ax[h.dim - 1].N, h.ntypes);
     for (int id : ids) {
         const Replica& R = *reps_[id];
         const RepDev& h = R.h;
@@ -741,7 +744,8 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         }
         const int la = D - 1, Nla = la == 2 ? h.Nz : h.Ny, Q = la == 2 ? h.Ny * h.Nxh : h.Nxh;
         if (h.last_reg) {
-            const Phase cls[3] = {PH_LASTR, PH_LASTR4, PH_LASTRW};
+            // class 0 joins the launch of another class of the set
+            const Phase cls[3] = {last_classes & 4 ? PH_LASTRW : (last_classes & 2 ? PH_LASTR4 : PH_LASTR), PH_LASTR4, PH_LASTRW};
             add(cls[last_reg_class(h.ax[la].N, h.ntypes)], (Q + h.nl_last - 1) / h.nl_last,
                 last_reg_lds_bytes(h.ax[la], h.nf));
         }

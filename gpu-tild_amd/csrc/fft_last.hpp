@@ -23,8 +23,8 @@
 // the instructions and held up to 256 registers; the stage was the longest of the block
 // (2.7 of 7.7 us on a 192-point film's 13 blocks, where it ran one wave per SIMD).
 // The transforms and sums are those of the LDS-staged pass (whose inverse runs the same
-// plan, RepDev::axr), bit for bit but for the kept plans (reg_plan_kept), whose products
-// the compiler fuses with other sums here.
+// plan, RepDev::axr), bit for bit but for the kept plans (reg_plan_kept), whose twiddle
+// products fuse the other of their two sums' terms here (cmul_kept).
 #pragma once
 #include "device.hpp"
 #include "fft_dev.hpp"
@@ -117,13 +117,6 @@ __device__ __forceinline__ void last_reg_block(const RepDev& r, int blk, float2*
     if (liveB) {
 #pragma unroll
         for (int rr = 0; rr < R2; ++rr) w[rr] = X1[(i + R1 * rr) * ldx + f * NB + b];
-        // With four types or charges the twiddles of the kept plans count as read here: which
-        // of a sum's two products the compiler fuses follows the order their operands are
-        // read in, and this order keeps the rounding that such decks have had.
-        if constexpr (P::KEPT && (TT == 4 || CH)) {
-#pragma unroll
-            for (int rr = 1; rr < R2; ++rr) asm volatile("" : "+v"(t1[rr].x), "+v"(t1[rr].y));
-        }
         plan_second<P, !P::KEPT>(w, [&](int m) { return t1[m]; });
         if constexpr (XCH) {
 #pragma unroll
@@ -216,7 +209,7 @@ __device__ __forceinline__ void last_reg_block(const RepDev& r, int blk, float2*
 
 template <class P, int NT, int TT, int CH, int CLS>
 __device__ __forceinline__ void last_reg_variant_block(const RepDev& r, int blk, float2* lds, int koff) {
-    if constexpr (last_reg_variant(P::A0, P::R1, P::R2, P::REV, TT) && last_reg_class(P::N, TT) == CLS)
+    if constexpr (last_reg_variant(P::A0, P::R1, P::R2, P::REV, TT) && (last_reg_class(P::N, TT) == CLS || last_reg_class(P::N, TT) == 0))
         last_reg_block<P, NT, TT, CH>(r, blk, lds, koff);
 }
 
@@ -240,7 +233,9 @@ __device__ __forceinline__ void last_reg_types(const RepDev& r, int blk, float2*
 
 // One instantiation per class of variants (last_reg_class), each compiled in a file of
 // its own: a class's registers do not lower the occupancy of another's, and the classes
-// compile side by side.
+// compile side by side.  The kernels of classes 1 and 2 hold class 0 too: in a set of several
+// classes its replicas join their launch (films of 64 and 128 points in one launch 7.5 us a
+// step, in two 12.7; six 64^3 and six 64 x 64 x 128 melts 35.9 and 43.2).
 template <int NT, int CLS>
 __global__ void __launch_bounds__(NT) k_last_reg(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap,
                                                  int koff) {

@@ -1,4 +1,4 @@
-// fft_last2.hip -- k_last_reg for longer axes, one or two types.
+// fft_last2.hip -- k_last_reg for longer axes, one or two types (and those of fft_last0.hip).
 #include "fft_last.hpp"
 
 namespace tild {

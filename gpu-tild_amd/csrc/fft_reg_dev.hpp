@@ -39,8 +39,9 @@ __device__ __forceinline__ float2 cmul_fused(float2 a, float2 b) {
     const float yy = a.y * b.y, yx = a.y * b.x;
     return make_float2(__builtin_fmaf(a.x, b.x, -yy), __builtin_fmaf(a.x, b.y, yx));
 }
-// ... those of the kept plans' forward plane pass, which is compiled into two kernels and
-// whose bits may not depend on which of them a set of replicas runs
+// ... those of the kept plans in the forward plane pass and the fused last-axis pass,
+// which are compiled into several kernels: a replica's bits may not depend on which of
+// them its set runs
 __device__ __forceinline__ float2 cmul_kept(float2 a, float2 b) {
 #pragma clang fp contract(off)
     const float yy = a.y * b.y, xy = a.x * b.y;
@@ -48,7 +49,7 @@ __device__ __forceinline__ float2 cmul_kept(float2 a, float2 b) {
 }
 template <bool FUSED> __device__ __forceinline__ float2 cmul_as(float2 a, float2 b) {
     if constexpr (FUSED) return cmul_fused(a, b);
-    else return cmul(a, b);
+    else return cmul_kept(a, b);
 }
 
 // The n values are computed here: a sum that the compiler moves to its use in a later block
@@ -105,7 +106,7 @@ __device__ __forceinline__ int tw2_index(int i, int m) {
 }
 
 // The second group of plan P on w[s], s < R2, in place (output q natural); tw(m) = the m-th
-// twiddle of this thread.  FUSED: products as the LDS-staged stages fuse them.
+// twiddle of this thread.  FUSED: products as the LDS-staged stages fuse them, else cmul_kept.
 template <class P, bool FUSED, class TW>
 __device__ __forceinline__ void plan_second(float2* w, TW tw) {
     constexpr int C = P::B0, D = P::B1;

@@ -142,7 +142,7 @@ __host__ __device__ constexpr bool last_reg_variant(int A0, int R1, int R2, bool
     return TT <= (R1 * R2 > 100 || A0 == 16 ? 2 : 4) && TT * (rev ? R2 : R1) <= 50;
 }
 // the kernel instantiation of a variant: axes up to 100 points with up to two types (class
-// 0) or three and four (class 1), and longer axes (class 2)
+// 0, held by the other two as well) or three and four (class 1), and longer axes (class 2)
 __host__ __device__ constexpr int last_reg_class(int N, int TT) { return N > 100 ? 2 : (TT >= 3 ? 1 : 0); }
 bool last_reg_plan(const AxisPlan& pl, int ntypes, int nf);
 // columns of a block: one thread per (column, index of the larger group, field)

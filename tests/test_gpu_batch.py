@@ -160,3 +160,35 @@ def test_x_c2r_keeps_its_bits_in_a_mixed_set(tmp_path):
         assert np.array_equal(b.positions(ids[k]), e.positions()), grids[k]
         e.close()
     b.close()
+
+
+@pytest.mark.parametrize("other", ["long_axis", "three_types"])
+def test_last_axis_keeps_its_bits_in_a_mixed_set(other, tmp_path):
+    # short axes of one or two types run the fused last-axis pass in the kernel of the longer
+    # axes, or of the larger type counts, that share their set
+    def deck(d, grid, ntypes, charged):
+        box = tuple(0.5 * n for n in grid) + ((1.0,) if len(grid) == 2 else ())
+        d.mkdir()
+        pos, types, mols, bonds = tild_gen.diblock(np.random.default_rng(grid[-1]), 150, 10, 0.5, box, len(grid))
+        types = 1 + np.arange(len(types)) % ntypes
+        styles = [("gaussian", i, j, 0.5 + 0.2 * i * j, 0.5) for i in range(1, ntypes + 1) for j in range(i, ntypes + 1)]
+        q = np.where(mols % 2 == 0, 1.0, -1.0) if charged else None
+        tild_gen.write_data(d / "input.data", pos, types, mols, bonds, box, ntypes, len(grid), charges=q)
+        return tild.System(tild_gen.deck("input.data", len(grid), grid, styles, "EM", 0.02, 3,
+                                         **(dict(charges=(1.0, 0.7)) if charged else {})), d)
+
+    cases = [((20, 18, n), 1 + k % 2, k % 3 == 0) for k, n in enumerate((24, 25, 27, 30, 32, 36, 40, 45, 48, 50, 64, 80, 96))]
+    cases += [((18, n), 1 + k % 2, k % 3 == 1) for k, n in enumerate((24, 30, 48, 50, 64, 72, 80, 100))]
+    cases += {"long_axis": [((20, 18, 128), 2, False), ((18, 160), 1, True)],
+              "three_types": [((20, 18, 40), 3, False), ((18, 64), 4, True)]}[other]
+    systems = [deck(tmp_path / str(k), *c) for k, c in enumerate(cases)]
+    b = tild.Batch(device=0)
+    ids = [b.add(s, 20 + k) for k, s in enumerate(systems)]
+    b.step(8)
+    for k, s in enumerate(systems):
+        e = tild.Engine(s, device=0, seed=20 + k)
+        assert e.geometry()["last_reg"] == 1
+        e.step(8)
+        assert np.array_equal(b.positions(ids[k]), e.positions()), cases[k]
+        e.close()
+    b.close()
