@@ -681,11 +681,65 @@ int Batch::upload_desc(int id, std::string& err) {
 }
 
 // ---------------------------------------------------------------- work maps
+// A pass launches a kernel per form that the set's replicas run, and a launch more costs 4 to
+// 5 us a step.  Where some replica has only the LDS-staged form, that launch is there anyway,
+// and the others of a small set, whose register forms give the same bits, join it: the register
+// form gains less on them than its launch costs.  Both sides measured, us a step: forward plane
+// 24 x 32 with 20 x 32 together 6.6, apart 11.0, 40 x 80 x 160 with 20 x 40 10.2 and 17.0, four
+// 40 x 80 x 80 16.5 and 20.6, eight 24.8 and 25.3; y inverse and x C2R of these 11.2 and 16.3,
+// 18.7 and 23.8, 27.6 and 31.1, 46.8 and 45.1; x C2R of films of 64 and 256 points 6.7 and 10.3.
+// So the line lies at 2^21 nodes; plans of grouped stages, whose staged form takes two to three
+// times as long (36^3 7.4 apart 10.9, but 72^3 13.8 against 6.9 + 4), count four times.
+constexpr double kJoinNodes = 2097152.0;
+// Deposits that transform x have more registers (128 against 52) and LDS, which would bound the
+// others' blocks per CU (sweep of 24 replicas, 10 of them of odd sides: 23.7 us a step in one
+// launch, 21.7 in two); sets of fewer tiles than two a CU are resident at once in either (27^3
+// with 20^3 6.9 in one launch, 10.5 in two).
+constexpr int kJoinTiles = 512;
+
+Batch::SetForms Batch::set_forms(const std::vector<int>& ids) const {
+    SetForms f;
+    double fwd = 0.0, inv = 0.0, c2r = 0.0;
+    bool square = false, square_inv = false, rect = false, yfwd = false, staged_plane = false, staged_y = false,
+         staged_c2r = false, y_staged = false, c2r_fits = true;
+    int tiles = 0;
+    for (int id : ids) {
+        const RepDev& h = reps_[id]->h;
+        const double nodes = (double)h.nf * (double)h.M;
+        const double weight = h.ax[0].nst > 2 || h.ax[1].nst > 2 ? 4.0 : 1.0;
+        if (h.spread_mode == 2) tiles += h.ntiles;
+        if (h.last_reg) f.last_classes |= 1u << last_reg_class(h.ax[h.dim - 1].N, h.ntypes);
+        if (h.dim == 3) {
+            if (h.plane_reg) square = true;
+            else if (h.plane_rect) { rect = true; fwd += weight * nodes; }
+            else if (h.yfwd_reg) { yfwd = true; fwd += weight * nodes; }
+            else if (h.plane_fwd) staged_plane = true;
+            else staged_y = true;
+            if (h.plane_inv) square_inv = true;
+            else if (h.plane_pair) inv += weight * nodes;
+            else if (h.grad_reg) f.y_reg = true;
+            else y_staged = true;
+        }
+        const int nc = (h.nf * h.dim + 1) / 2;
+        if (h.c2r_reg) {
+            c2r += (h.ax[0].nst > 2 ? 4.0 : 1.0) * nodes;
+            c2r_fits = c2r_fits && h.nr_c2r * nc * h.Nx <= kFftBudget && lds_bytes(h.Nx, h.nr_c2r * nc) <= kMaxLds;
+        } else if (!(h.dim == 3 && (h.plane_inv || h.plane_pair))) staged_c2r = true;
+    }
+    // only where the register form's launch then goes: not where a square plane keeps it
+    f.fwd_staged = !square && (!rect || staged_plane) && (!yfwd || staged_y) && fwd <= kJoinNodes;
+    f.inv_staged = !square_inv && staged_c2r && (f.y_reg || y_staged) && inv <= kJoinNodes;
+    f.c2r_staged = staged_c2r && c2r_fits && c2r <= kJoinNodes;
+    f.one_deposit = tiles <= kJoinTiles;
+    return f;
+}
+
 int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& err, bool reorder_only) {
     for (int p = 0; p < PH_COUNT; ++p) { maps[p].host.clear(); maps[p].lds = 0; maps[p].n = 0; maps[p].xfft = false; maps[p].allforms = false; }
-    unsigned last_classes = 0;   // of the fused last-axis pass in the set
-    for (int id : ids)
-        if (const RepDev& h = reps_[id]->h; h.last_reg) last_classes |= 1u << last_reg_class(h.ax[h.dim - 1].N, h.ntypes);
+    const SetForms forms = set_forms(ids);
+    bool tilex = false;   // some deposit transforms x
+    for (int id : ids) tilex = tilex || (reps_[id]->h.spread_mode == 2 && !reps_[id]->h.plane_fwd);
+    auto deposit_phase = [&](const RepDev& h) { return !h.plane_fwd || (tilex && forms.one_deposit) ? PH_TILEX : PH_TILE; };
     for (int id : ids) {
         const Replica& R = *reps_[id];
         const RepDev& h = R.h;
@@ -708,10 +762,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         if (h.spread_mode == 2) {
             add(PH_TCOUNT, (h.ns + kCountBlock - 1) / kCountBlock, 0);
             add(PH_SCAN, 1, 0);
-            // deposits that transform x apart: their registers (128 against 52) and LDS
-            // would bound the others' blocks per CU (sweep of 24 replicas, 10 of them of odd
-            // sides: 23.7 us a step in one launch, 21.7 in two)
-            const Phase dep = h.plane_fwd ? PH_TILE : PH_TILEX;
+            const Phase dep = deposit_phase(h);
             add(dep, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd, h.reg_key[0] && h.grid_off32));
             maps[dep].allforms = maps[dep].allforms || !h.srec;
             maps[PH_TILEX].xfft = true;
@@ -723,38 +774,38 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         {
             MidGeom g = mid_geom(h, 1, h.nf);
             add(PH_PY, g.nouter * g.nchunk, lds_bytes(g.N, g.nl));
+            const bool reg = !forms.fwd_staged;
             maps[PH_PLANER].allforms = maps[PH_PLANER].allforms || h.plane_rect || h.yfwd_reg;
             if (D == 3 && h.plane_reg) add(PH_PLANER, h.nf * h.Nz, plane_reg_lds_bytes(h.ax[0]));
-            else if (D == 3 && h.plane_rect) add(PH_PLANER, h.nf * h.Nz, plane_rect_lds_bytes(h.Nx, h.Ny));
-            else if (D == 3 && h.yfwd_reg) add(PH_PLANER, yfwd_reg_blocks(h.ax[1], h.Nxh, h.nf * h.Nz), yfwd_reg_lds_bytes(h.ax[1]));
+            else if (D == 3 && h.plane_rect && reg) add(PH_PLANER, h.nf * h.Nz, plane_rect_lds_bytes(h.Nx, h.Ny));
+            else if (D == 3 && h.yfwd_reg && reg) add(PH_PLANER, yfwd_reg_blocks(h.ax[1], h.Nxh, h.nf * h.Nz), yfwd_reg_lds_bytes(h.ax[1]));
             else if (D == 3 && h.plane_fwd) add(PH_PLANEF, h.nf * h.Nz, plane_r2c_lds(h));
             else if (D == 3) add(PH_MIDY_H, g.nouter * g.nchunk, lds_bytes(g.N, g.nl));
         }
         if (D == 3) {
             MidGeom g = mid_grad_geom(h);
             if (h.plane_inv) add(PH_PLANEI, h.nf * h.Nz, plane_inv_lds_bytes(h.ax[1]));
-            else if (h.plane_pair) add(PH_PLANEI, h.Nz * ((3 * h.nf + 2 * h.plane_pair - 1) / (2 * h.plane_pair)), plane_pair_lds_bytes(h.Nx, h.Ny, h.plane_pair));
-            else if (h.grad_reg) {
+            else if (h.plane_pair && !forms.inv_staged) add(PH_PLANEI, h.Nz * ((3 * h.nf + 2 * h.plane_pair - 1) / (2 * h.plane_pair)), plane_pair_lds_bytes(h.Nx, h.Ny, h.plane_pair));
+            else if (h.grad_reg && (!h.plane_pair || forms.y_reg)) {
                 maps[PH_MIDY_GR].allforms = maps[PH_MIDY_GR].allforms || h.ax[1].nst > 2;
                 add(PH_MIDY_GR, h.nf * h.Nz * grad_reg_chunks(h.ax[1], h.Nxh), grad_reg_lds_bytes(h.ax[1]));
-            }
-            else add(PH_MIDY_G, g.nouter * g.nchunk, lds_bytes(g.N, 3 * g.nl));
+            } else add(PH_MIDY_G, g.nouter * g.nchunk, lds_bytes(g.N, 3 * g.nl));
             MidGeom gz = mid_geom(h, 2, h.nf);
             add(PH_MIDZ_H, gz.nouter * gz.nchunk, lds_bytes(gz.N, gz.nl));
         }
         const int la = D - 1, Nla = la == 2 ? h.Nz : h.Ny, Q = la == 2 ? h.Ny * h.Nxh : h.Nxh;
         if (h.last_reg) {
             // class 0 joins the launch of another class of the set
-            const Phase cls[3] = {last_classes & 4 ? PH_LASTRW : (last_classes & 2 ? PH_LASTR4 : PH_LASTR), PH_LASTR4, PH_LASTRW};
+            const Phase cls[3] = {forms.last_classes & 4 ? PH_LASTRW : (forms.last_classes & 2 ? PH_LASTR4 : PH_LASTR), PH_LASTR4, PH_LASTRW};
             add(cls[last_reg_class(h.ax[la].N, h.ntypes)], (Q + h.nl_last - 1) / h.nl_last,
                 last_reg_lds_bytes(h.ax[la], h.nf));
         }
         else add(PH_LAST, (Q + h.nl_last - 1) / h.nl_last, last_lds_bytes(Nla, h.nf, h.last_dirs, h.nl_last));
         const int nc = (h.nf * D + 1) / 2;
-        if (h.c2r_reg) {
+        if (h.c2r_reg && !forms.c2r_staged) {
             maps[PH_C2RR].allforms = maps[PH_C2RR].allforms || h.ax[0].nst > 2;
             add(PH_C2RR, (rows + h.nr_c2r - 1) / h.nr_c2r, c2r_reg_lds_bytes(h.Nx, h.nr_c2r * nc));
-        } else if (!h.plane_inv && !h.plane_pair) add(PH_C2R, (rows + h.nr_c2r - 1) / h.nr_c2r, lds_bytes(h.Nx, h.nr_c2r * nc));
+        } else if (!h.plane_inv && !(h.plane_pair && !forms.inv_staged)) add(PH_C2R, (rows + h.nr_c2r - 1) / h.nr_c2r, lds_bytes(h.Nx, h.nr_c2r * nc));
         add(PH_KPROPS, h.nchunk > 0 ? h.nchunk : 1, 0);
     }
     // Deposit block size: 512 threads when the set's tiles hold ~600 beads or more on
@@ -765,7 +816,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         long long beads = 0, tiles = 0;
         int want = -1;   // the block size the launch's replicas ask for, if they agree
         for (int id : ids)
-            if (reps_[id]->h.spread_mode == 2 && (dep == PH_TILE) == (reps_[id]->h.plane_fwd != 0)) {
+            if (reps_[id]->h.spread_mode == 2 && deposit_phase(reps_[id]->h) == dep) {
                 const long long np = std::max(reps_[id]->h.P, 1) + 1, d = reps_[id]->dim;
                 beads += (long long)reps_[id]->ns * (d == 3 ? np * np * np / 8 : np * np / 4);
                 tiles += reps_[id]->h.ntiles;

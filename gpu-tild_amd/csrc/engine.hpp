@@ -213,6 +213,14 @@ private:
     // that are reused while large enough (the set of replicas due changes from one
     // reorder to the next, so these maps are not cached per set)
     int build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& err, bool reorder_only = false);
+    // forms of a set's passes that its replicas decide together
+    struct SetForms {
+        bool fwd_staged = false, inv_staged = false, c2r_staged = false;   // register forms that join the staged launch
+        bool y_reg = false;          // the set runs k_grad_reg without the planes that join
+        bool one_deposit = false;    // deposits with and without the x transform share a launch
+        unsigned last_classes = 0;   // classes of the fused last-axis pass
+    };
+    SetForms set_forms(const std::vector<int>& ids) const;
     PhaseMap reorder_maps_[PH_COUNT];
     int build_tables(Replica& R, const System& S, std::string& err);
     int forward_spectra(int id, std::string& err);   // rho -> H (properties)

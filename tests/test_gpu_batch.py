@@ -192,3 +192,30 @@ def test_last_axis_keeps_its_bits_in_a_mixed_set(other, tmp_path):
         assert np.array_equal(b.positions(ids[k]), e.positions()), cases[k]
         e.close()
     b.close()
+
+
+@pytest.mark.parametrize("grids", [
+    [(24, 32, 40), (20, 32, 40)], [(40, 80, 24), (20, 40, 24)], [(36, 36, 36), (20, 20, 20)], [(27, 27, 27), (20, 20, 20)],
+    [(45, 36, 20), (20, 40, 24)], [(25, 30, 20), (15, 25, 30)], [(48, 80, 9), (20, 50, 9), (25, 25, 9)],
+    [(128, 64, 9), (64, 128, 9), (20, 20, 9)], [(100, 128, 9), (125, 160, 9), (20, 25, 9)], [(64, 64), (96, 96), (20, 20)],
+    [(160, 40), (225, 40), (24, 30, 20), (250, 20)], [(24, 24, 24), (24, 32, 20), (20, 32, 20)],
+], ids=lambda g: "_".join("x".join(map(str, k)) for k in g))
+def test_sides_with_and_without_a_compiled_plan_share_a_set(grids, tmp_path):
+    # in small sets the register forms join the staged launches of the replicas that have no
+    # other; each replica keeps the bits it has alone
+    systems = []
+    for k, g in enumerate(grids):
+        mk = decks.melt3d if len(g) == 3 else decks.melt2d
+        t, d = mk(tmp_path / str(k), grid=g, box=tuple(0.5 * n for n in g), n_chains=200, delt=0.02)
+        systems.append(tild.System(t, d))
+    b = tild.Batch(device=0)
+    ids = [b.add(s, 20 + k) for k, s in enumerate(systems)]
+    b.step(8, graph=False)
+    b.step(70, graph=True)
+    for k, s in enumerate(systems):
+        e = tild.Engine(s, device=0, seed=20 + k)
+        e.step(78)
+        assert np.array_equal(b.positions(ids[k]), e.positions()), grids[k]
+        assert all(np.array_equal(b.density(ids[k], t), e.density(t)) for t in range(s.ntypes))
+        e.close()
+    b.close()
