@@ -331,6 +331,13 @@ tild_status tild_engine_geometry(tild_engine* e, tild_geometry* out) {
     return geometry_of(e->batch->rep(e->id), out);
 }
 
+tild_status tild_engine_passes(tild_engine* e, tild_passes* out) {
+    if (!e || !out) return fail(TILD_ERR_ARG, "null argument");
+    const tild::RepDev& h = e->batch->rep(e->id)->h;
+    *out = tild_passes{h.plane_rect, h.yfwd_reg, h.plane_pair > 0 ? 1 : 0, h.c2r_reg};
+    return TILD_OK;
+}
+
 tild_status tild_batch_profile(tild_batch* b, const int* replicas, int nrep, int nsteps, double* ms, int nphase) {
     if (!b || nrep < 0 || (nrep > 0 && !replicas)) return fail(TILD_ERR_ARG, "bad argument");
     std::vector<int> ids(replicas, replicas + nrep);

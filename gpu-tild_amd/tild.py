@@ -27,7 +27,7 @@ EXPORTS = [
     "tild_engine_get_state", "tild_engine_set_state",
     "tild_engine_synchronize", "tild_engine_get_bins", "tild_engine_profile", "tild_engine_nlist", "tild_fft_r2c", "tild_fft_c2r",
     "tild_fft_c2r_noalloc", "tild_system_compute", "tild_engine_sk_accumulate", "tild_engine_sk_average",
-    "tild_engine_geometry", "tild_batch_geometry",
+    "tild_engine_geometry", "tild_batch_geometry", "tild_engine_passes",
     "tild_batch_create", "tild_batch_destroy", "tild_batch_last_error", "tild_batch_add", "tild_batch_remove",
     "tild_batch_step", "tild_batch_properties", "tild_batch_get_positions", "tild_batch_set_positions",
     "tild_batch_get_density", "tild_batch_replica_step", "tild_batch_profile",
@@ -60,6 +60,13 @@ class Geometry(ctypes.Structure):
                 ("grad_reg", ctypes.c_int), ("plane_reg", ctypes.c_int), ("plane_inv", ctypes.c_int),
                 ("tuned", ctypes.c_int),
                 ("from_cache", ctypes.c_int), ("step_ms", ctypes.c_double)]
+
+    def as_dict(self):
+        return {k: getattr(self, k) for k, _ in self._fields_}
+
+
+class Passes(ctypes.Structure):
+    _fields_ = [(k, ctypes.c_int) for k in ("plane_rect", "yfwd_reg", "plane_pair", "c2r_reg")]
 
     def as_dict(self):
         return {k: getattr(self, k) for k, _ in self._fields_}
@@ -166,6 +173,7 @@ def lib():
         L.tild_engine_sk_accumulate.argtypes = [vp, ctypes.c_int, ctypes.c_int]
         L.tild_engine_sk_average.argtypes = [vp, ctypes.c_int, fp, sz, ip]
         L.tild_engine_geometry.argtypes = [vp, vp]
+        L.tild_engine_passes.argtypes = [vp, vp]
         L.tild_batch_geometry.argtypes = [vp, ctypes.c_int, vp]
         _lib = L
     return _lib
@@ -332,6 +340,12 @@ class Engine:
         g = Geometry()
         self._chk(lib().tild_engine_geometry(self._h, ctypes.byref(g)), "geometry")
         return g.as_dict()
+
+    def passes(self):
+        """Register-resident forms of the FFT passes that geometry() does not name."""
+        p = Passes()
+        self._chk(lib().tild_engine_passes(self._h, ctypes.byref(p)), "passes")
+        return p.as_dict()
 
     def sk_accumulate(self, t, slot=None):
         """avg_sk: add rho_t(k) rho_t(k) / M of the last force evaluation's densities to

@@ -222,6 +222,14 @@ typedef struct {
     double step_ms;      /* kernel time per step measured by the tuner (0 if not tuned) */
 } tild_geometry;
 tild_status tild_engine_geometry(tild_engine* e, tild_geometry* out);
+/* The register-resident forms tild_geometry does not name, 1 where the engine runs them. */
+typedef struct {
+    int plane_rect;      /* forward plane pass, other planes than plane_reg's */
+    int yfwd_reg;        /* forward y pass (odd sides, whose deposit transforms x) */
+    int plane_pair;      /* y inverse and x C2R as one pass, other planes than plane_inv's */
+    int c2r_reg;         /* x C2R where no plane pass runs it */
+} tild_passes;
+tild_status tild_engine_passes(tild_engine* e, tild_passes* out);
 /* Compute::doCompute for avg_sk (Compute.cu:83-117): adds rho_t(k) rho_t(k) / M -- the
    complex square of the unnormalised transform, as d_multiplyComplex forms it, not
    |rho_t(k)|^2 -- of the densities of the last force evaluation (after
