@@ -525,7 +525,7 @@ int Batch::add_plain(const System& S, uint32_t seed, std::string& err) {
     // the register form of the x C2R into the records, where the plane pass does not run: one
     // stage-B task per thread, and no more rows per block than leave a block for every CU
     // (a small launch is bound by one block's chain of phases)
-    h.c2r_reg = h.reg_key[0] && h.grid_off32 && !h.FPtab && !h.plane_inv && !h.plane_pair ? 1 : 0;
+    h.c2r_reg = h.reg_key[0] && c2r_reg_plan(h.ax[0], D) && h.grid_off32 && !h.FPtab && !h.plane_inv && !h.plane_pair ? 1 : 0;
     if (h.c2r_reg) {
         const RegDims rd = reg_dims(h.ax[0]);
         int nr = std::max(1, kC2rRegThreads / (nc * std::max(rd.R1, rd.R2)));

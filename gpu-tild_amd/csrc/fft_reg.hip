@@ -761,15 +761,14 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) k_
 // ------------------------------------------------------------------ x C2R
 // Inverse x transform of the half spectra into the gather records (the operation of
 // k_x_c2r, kernels.hip) for compiled x plans, where no plane pass runs it (2D, and planes
-// above half a CU's LDS); nr_c2r rows per block, nc complex lines per row:
+// above half a CU's LDS; c2r_reg_plan); nr_c2r rows per block, nc complex lines per row:
 //   A  task (line b, i < R2): Z = A + i B at k = i + R2 r of the full spectrum straight
 //      from the half spectra (the upper half by Hermitian symmetry), first group; exchange;
 //   B  task (b, i < R1): second group -> the real lines, over the values the task read;
 //   C  the records (g_x, g_y, g_z), stored in order.
 // Two barriers; the staged form has four and waits for its second stage's twiddles (film
-// 64^2 5.6 -> 4.3 us, the latency of a launch of few blocks; 192^2 5.2 -> 4.8).  It
-// reads each half-spectrum value twice (the second time from cache), which is why grids of
-// many planes take the plane pass instead.
+// 64^2 5.6 -> 4.3 us, the latency of a launch of few blocks; 192^2 5.2 -> 4.8).  It reads
+// each half-spectrum value twice, the second time from cache.
 namespace {
 template <class P, int NT>
 __device__ __forceinline__ void c2r_reg_block(const RepDev& r, int blk, float2* lds) {
@@ -875,6 +874,18 @@ __global__ void __launch_bounds__(NT) k_c2r_reg(const RepDev* __restrict__ reps,
 #undef TILD_CASE
         default: break;   // reg_key holds compiled plans only
     }
+}
+
+// x plans for the register form.  In three dimensions not 160 points, whose LDS-staged form runs
+// its two stages compiled (lds_fft2), nor 125, where a group of 5 leaves a fifth of the threads
+// for the other's 25 values: staged and register form, us, 160 x 80 x 24 6.8 and 8.3, 160 x 80 x
+// 80 14.7 and 15.5, 160^3 44.6 and 43.3; 125 x 100 x 100 22.3 and 23.7, with four types and
+// charges 125 x 125 x 40 24.6 and 32.0.  The others gain, at any number of planes: 80 x 160 x 80
+// 14.0 and 13.2, 100^3 17.2 and 14.1, 128 x 128 x 24 9.3 and 8.0, x 160 36.6 and 27.2, 180 x 180
+// x 50 35.2 and 23.4; and films gain or are alike at every length.
+bool c2r_reg_plan(const AxisPlan& pl, int dim) {
+    const RegDims d = reg_dims(pl);
+    return dim == 2 || !((d.R1 == 16 && d.R2 == 10) || d.R2 >= 5 * d.R1);
 }
 
 hipError_t launch_c2r_reg(const LaunchCtx& c) {

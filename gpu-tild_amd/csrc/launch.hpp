@@ -240,6 +240,7 @@ inline size_t plane_r2c_lds(const RepDev& h) {
 // field phases): one exchange buffer and the second group's twiddles.
 constexpr int kC2rRegThreads = 256;
 inline size_t c2r_reg_lds_bytes(int N, int nlines) { return fft_buf_bytes(N, nlines) + (size_t)N * sizeof(float2); }
+bool c2r_reg_plan(const AxisPlan& pl, int dim);
 hipError_t launch_c2r_reg(const LaunchCtx& c);
 // One-time kernel attributes (dynamic LDS above 64 KiB for the plane pass).
 hipError_t configure_kernels();

@@ -58,3 +58,9 @@ def test_film_equals_staged(grid, ntypes, charged, tmp_path):
 def test_box_equals_staged(grid, ntypes, charged, c2r, tmp_path):
     _compare(_system(tmp_path, grid, ntypes, charged), {"last_reg": 1, "plane_reg": 0, "plane_inv": 0},
              {"plane_rect": int(grid[1] % 2 == 0), "yfwd_reg": int(grid[1] % 2 == 1), "plane_pair": 1 - c2r, "c2r_reg": c2r})
+
+
+# in boxes the x C2R of 125 and 160 points runs staged, where that form is the faster one
+@pytest.mark.parametrize("grid,c2r", [((125, 100, 9), 0), ((160, 80, 9), 0), ((120, 128, 9), 1), ((125, 27), 1), ((160, 27), 1)])
+def test_x_c2r_rule(grid, c2r, tmp_path):
+    _compare(_system(tmp_path, grid, 2, False), {"last_reg": int(len(grid) == 2)}, {"c2r_reg": c2r})
