@@ -735,7 +735,7 @@ Batch::SetForms Batch::set_forms(const std::vector<int>& ids) const {
 }
 
 int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& err, bool reorder_only) {
-    for (int p = 0; p < PH_COUNT; ++p) { maps[p].host.clear(); maps[p].lds = 0; maps[p].n = 0; maps[p].xfft = false; maps[p].allforms = false; }
+    for (int p = 0; p < PH_COUNT; ++p) { maps[p].host.clear(); maps[p].lds = 0; maps[p].n = 0; maps[p].xfft = kXNone; maps[p].allforms = false; }
     const SetForms forms = set_forms(ids);
     bool tilex = false;   // some deposit transforms x
     for (int id : ids) tilex = tilex || (reps_[id]->h.spread_mode == 2 && !reps_[id]->h.plane_fwd);
@@ -763,9 +763,10 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
             add(PH_TCOUNT, (h.ns + kCountBlock - 1) / kCountBlock, 0);
             add(PH_SCAN, 1, 0);
             const Phase dep = deposit_phase(h);
-            add(dep, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd, h.reg_key[0] && h.grid_off32));
+            const bool xreg = h.reg_key[0] && h.grid_off32;
+            add(dep, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd, xreg));
             maps[dep].allforms = maps[dep].allforms || !h.srec;
-            maps[PH_TILEX].xfft = true;
+            if (!h.plane_fwd) maps[dep].xfft = std::max(maps[dep].xfft, (int)(xreg ? kXRegister : kXStaged));
             if (R.reorder_every > 0) add(PH_RTILE, h.ntiles, 0);
         } else {
             add(PH_SPREADA, R.nblk_part, 0);

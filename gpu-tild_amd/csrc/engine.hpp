@@ -43,7 +43,7 @@ struct PhaseMap {
     size_t lds = 0;
     int n = 0;
     int threads = 0;   // block size where a pass has more than one (0: its default)
-    bool xfft = true;  // tiled deposit: some replica of the set transforms along x in it
+    int xfft = kXRegister;   // tiled deposit: the x transforms its replicas run
     bool allforms = true;   // some replica of the set needs the instantiation of every form (LaunchCtx)
     int cap = 0;       // work items the device buffer holds
 };

@@ -56,6 +56,9 @@ inline size_t last_lds_bytes(int N, int nf, int DB, int nl) {
     return (size_t)N * nf * nl * sizeof(float2) + 2 * fft_buf_bytes(N, nf * DB * nl) + kMaxRamp * sizeof(float);
 }
 
+// x transforms of a deposit launch: none (the forward plane passes make them), the LDS-staged one,
+// or also those of the compiled plans
+enum { kXNone = 0, kXStaged = 1, kXRegister = 2 };
 struct LaunchCtx {
     const RepDev* reps;
     const WorkItem* wmap;
@@ -65,7 +68,7 @@ struct LaunchCtx {
     // step profile: events that take the kernel's own start and stop times
     hipEvent_t t0 = nullptr, t1 = nullptr;
     int threads = 0;    // block size where a pass has more than one (0: its default)
-    bool xfft = true;   // tiled deposit: some replica of the set transforms along x in it
+    int xfft = kXRegister;   // tiled deposit: the x transforms its replicas run
     // some replica of the set needs the instantiation that holds every form.  Deposit:
     // position records; particles: orders above 1; forward plane pass: rectangles and y
     // columns; y inverse, x C2R: plans with a group of two stages

@@ -484,18 +484,19 @@ __device__ __forceinline__ void deposit_xfft(const RepDev& r, const unsigned lon
 // 1,000 beads plus their halo share (three blocks of 512 fit a CU; on the 640,000-bead
 // melt 17.5 us, against 19.6 with 256 threads and 22.8 with 1,024, where one block
 // fills a CU); NT = 256 for small tiles, where a larger block mostly idles.
-// XFFT false: every replica of the set leaves the x transform to its forward plane pass,
-// so the block needs neither the transform's registers (79 VGPRs, six waves per SIMD)
-// nor its two LDS buffers (half of the block's LDS).
+// XFFT: kXNone where every replica of the set leaves the x transform to its forward plane
+// pass, so that the block needs neither the transform's registers (52, eight waves per SIMD)
+// nor its LDS buffers (half of the block's LDS); kXStaged without compiled x plans (71, seven
+// waves; a 512^2 film 10.0 us, and 11.3 in the kernel of all plans); kXRegister (128, four).
 // ANYREC: some replica of the set deposits position records (orders 0 and 2-4); without
 // them the kernel holds the stencil-record path only, and its registers.
-template <int kDepositThreads, bool XFFT, bool ANYREC>
-__global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* __restrict__ reps,
-                                                              const WorkItem* __restrict__ wmap, int koff) {
+template <int kDepositThreads, int XFFT, bool ANYREC>
+__global__ void __launch_bounds__(kDepositThreads) __attribute__((amdgpu_waves_per_eu(XFFT == kXStaged ? 6 : kDepositThreads / 256)))
+k_tile_deposit(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap, int koff) {
     extern __shared__ unsigned long long tile_lds[];
     const WorkItem wi = wmap[blockIdx.x];
     const RepDev& r = reps[wi.rep];
-    if (XFFT) warm_desc<0, 3, 4, 5, 6, 7>(r);
+    if (XFFT != kXNone) warm_desc<0, 3, 4, 5, 6, 7>(r);
     else warm_desc<0, 3, 4, 5, 6>(r);
     const int D = r.dim, Nx = r.Nx, Nxh = r.Nxh;
     const int By = r.By, Bz = r.Bz, nf = r.nf;
@@ -533,15 +534,15 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
     if (t == 0 && threadIdx.x == 0) G(r.tovf)[(par ^ 1) * 32] = 0;
     for (int k = threadIdx.x; k < rows * Nx; k += kDepositThreads) patch[k] = 0ull;
     const int T = r.ntypes;
-    const int Ny = r.Ny, M = r.M, plane_fwd = XFFT ? r.plane_fwd : 1;
+    const int Ny = r.Ny, M = r.M, plane_fwd = XFFT != kXNone ? r.plane_fwd : 1;
     // where the plane pass transforms the densities the FFT scratch is free: it holds
     // the first density element of each tile row (f, lz, ly)
     int* const rowoff = (int*)fbuf;
     // register form of the x transform: its twiddles and row table sit behind the exchange
-    const bool xreg = XFFT && !plane_fwd && r.reg_key[0] && r.grid_off32;
+    const bool xreg = XFFT == kXRegister && !plane_fwd && r.reg_key[0] && r.grid_off32;
     float2* const xtw = fbuf + (size_t)Nx * (((rows + 1) / 2) | 1);
     int* const rowid = (int*)(xtw + Nx);
-    if (XFFT && xreg) {
+    if (XFFT == kXRegister && xreg) {
         const int ntw = reg_ntw(r.reg_key[0], Nx);
         for (int k = threadIdx.x; k < ntw; k += kDepositThreads) xtw[k] = gld(r.reg_tw[0] + k);
         for (int rr = threadIdx.x; rr < rows; rr += kDepositThreads) {
@@ -619,7 +620,7 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
     }
     __syncthreads();
     // densities of the tile rows -> rho and the x-axis R2C (pairs of rows)
-    if (XFFT && xreg) {
+    if (XFFT == kXRegister && xreg) {
         switch (r.reg_key[0]) {   // uniform
 #define TILD_CASE(A0, A1, B0, B1)      \
     case reg_plan_key(A0, A1, B0, B1): \
@@ -686,7 +687,7 @@ __global__ void __launch_bounds__(kDepositThreads) k_tile_deposit(const RepDev* 
         }
         if (!plane_fwd) fbuf[n * ldb + j] = make_float2(v[0], v[1]);
     }
-    if constexpr (!XFFT) return;
+    if constexpr (XFFT == kXNone) return;
     if (plane_fwd) return;   // the plane pass transforms the densities
     __syncthreads();
     const float2* res = lds_fft<kDepositThreads>(fbuf, fbuf + (size_t)Nx * ldb, ldb, npairs, r.ax[0]);
@@ -738,17 +739,20 @@ hipError_t launch_tile_regions_set(const LaunchCtx& c) {
     hipLaunchKernelGGL(k_tile_regions_set, dim3(c.n), dim3(1024), 0, c.stream, c.reps, c.wmap);
     CHECK_LAUNCH(); return hipSuccess;
 }
-template <int NT, bool XFFT, bool ANYREC>
+template <int NT, int XFFT, bool ANYREC>
 static void deposit_launch(const LaunchCtx& c, int koff) {
     TILD_LAUNCH(c, (k_tile_deposit<NT, XFFT, ANYREC>), dim3(c.n), dim3(NT), c.lds, c.reps, c.wmap, koff);
 }
 hipError_t launch_tile_deposit(const LaunchCtx& c, int koff) {
     if (!c.n) return hipSuccess;
-    static void (*const kernels[8])(const LaunchCtx&, int) = {
-        deposit_launch<256, false, false>, deposit_launch<256, false, true>, deposit_launch<256, true, false>,
-        deposit_launch<256, true, true>,   deposit_launch<512, false, false>, deposit_launch<512, false, true>,
-        deposit_launch<512, true, false>,  deposit_launch<512, true, true>};
-    kernels[(c.threads >= 512 ? 4 : 0) + (c.xfft ? 2 : 0) + (c.allforms ? 1 : 0)](c, koff);
+    static void (*const kernels[2][3][2])(const LaunchCtx&, int) = {
+        {{deposit_launch<256, kXNone, false>, deposit_launch<256, kXNone, true>},
+         {deposit_launch<256, kXStaged, false>, deposit_launch<256, kXStaged, true>},
+         {deposit_launch<256, kXRegister, false>, deposit_launch<256, kXRegister, true>}},
+        {{deposit_launch<512, kXNone, false>, deposit_launch<512, kXNone, true>},
+         {deposit_launch<512, kXStaged, false>, deposit_launch<512, kXStaged, true>},
+         {deposit_launch<512, kXRegister, false>, deposit_launch<512, kXRegister, true>}}};
+    kernels[c.threads >= 512 ? 1 : 0][c.xfft][c.allforms ? 1 : 0](c, koff);
     CHECK_LAUNCH(); return hipSuccess;
 }
 

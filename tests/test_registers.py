@@ -33,8 +33,8 @@ def _vgprs(tmp):
     return out
 
 
-# 512 registers per SIMD lane: 128 are four waves, 168 three
-@pytest.mark.parametrize("kernel,limit", [("k_grad_reg", 128), ("k_c2r_reg", 128)])
+# 512 registers per SIMD lane: 128 are four waves, 84 six
+@pytest.mark.parametrize("kernel,limit", [("k_grad_reg", 128), ("k_c2r_reg", 128), ("k_tile_depositILi512ELi1ELb0E", 84)])
 def test_the_lean_instantiation_keeps_its_waves(kernel, limit, tmp_path):
     if not pathlib.Path(READELF).exists():
         pytest.skip("no llvm-readelf")
