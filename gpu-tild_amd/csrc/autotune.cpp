@@ -90,10 +90,13 @@ std::string class_key(int device, const System& S, int spread_mode) {
     int cus = 0;
     if (hipGetDeviceProperties(&p, device) == hipSuccess) { arch = p.gcnArchName; cus = p.multiProcessorCount; }
     const int oct2 = (int)std::floor(2.0 * std::log2((double)std::max(S.ns, 1)));
+    // entries measured on other kernels do not apply: the revision of the passes that the
+    // geometry settings reach, raised when these change
+    constexpr int kPassRevision = 2;
     std::ostringstream k;
     k << arch << "|cu" << cus << "|d" << S.Dim << "|" << S.Nx[0] << "x" << S.Nx[1] << "x" << (S.Dim == 3 ? S.Nx[2] : 1)
       << "|nf" << (S.ntypes + (S.charges.enabled ? 1 : 0)) << "|P" << S.pmeorder << "|ns2log" << oct2
-      << "|spread" << spread_mode;
+      << "|spread" << spread_mode << "|rev" << kPassRevision;
     return k.str();
 }
 
@@ -120,7 +123,7 @@ int Batch::add_with(const System& S, uint32_t seed, const Geometry& g, std::stri
 constexpr int kTuneCopies = 32;
 constexpr double kTuneBeads = 4.0e5;
 
-double Batch::measure_geometry(const System& S, uint32_t seed, const Geometry& g, std::string& err, int* passes) {
+double Batch::measure_geometry(const System& S, uint32_t seed, const Geometry& g, std::string& err, TunedForms& forms) {
     constexpr double kInf = std::numeric_limits<double>::infinity();
     const int copies = std::max(1, std::min(kTuneCopies, (int)std::lround(kTuneBeads / std::max(S.ns, 1))));
     std::vector<int> ids;
@@ -138,12 +141,13 @@ double Batch::measure_geometry(const System& S, uint32_t seed, const Geometry& g
     }
     tuning_ = false;
     // which forms of the FFT passes the geometry runs: a geometry that switches between
-    // forms that agree only to rounding is not a candidate (tuning changes no result)
+    // forms that agree only to rounding is not a candidate (tuning changes no result).  The
+    // forms not named here give the bits of the staged passes.
     {
         const RepDev& h = reps_[ids[0]]->h;
         const int sig = h.plane_reg | (h.last_reg << 1) | (h.grad_reg << 2) | (h.plane_inv << 3);
-        if (*passes < 0) *passes = sig;
-        else if (sig != *passes) {
+        if (forms.signature < 0) forms = TunedForms{sig, h.last_reg != 0, h.plane_fwd != 0, h.plane_inv || h.plane_pair};
+        else if (sig != forms.signature) {
             for (int r : ids) remove(r);
             return kInf;
         }
@@ -174,49 +178,36 @@ int Batch::tune_geometry(const System& S, uint32_t seed, TuneResult& out, std::s
         }
     }
     Geometry best;
-    int passes = -1;
-    double best_t = measure_geometry(S, seed, best, err, &passes);
+    TunedForms forms;
+    double best_t = measure_geometry(S, seed, best, err, forms);
     if (!std::isfinite(best_t)) {
         if (err.empty()) err = "autotune: the default block geometry does not run this deck";
         return -TILD_ERR_DEVICE;
     }
     const bool tiled_ok = spread_mode_ != 1;
-    // The register-resident passes are taken wherever the deck allows them: the fused
-    // z pass has no batching of inverse directions to tune, and the forward plane pass
-    // stays on where its register form applies (the separate passes agree with it to
-    // rounding only, and tuning changes no result).
-    bool reg_ok = false, plane_reg = false, plane_inv = false;
-    {
-        const int la = S.Dim - 1, nf = S.ntypes + (S.charges.enabled ? 1 : 0);
-        AxisPlan lp, px, py;
-        std::vector<float2> tw((size_t)std::max({S.Nx[0], S.Nx[1], S.Nx[la], 1}));
-        int ntw = 0;
-        reg_ok = plan_axis(S.Nx[la], lp, tw.data(), &ntw) == nullptr && last_reg_plan(lp, S.ntypes, nf);
-        plane_reg = S.Dim == 3 && plan_axis(S.Nx[0], px, tw.data(), &ntw) == nullptr &&
-                    plan_axis(S.Nx[1], py, tw.data(), &ntw) == nullptr && plane_reg_plan(px, py);
-        // the inverse plane pass leaves no x C2R rows to batch
-        plane_inv = plane_reg && S.Fields.empty() && plane_inv_plan(px, py) && px.rad[0] == py.rad[0] &&
-                    px.rad[1] == py.rad[1];
-    }
+    // The register-resident passes are taken wherever the deck allows them: the fused z pass
+    // has no batching to tune, the inverse plane passes leave no x C2R rows to batch, and the
+    // forward plane pass stays on where its square register form applies (the separate passes
+    // agree with it to rounding only, and tuning changes no result).
+    const bool plane_reg = forms.signature & 1;
     struct Axis { int Geometry::*field; std::vector<int> cand; bool on; };
     const std::vector<Axis> axes = {
-        {&Geometry::plane, {0, -1}, S.Dim == 3 && tiled_ok && !plane_reg},
+        {&Geometry::plane, {0, -1}, forms.plane_fwd && !plane_reg},
         {&Geometry::tile_target, {128, 256, 512, 1024}, tiled_ok},
         {&Geometry::dep_threads, {256, 512}, tiled_ok},
-        {&Geometry::last_lines, {0, 2, 4, 8, 16}, true},
-        {&Geometry::last_dirs, {1, 2}, true},
+        {&Geometry::last_lines, {0, 2, 4, 8, 16}, !forms.last_reg},
+        {&Geometry::last_dirs, {1, 2}, !forms.last_reg},
         {&Geometry::mid_elems, {0, 1024}, true},
-        {&Geometry::c2r_rows, {0, 1, 2, 4, 8, 16}, !plane_inv},
+        {&Geometry::c2r_rows, {0, 1, 2, 4, 8, 16}, !forms.plane_inverse},
     };
     for (const Axis& a : axes) {
         if (!a.on) continue;
-        if (a.field == &Geometry::last_dirs && reg_ok) continue;
         for (int c : a.cand) {
             if (best.*a.field == c) continue;
             Geometry g = best;
             g.*a.field = c;
             std::string e;
-            const double t = measure_geometry(S, seed, g, e, &passes);
+            const double t = measure_geometry(S, seed, g, e, forms);
             if (!e.empty()) { err = e; return -TILD_ERR_DEVICE; }
             if (t < 0.98 * best_t) { best = g; best_t = t; }
         }

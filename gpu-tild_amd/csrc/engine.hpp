@@ -189,9 +189,13 @@ public:
 private:
     // the sweep behind set_autotune (autotune.cpp)
     int tune_geometry(const System& S, uint32_t seed, TuneResult& out, std::string& err);
-    // kernel ms per replica of a step of g; *passes: the FFT-pass forms g runs, set by the
-    // first call (< 0 on entry), and any later g running other forms measures +inf
-    double measure_geometry(const System& S, uint32_t seed, const Geometry& g, std::string& err, int* passes);
+    // kernel ms per replica of a step of g; forms: those of the FFT passes that g runs, set by
+    // the first call, and any later g of another signature measures +inf
+    struct TunedForms {
+        int signature = -1;
+        bool last_reg = false, plane_fwd = false, plane_inverse = false;
+    };
+    double measure_geometry(const System& S, uint32_t seed, const Geometry& g, std::string& err, TunedForms& forms);
     int add_with(const System& S, uint32_t seed, const Geometry& g, std::string& err);
     int add_plain(const System& S, uint32_t seed, std::string& err);
     bool autotune_ = false, tuning_ = false;
