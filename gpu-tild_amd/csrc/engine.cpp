@@ -797,6 +797,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
         const int la = D - 1, Nla = la == 2 ? h.Nz : h.Ny, Q = la == 2 ? h.Ny * h.Nxh : h.Nxh;
         if (h.last_reg) {
             // class 0 joins the launch of another class of the set
+            maps[PH_LASTR4].allforms = (forms.last_classes & 7) == 3;
             const Phase cls[3] = {forms.last_classes & 4 ? PH_LASTRW : (forms.last_classes & 2 ? PH_LASTR4 : PH_LASTR), PH_LASTR4, PH_LASTRW};
             add(cls[last_reg_class(h.ax[la].N, h.ntypes)], (Q + h.nl_last - 1) / h.nl_last,
                 last_reg_lds_bytes(h.ax[la], h.nf));

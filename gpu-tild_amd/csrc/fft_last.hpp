@@ -209,7 +209,7 @@ __device__ __forceinline__ void last_reg_block(const RepDev& r, int blk, float2*
 
 template <class P, int NT, int TT, int CH, int CLS>
 __device__ __forceinline__ void last_reg_variant_block(const RepDev& r, int blk, float2* lds, int koff) {
-    if constexpr (last_reg_variant(P::A0, P::R1, P::R2, P::REV, TT) && (last_reg_class(P::N, TT) == CLS || last_reg_class(P::N, TT) == 0))
+    if constexpr (last_reg_variant(P::A0, P::R1, P::R2, P::REV, TT) && last_reg_held(last_reg_class(P::N, TT), CLS))
         last_reg_block<P, NT, TT, CH>(r, blk, lds, koff);
 }
 
@@ -233,9 +233,11 @@ __device__ __forceinline__ void last_reg_types(const RepDev& r, int blk, float2*
 
 // One instantiation per class of variants (last_reg_class), each compiled in a file of
 // its own: a class's registers do not lower the occupancy of another's, and the classes
-// compile side by side.  The kernels of classes 1 and 2 hold class 0 too: in a set of several
-// classes its replicas join their launch (films of 64 and 128 points in one launch 7.5 us a
-// step, in two 12.7; six 64^3 and six 64 x 64 x 128 melts 35.9 and 43.2).
+// compile side by side.  In a set of several classes those of class 0 join the launch of
+// another (films of 64 and 128 points in one launch 7.5 us a step, in two 12.7; six 64^3 and
+// six 64 x 64 x 128 melts 35.9 and 43.2): the kernel of class 2 holds them too, at no cost to
+// it, and kernel 3 holds classes 0 and 1 for such sets, since class 1 alone lost by it
+// (coacervate on 64^3 8.8 -> 9.7 us).
 template <int NT, int CLS>
 __global__ void __launch_bounds__(NT) k_last_reg(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wmap,
                                                  int koff) {

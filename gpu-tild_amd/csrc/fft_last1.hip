@@ -1,4 +1,4 @@
-// fft_last1.hip -- k_last_reg for axes up to 100 points, three or four types (and those of fft_last0.hip).
+// fft_last1.hip -- k_last_reg for axes up to 100 points, three or four types.
 #include "fft_last.hpp"
 
 namespace tild {

@@ -979,11 +979,16 @@ bool last_reg_plan(const AxisPlan& pl, int ntypes, int nf) {
 
 hipError_t launch_last_reg(const LaunchCtx& c, int koff, int cls) {
     if (!c.n) return hipSuccess;
-    return cls == 0 ? launch_last_reg_0(c, koff) : (cls == 1 ? launch_last_reg_1(c, koff) : launch_last_reg_2(c, koff));
+    switch (cls == 1 && c.allforms ? kLastRegShort : cls) {
+        case 0: return launch_last_reg_0(c, koff);
+        case 1: return launch_last_reg_1(c, koff);
+        case 2: return launch_last_reg_2(c, koff);
+        default: return launch_last_reg_3(c, koff);
+    }
 }
 
 hipError_t configure_last_reg() {
-    for (hipError_t e : {configure_last_reg_0(), configure_last_reg_1(), configure_last_reg_2()})
+    for (hipError_t e : {configure_last_reg_0(), configure_last_reg_1(), configure_last_reg_2(), configure_last_reg_3()})
         if (e != hipSuccess) return e;
     return hipSuccess;
 }

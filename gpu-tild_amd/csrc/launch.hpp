@@ -71,7 +71,8 @@ struct LaunchCtx {
     int xfft = kXRegister;   // tiled deposit: the x transforms its replicas run
     // some replica of the set needs the instantiation that holds every form.  Deposit:
     // position records; particles: orders above 1; forward plane pass: rectangles and y
-    // columns; y inverse, x C2R: plans with a group of two stages
+    // columns; y inverse, x C2R: plans with a group of two stages;
+    // fused last-axis pass, class 1: class 0 with it
     bool allforms = true;
 };
 
@@ -145,8 +146,13 @@ __host__ __device__ constexpr bool last_reg_variant(int A0, int R1, int R2, bool
     return TT <= (R1 * R2 > 100 || A0 == 16 ? 2 : 4) && TT * (rev ? R2 : R1) <= 50;
 }
 // the kernel instantiation of a variant: axes up to 100 points with up to two types (class
-// 0, held by the other two as well) or three and four (class 1), and longer axes (class 2)
+// 0) or three and four (class 1), and longer axes (class 2)
 __host__ __device__ constexpr int last_reg_class(int N, int TT) { return N > 100 ? 2 : (TT >= 3 ? 1 : 0); }
+constexpr int kLastRegShort = 3;   // the kernel of classes 0 and 1
+// whether the kernel of class k holds class c
+__host__ __device__ constexpr bool last_reg_held(int c, int k) {
+    return c == k || (c == 0 && k == 2) || (c <= 1 && k == kLastRegShort);
+}
 bool last_reg_plan(const AxisPlan& pl, int ntypes, int nf);
 // columns of a block: one thread per (column, index of the larger group, field)
 __host__ __device__ constexpr int last_reg_cols(int R1, int R2, int nf) {
@@ -162,9 +168,11 @@ hipError_t launch_last_reg(const LaunchCtx& c, int koff, int cls);
 hipError_t launch_last_reg_0(const LaunchCtx& c, int koff);   // one per class, in files of their own
 hipError_t launch_last_reg_1(const LaunchCtx& c, int koff);
 hipError_t launch_last_reg_2(const LaunchCtx& c, int koff);
+hipError_t launch_last_reg_3(const LaunchCtx& c, int koff);
 hipError_t configure_last_reg_0();
 hipError_t configure_last_reg_1();
 hipError_t configure_last_reg_2();
+hipError_t configure_last_reg_3();
 // The y inverse of the gradient spectra with register-resident columns (3D, y plans as
 // above with R1 <= 16): blocks of kGradRegThreads threads, grad_reg_lines(plan) columns
 // each, grad_reg_chunks per (field, z) plane.
