@@ -75,8 +75,8 @@ def phase_bytes(ns, D, M, Mh, nf, T, gjf, charged, ncoef, reorder_every, plane_i
 
 # the kernel of each profiled phase on the default (tiled, forward-plane) path, as named
 # in the rocprofv3 summaries
-PHASE_KERNEL = {"claim": "k_tile_claim", "deposit": "k_tile_deposit<512, false, false>", "plane_r2c": "k_plane_reg<512, false>",
-                "last_fused": "k_last_reg<256, 2>", "y_ifft": "k_grad_reg<128>", "x_c2r": "k_x_c2r<true, 256>",
+PHASE_KERNEL = {"claim": "k_tile_claim", "deposit": "k_tile_deposit<512, 0, false>", "plane_r2c": "k_plane_reg<512, false>",
+                "last_fused": "k_last_reg<256, 2>", "y_ifft": "k_grad_reg<128, false>", "x_c2r": "k_x_c2r<true, 256>",
                 "particles": "k_particles<true, true, false>",
                 "advance": "k_advance", "reorder": None}
 # with the inverse plane pass (square x-y planes)

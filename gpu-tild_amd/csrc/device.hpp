@@ -114,8 +114,8 @@ struct alignas(64) RepDev {
     int plane_reg; // 1: the forward plane pass runs register-resident (k_plane_reg)
     int plane_inv; // 1: y inverse and x C2R run as one register-resident plane pass (k_plane_inv)
     int c2r_reg;   // 1: the x C2R runs register-resident (k_c2r_reg)
-    int plane_rect;   // 1: the forward plane pass of other planes runs register-resident (k_plane_rect)
-    int yfwd_reg;  // 1: the forward y pass runs register-resident (k_yfwd_reg)
+    int plane_rect;   // 1: the forward plane pass of other planes runs register-resident (plane_rect_block)
+    int yfwd_reg;  // 1: the forward y pass runs register-resident (yfwd_piece)
     int plane_pair; // > 0: y inverse and x C2R run as one pass (k_plane_inv), this many pairs of lines a block
     // FFT plans (x, y, z)
     AxisPlan ax[3];

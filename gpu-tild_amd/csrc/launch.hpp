@@ -119,10 +119,10 @@ __host__ __device__ constexpr int reg_plan_key(int a0, int a1, int b0, int b1) {
     k = k * 32 + b0;
     return b1 > 1 ? k * 32 + b1 : k;
 }
-// Plans of the first two lines: the fused z pass, the y inverse and the plane passes have
-// run these in registers all along, with products and sums fused as the compiler chose
-// there; every other register pass fuses them as the LDS-staged pass it stands for, so that
-// no length's results depend on which of the two runs.
+// Plans of the first two lines: the fused z pass and the plane passes of square planes have run
+// these in registers all along, and fuse the other product of a twiddle's two sums (cmul_kept;
+// the inverse plane pass as the compiler does); every other register pass fuses them as the
+// LDS-staged pass it stands for, so that no length's results depend on which of the two runs.
 __host__ __device__ constexpr bool reg_plan_kept(int n) {
     return n == 24 || n == 25 || n == 30 || n == 32 || n == 40 || n == 48 || n == 50 || n == 64 || n == 80 || n == 128 ||
            n == 160;

@@ -114,11 +114,12 @@ typedef struct {
     int fft_staged;      /* nonzero: every FFT pass of the step stages every value through
                             LDS even where its register-resident form applies (36 axis
                             lengths of 21 to 240 points; the z pass at most four types,
-                            two above 100 points).  On axes of 24, 25, 30, 32, 40, 48, 50,
-                            64, 80, 128 and 160 points the forms agree to rounding (about
-                            1e-7 relative), not bit for bit: the compiler fuses multiplies
-                            into additions where one keeps in registers what the other
-                            stages through LDS.  On other axes they are identical. */
+                            two above 100 points and on 48).  The z pass on axes of 24,
+                            25, 30, 32, 40, 48, 50, 64, 80, 128 and 160 points, and the
+                            plane passes on square planes of these sides, agree with the
+                            staged forms to rounding (about 1e-7 relative), not bit for
+                            bit: they fuse the other product of a twiddle's sums.  All
+                            other forms are identical. */
 } tild_opts;
 
 /* Properties of calc_properties() (calc_properties.cu:20-116): FP64 reductions. */

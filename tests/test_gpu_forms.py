@@ -64,3 +64,10 @@ def test_box_equals_staged(grid, ntypes, charged, c2r, tmp_path):
 @pytest.mark.parametrize("grid,c2r", [((125, 100, 9), 0), ((160, 80, 9), 0), ((120, 128, 9), 1), ((125, 27), 1), ((160, 27), 1)])
 def test_x_c2r_rule(grid, c2r, tmp_path):
     _compare(_system(tmp_path, grid, 2, False), {"last_reg": int(len(grid) == 2)}, {"c2r_reg": c2r})
+
+
+@pytest.mark.parametrize("n", [24, 25, 30, 32, 40, 48, 50, 64, 80, 128, 160])
+def test_y_inverse_equals_staged(n, tmp_path):
+    # the lengths whose z pass differs: the y passes of planes without plane passes do not
+    _compare(_system(tmp_path, (20, n, 9), 2, False), {"last_reg": 0, "plane_reg": 0, "plane_inv": 0, "grad_reg": 1},
+             {"plane_rect": 0, "yfwd_reg": n % 2, "plane_pair": 0, "c2r_reg": 0})
