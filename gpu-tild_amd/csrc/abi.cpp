@@ -334,7 +334,8 @@ tild_status tild_engine_geometry(tild_engine* e, tild_geometry* out) {
 tild_status tild_engine_passes(tild_engine* e, tild_passes* out) {
     if (!e || !out) return fail(TILD_ERR_ARG, "null argument");
     const tild::RepDev& h = e->batch->rep(e->id)->h;
-    *out = tild_passes{h.plane_rect, h.yfwd_reg, h.plane_pair > 0 ? 1 : 0, h.c2r_reg};
+    const bool xreg = h.spread_mode == 2 && !h.plane_fwd && h.grid_off32 && tild::deposit_xreg(h.reg_key[0], h.dim);
+    *out = tild_passes{h.plane_rect, h.yfwd_reg, h.plane_pair > 0 ? 1 : 0, h.c2r_reg, xreg ? 1 : 0};
     return TILD_OK;
 }
 

@@ -763,7 +763,7 @@ int Batch::build_maps(const std::vector<int>& ids, PhaseMap* maps, std::string& 
             add(PH_TCOUNT, (h.ns + kCountBlock - 1) / kCountBlock, 0);
             add(PH_SCAN, 1, 0);
             const Phase dep = deposit_phase(h);
-            const bool xreg = h.reg_key[0] && h.grid_off32;
+            const bool xreg = deposit_xreg(h.reg_key[0], D) && h.grid_off32;
             add(dep, h.ntiles, tile_lds_bytes(h.Nx, h.nf, h.By, h.Bz, h.plane_fwd, xreg));
             maps[dep].allforms = maps[dep].allforms || !h.srec;
             if (!h.plane_fwd) maps[dep].xfft = std::max(maps[dep].xfft, (int)(xreg ? kXRegister : kXStaged));

@@ -130,6 +130,13 @@ __host__ __device__ constexpr bool reg_plan_kept(int n) {
 // Plans with a group of two stages hold more values a thread (reg_plan_grouped): sets without
 // them run kernels compiled without them, whose registers leave room for more waves.
 __host__ __device__ constexpr bool reg_plan_grouped(int A1, int B1) { return A1 > 1 || B1 > 1; }
+// x transform of the tiled deposit: in registers for compiled plans, but for films of 80 and 160
+// points, whose LDS-staged form runs its two stages compiled (lds_fft2) in 71 registers against
+// 128: staged and in registers, us, 160 x 64 6.5 and 7.1, 160 x 1024 7.6 and 8.1, 80 x 1024 6.2 and
+// 7.0; odd-sided boxes 160 x 125 x 24 12.3 and 11.0, 80 x 45 x 60 with five fields 12.0 and 10.2.
+__host__ __device__ constexpr bool deposit_xreg(int key, int dim) {
+    return key != 0 && !(dim == 2 && (key == reg_plan_key(16, 1, 10, 1) || key == reg_plan_key(10, 1, 8, 1)));
+}
 // key, group sizes and first stage of the second group of an axis plan (key 0: not compiled)
 struct RegDims {
     int key, R1, R2, group2;

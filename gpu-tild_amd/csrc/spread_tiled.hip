@@ -539,7 +539,7 @@ k_tile_deposit(const RepDev* __restrict__ reps, const WorkItem* __restrict__ wma
     // the first density element of each tile row (f, lz, ly)
     int* const rowoff = (int*)fbuf;
     // register form of the x transform: its twiddles and row table sit behind the exchange
-    const bool xreg = XFFT == kXRegister && !plane_fwd && r.reg_key[0] && r.grid_off32;
+    const bool xreg = XFFT == kXRegister && !plane_fwd && deposit_xreg(r.reg_key[0], D) && r.grid_off32;
     float2* const xtw = fbuf + (size_t)Nx * (((rows + 1) / 2) | 1);
     int* const rowid = (int*)(xtw + Nx);
     if (XFFT == kXRegister && xreg) {

@@ -66,7 +66,7 @@ class Geometry(ctypes.Structure):
 
 
 class Passes(ctypes.Structure):
-    _fields_ = [(k, ctypes.c_int) for k in ("plane_rect", "yfwd_reg", "plane_pair", "c2r_reg")]
+    _fields_ = [(k, ctypes.c_int) for k in ("plane_rect", "yfwd_reg", "plane_pair", "c2r_reg", "deposit_xreg")]
 
     def as_dict(self):
         return {k: getattr(self, k) for k, _ in self._fields_}

@@ -229,6 +229,7 @@ typedef struct {
     int yfwd_reg;        /* forward y pass (odd sides, whose deposit transforms x) */
     int plane_pair;      /* y inverse and x C2R as one pass, other planes than plane_inv's */
     int c2r_reg;         /* x C2R where no plane pass runs it */
+    int deposit_xreg;    /* x transform of the tiled deposit (films, odd sides) */
 } tild_passes;
 tild_status tild_engine_passes(tild_engine* e, tild_passes* out);
 /* Compute::doCompute for avg_sk (Compute.cu:83-117): adds rho_t(k) rho_t(k) / M -- the

@@ -71,3 +71,11 @@ def test_y_inverse_equals_staged(n, tmp_path):
     # the lengths whose z pass differs: the y passes of planes without plane passes do not
     _compare(_system(tmp_path, (20, n, 9), 2, False), {"last_reg": 0, "plane_reg": 0, "plane_inv": 0, "grad_reg": 1},
              {"plane_rect": 0, "yfwd_reg": n % 2, "plane_pair": 0, "c2r_reg": 0})
+
+
+# the x transform of the deposit: staged for films of 80 and 160 points, whose staged form is the
+# faster one, in registers for other compiled plans; none with the forward plane pass
+@pytest.mark.parametrize("grid,xreg", [((80, 27), 0), ((160, 45), 0), ((64, 27), 1), ((128, 45), 1), ((100, 27), 1),
+                                       ((80, 45, 21), 1), ((160, 27, 21), 1), ((80, 36, 21), 0), ((20, 45), 0)])
+def test_deposit_x_transform_rule(grid, xreg, tmp_path):
+    _compare(_system(tmp_path, grid, 2, False), {}, {"deposit_xreg": xreg})
